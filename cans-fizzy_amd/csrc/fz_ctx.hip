@@ -78,6 +78,7 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
   if (const char *e = getenv("FZ_CORREC_MY")) c->correc_my = atoi(e);
   if (c->correc_my != 8 && c->correc_my != 16) c->correc_my = 4;  // the tile heights the kernel is built for
   if (const char *e = getenv("FZ_P2_XDIV")) c->p2_xdiv = atoi(e);
+  if (const char *e = getenv("FZ_MARCH_PLANES")) c->march = atoi(e);
   if (const char *e = getenv("FZ_ACDI_VARIANT")) c->acdi_variant = atoi(e);
   if (const char *e = getenv("FZ_YOUNGS_VARIANT")) c->youngs_variant = atoi(e);
   // the Thomas kernel without a pivot array pays off once the columns fill
@@ -145,6 +146,10 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
     fz_ctx_destroy(c);
     return fz_set_error(FZ_ERR_HIP, "hipHostMalloc: %s", hipGetErrorString(e));
   }
+  int dev_id = 0, ncu = 0;
+  if (hipGetDevice(&dev_id) == hipSuccess &&
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id) == hipSuccess && ncu > 0)
+    c->ncu = ncu;
   const int rs = fz_scratch_setup(c);
   if (rs != FZ_OK) {
     fz_ctx_destroy(c);

@@ -321,6 +321,39 @@ static int fits_buffers(const fz_ctx *c, const char *who) {
   return fz_set_error(FZ_ERR_UNSUPPORTED, "%s: halo'd fields above 4 GiB are not supported", who);
 }
 
+// Planes per block of the kernels that march up z (sets grid.z, the blocks
+// of one case). Sixteen planes read each plane of a large grid nearly once,
+// and a grid that fills the device several times over takes them. A smaller
+// one waits for its blocks' marches: it takes the number of planes with the
+// least (rounds of resident blocks) x (planes + start-up), res blocks per CU
+// being resident and the start-up (the planes around the first, one memory
+// latency each) costing about START levels. WHOLE: a last round that is
+// not full costs a full one (the momentum kernel, bound by latency; the
+// others share the bandwidth that its absence leaves, and 1.3 rounds take
+// 1.3 times as long as one). Measured, 16 planes against this choice: 64x2x64
+// momentum 45 -> 10 us, ACDI 43 -> 10, correction 26 -> 9, normals 18 -> 8;
+// 64x64x128 53 -> 27, 48 -> 23, 30 -> 15, 20 -> 12; 96x96x192 90 -> 81,
+// 95 -> 78, 48 -> 42, 35 -> 30; 128x128x256 and larger unchanged.
+// FZ_MARCH_PLANES fixes it.
+template <bool WHOLE = false>
+static int march_planes(const fz_ctx *c, dim3 &grid, int nz, int ncase, int res) {
+  constexpr long START = 3;
+  const long per_plane = (long)grid.x * grid.y * ncase, slots = (long)c->ncu * res;
+  int kz = 16;
+  if (c->march > 0) {
+    kz = c->march;
+  } else if (per_plane * ((nz + 15) / 16) < 8 * slots) {
+    long best = -1;
+    for (int t = 16; t >= 1; t--) {
+      const long nb = per_plane * ((nz + t - 1) / t);
+      const long rounds = WHOLE ? (nb + slots - 1) / slots * slots : (nb > slots ? nb : slots);  // x slots
+      if (best < 0 || rounds * (t + START) < best) best = rounds * (t + START), kz = t;
+    }
+  }
+  grid.z = (unsigned)((nz + kz - 1) / kz);
+  return kz;
+}
+
 // A kernel that writes the interior cells of a field that is periodic in x
 // can write the x halo of the cell's row as well (xper): the halo cells 0
 // and n1+1 take the values of the cells n1 and 1, as the periodic boundary
@@ -391,8 +424,8 @@ static int xhalo_copy(fz_ctx *c, T *f0, T *f1, T *f2, T *f3) {
 // five (dp) or two (u, v) neighbour loads, whose address processing bounds
 // the one-cell-per-load kernel. Same expressions, same values.
 constexpr int COR_MX = 64, COR_PX = COR_MX + 2;
-template <int KZ, int MY, bool BT = false>
-__global__ void __launch_bounds__(COR_MX *MY) k_correc_lds(fz_dims d, const double *__restrict__ dzci,
+template <int MY, bool BT = false>
+__global__ void __launch_bounds__(COR_MX *MY) k_correc_lds(fz_dims d, int kz, const double *__restrict__ dzci,
                                                               double factori_v, double factorj_v, double dt_v,
                                                               double dxi, double dyi, const double *__restrict__ stc,
                                                               double rhop, const double *__restrict__ dp,
@@ -430,7 +463,7 @@ __global__ void __launch_bounds__(COR_MX *MY) k_correc_lds(fz_dims d, const doub
   const int xlo = rlo & 1u, ylo = (rlo >> 1) & 1u, zlo = (rlo >> 2) & 1u;
   const int i0 = xlo + (int)bx * COR_MX, j0 = ylo + (int)by * MY;
   const int i = i0 + tx, j = j0 + ty;
-  const int k0 = zlo + (int)bz * KZ, kend = min(k0 + KZ - 1, d.n3 + 1 - zlo), ktop = min(kend + 1, d.n3 + 1);
+  const int k0 = zlo + (int)bz * kz, kend = min(k0 + kz - 1, d.n3 + 1 - zlo), ktop = min(kend + 1, d.n3 + 1);
   const bool act = i <= d.n1 + 1 - xlo && j <= d.n2 + 1 - ylo;
   const bool in_ij = i >= 1 && i <= d.n1 && j >= 1 && j <= d.n2;
   const int c = (ty + 1) * COR_PX + (tx + 1);
@@ -542,13 +575,13 @@ int fz_launch_correc_step(fz_ctx *c, double rho0, double dt, const double *stc, 
                           double *p_out, unsigned long long *slots, int xper, unsigned rlo) {
   if (c->correc_kz == 1) {  // dp, u, v staged in LDS
     FZ_TRY(fits_buffers(c, "correc_step"));
-    constexpr int KZ = 16;
     const int my = c->correc_my;
     // (rlo: the directions whose range is 1 to n, see k_correc_lds)
     const int ex = 2 - 2 * (int)(rlo & 1u), ey = 2 - 2 * (int)((rlo >> 1) & 1u), ez = 2 - 2 * (int)((rlo >> 2) & 1u);
-    const dim3 grid((c->d.n1 + ex + COR_MX - 1) / COR_MX, (c->d.n2 + ey + my - 1) / my, (c->d.n3 + ez + KZ - 1) / KZ);
+    dim3 grid((c->d.n1 + ex + COR_MX - 1) / COR_MX, (c->d.n2 + ey + my - 1) / my);
+    const int kz = march_planes(c, grid, c->d.n3 + ez, 1, 24 / my);
 #define FZ_CORREC_LDS(MY)                                                                                          \
-  FZ_LAUNCH(c, "correc_step", (k_correc_lds<KZ, MY>), grid, dim3(COR_MX, MY), 0, c->d, c->dzci, dt * c->dli[0],     \
+  FZ_LAUNCH(c, "correc_step", (k_correc_lds<MY>), grid, dim3(COR_MX, MY), 0, c->d, kz, c->dzci, dt * c->dli[0],     \
             dt * c->dli[1], dt, c->dli[0], c->dli[1], stc, rho0, dp, p, u, v, w, un, vn, wn, p_out, slots, kNoBRef, \
             xper, rlo)
     if (my == 16) FZ_CORREC_LDS(16);
@@ -734,8 +767,8 @@ struct LdsZ {
   }
 };
 
-template <typename T, int KZ, bool BT = false>  // BT: a batched launch (fz_bref)
-__global__ void __launch_bounds__(ACD_MX *ACD_MY) k_acdi_lds(fz_dims d, const double *__restrict__ dzci,
+template <typename T, bool BT = false>  // BT: a batched launch (fz_bref)
+__global__ void __launch_bounds__(ACD_MX *ACD_MY) k_acdi_lds(fz_dims d, int kz, const double *__restrict__ dzci,
                                                             const double *__restrict__ dzfi, double dxi, double dyi,
                                                             const double *__restrict__ d_gam, double gam_v,
                                                             double seps, double factor1_v, double factor2_v,
@@ -773,10 +806,10 @@ __global__ void __launch_bounds__(ACD_MX *ACD_MY) k_acdi_lds(fz_dims d, const do
   const double gam = d_gam ? *d_gam : gam_v;
   const double factor1 = stc ? stc[FZ_STC_F1] : factor1_v, factor2 = stc ? stc[FZ_STC_F2] : factor2_v;
   const int tx = threadIdx.x, ty = threadIdx.y, t = tx + ACD_MX * ty;
-  const int i0 = (int)bx * ACD_MX + 1, j0 = (int)by * ACD_MY + 1, k0 = (int)bz * KZ + 1;
+  const int i0 = (int)bx * ACD_MX + 1, j0 = (int)by * ACD_MY + 1, k0 = (int)bz * kz + 1;
   const int i = i0 + tx, j = j0 + ty;
   const bool act = i <= d.n1 && j <= d.n2;
-  const int kend = min(k0 + KZ - 1, d.n3);
+  const int kend = min(k0 + kz - 1, d.n3);
   const int c = (ty + 1) * ACD_PX + (tx + 1);
   const BufFld<double> GU = buf_fld(u, d), GV = buf_fld(v, d), GW = buf_fld(w, d);
   const BufFld<T> GNX = buf_fld(normx, d), GNY = buf_fld(normy, d), GNZ = buf_fld(normz, d), GPH = buf_fld(phi, d),
@@ -902,8 +935,8 @@ __device__ __forceinline__ void acdi_face(T psa, T psb, T pha, T phb, T nxa, T n
 // right-hand side from its six faces in acdi_cell's order, so the results
 // are those of k_acdi_lds bit for bit. The velocities are read at the cell
 // only (and below the tile's edges), straight from memory.
-template <typename T, int KZ, bool XPER = false, int MY = ACD_MY>
-__global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, const double *__restrict__ dzci,
+template <typename T, bool XPER = false, int MY = ACD_MY>
+__global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const double *__restrict__ dzci,
                                                            const double *__restrict__ dzfi, double dxi_d,
                                                            double dyi_d, const double *__restrict__ d_gam,
                                                            double gam_v, double seps_d, double factor1_v,
@@ -930,10 +963,10 @@ __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, const double 
   const T dxi = (T)dxi_d, dyi = (T)dyi_d, gam = (T)gam_dd, seps = (T)seps_d;
   const T gs = gam * seps, g4 = (T)0.25 * gam;
   const int tx = threadIdx.x, ty = threadIdx.y, t = tx + ACD_MX * ty;
-  const int i0 = (int)bx * ACD_MX + 1, j0 = (int)by * MY + 1, k0 = (int)bz * KZ + 1;
+  const int i0 = (int)bx * ACD_MX + 1, j0 = (int)by * MY + 1, k0 = (int)bz * kz + 1;
   const int i = i0 + tx, j = j0 + ty;
   const bool act = i <= d.n1 && j <= d.n2;
-  const int kend = min(k0 + KZ - 1, d.n3);
+  const int kend = min(k0 + kz - 1, d.n3);
   const int c = (ty + 1) * ACD_PX + (tx + 1);
   const BufFld<double> GU = buf_fld(u, d), GV = buf_fld(v, d), GW = buf_fld(w, d);
   const BufFld<T> GNX = buf_fld(normx, d), GNY = buf_fld(normy, d), GNZ = buf_fld(normz, d), GPH = buf_fld(phi, d),
@@ -1069,22 +1102,22 @@ int fz_launch_acdi_step(fz_ctx *c, const double *d_gam, double gam, double seps,
   // FP64 1047 against 1120 us for the plain one (2)
   const int variant = c->acdi_variant ? c->acdi_variant : 3;
   if (variant == 3) {  // each face evaluated once
-    constexpr int KZ = 16;
     // (the x-halo stores compiled only into the instance that makes them; a
     // run-time test there too: measured 550 against 565 us in FP32 without
     // it. FP32 tiles of 64 x 8: 550 -> 532 us; FP64 ones, 70 KB of LDS, 925
     // against 923 us, keep 64 x 4)
     constexpr int MY = sizeof(T) == 4 ? 8 : ACD_MY;
-    const dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + MY - 1) / MY, (c->d.n3 + KZ - 1) / KZ);
-    auto kern = xper ? k_acdi_sf<T, KZ, true, MY> : k_acdi_sf<T, KZ, false, MY>;
-    FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", kern, grid, dim3(ACD_MX, MY), 0, c->d, c->dzci,
+    dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + MY - 1) / MY);
+    const int kz = march_planes(c, grid, c->d.n3, 1, 3);
+    auto kern = xper ? k_acdi_sf<T, true, MY> : k_acdi_sf<T, false, MY>;
+    FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", kern, grid, dim3(ACD_MX, MY), 0, c->d, kz, c->dzci,
               c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc, first, u, v, w, normx, normy,
               normz, phi, psio, dpsio, psi_out, flux_x, flux_y, flux_z, xper);
   } else if (variant == 1) {  // fields staged in LDS
-    constexpr int KZ = 16;
-    const dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY, (c->d.n3 + KZ - 1) / KZ);
-    FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", (k_acdi_lds<T, KZ>), grid, dim3(ACD_MX, ACD_MY), 0,
-              c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc, first, u, v, w,
+    dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY);
+    const int kz = march_planes(c, grid, c->d.n3, 1, 3);
+    FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", (k_acdi_lds<T>), grid, dim3(ACD_MX, ACD_MY), 0,
+              c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc, first, u, v, w,
               normx, normy, normz, phi, psio, dpsio, psi_out, flux_x, flux_y, flux_z, kNoBRef);
   } else {
     FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", k_acdi_step<T>, fz_grid_interior(c->d),
@@ -1506,7 +1539,7 @@ struct RegAt27 {
   }
 };
 
-// k_youngs with each thread marching up KZ cells in z: the 3 x 3 plane
+// k_youngs with each thread marching up kz cells in z: the 3 x 3 plane
 // neighbourhoods of k-1, k, k+1 stay in registers, so a level loads the nine
 // values of the plane k+2 (issued before the level's arithmetic) instead of
 // 27. The cell arithmetic is youngs_cell's through a register accessor, the
@@ -1517,14 +1550,14 @@ struct RegAt27 {
 // tile grid, the blocks striding over the tiles (so 1 then 2 compute the
 // field in either case, the register-hungry checked form runs only when
 // needed, and a few hundred blocks of mode 2 find the flag clear and exit).
-template <typename T, int KZ, int MODE>
-__device__ __forceinline__ void youngs_mz_tile(const fz_dims &d, const double *__restrict__ dzci,
+template <typename T, int MODE>
+__device__ __forceinline__ void youngs_mz_tile(const fz_dims &d, int kz, const double *__restrict__ dzci,
                                                const double *__restrict__ dzfi, double dxi_d, double dyi_d,
                                                const T *__restrict__ psi, T *__restrict__ normx,
                                                T *__restrict__ normy, T *__restrict__ normz, T *__restrict__ kappa,
                                                int xper, bool nocheck, unsigned bx, unsigned by, unsigned bz) {
   const int i = (int)bx * blockDim.x + threadIdx.x + 1, j = (int)by * blockDim.y + threadIdx.y + 1;
-  const int k0 = (int)bz * KZ + 1, kend = min(k0 + KZ - 1, d.n3);
+  const int k0 = (int)bz * kz + 1, kend = min(k0 + kz - 1, d.n3);
   if (i > d.n1 || j > d.n2) return;  // (no barriers below)
   const BufFld<T> G = buf_fld(psi, d);
   const unsigned e00 = (unsigned)i + (unsigned)d.sy * (unsigned)j, sy = (unsigned)d.sy, sz = (unsigned)d.sz;
@@ -1574,8 +1607,8 @@ __device__ __forceinline__ void youngs_mz_tile(const fz_dims &d, const double *_
   }
 }
 
-template <typename T, int KZ, int MODE = 0>
-__global__ void __launch_bounds__(256) k_youngs_mz(fz_dims d, const double *__restrict__ dzci,
+template <typename T, int MODE = 0>
+__global__ void __launch_bounds__(256) k_youngs_mz(fz_dims d, int kz, const double *__restrict__ dzci,
                                                    const double *__restrict__ dzfi, double dxi_d, double dyi_d,
                                                    const T *__restrict__ psi, T *__restrict__ normx,
                                                    T *__restrict__ normy, T *__restrict__ normz,
@@ -1591,13 +1624,13 @@ __global__ void __launch_bounds__(256) k_youngs_mz(fz_dims d, const double *__re
     const unsigned per_plane = tiles.x * tiles.y, nt = per_plane * tiles.z;
     for (unsigned t = blockIdx.x; t < nt; t += gridDim.x) {
       const unsigned bz = t / per_plane, r = t - bz * per_plane, by = r / tiles.x, bx = r - by * tiles.x;
-      youngs_mz_tile<T, KZ, MODE>(d, dzci, dzfi, dxi_d, dyi_d, psi, normx, normy, normz, kappa, xper, false, bx, by,
+      youngs_mz_tile<T, MODE>(d, kz, dzci, dzfi, dxi_d, dyi_d, psi, normx, normy, normz, kappa, xper, false, bx, by,
                                   bz);
     }
   } else {
     unsigned cs_, bx, by, bz;
     fz_stencil_block_b(d.tile_y, gridDim.z, cs_, bx, by, bz);
-    youngs_mz_tile<T, KZ, MODE>(d, dzci, dzfi, dxi_d, dyi_d, psi, normx, normy, normz, kappa, xper, nocheck, bx, by,
+    youngs_mz_tile<T, MODE>(d, kz, dzci, dzfi, dxi_d, dyi_d, psi, normx, normy, normz, kappa, xper, nocheck, bx, by,
                                 bz);
   }
 }
@@ -1615,23 +1648,22 @@ static int launch_youngs(fz_ctx *c, const char *name, const T *psi, T *normx, T 
   // two waves per SIMD, and took 758 against 705-745 us for one cell per
   // thread; capped, it spills), one cell per thread elsewhere
   const int yv = c->youngs_variant ? c->youngs_variant : (sizeof(T) == 4 ? 1 : 3);
-  constexpr int KZ = 16;
   dim3 mgrid = fz_grid_interior(c->d);
-  mgrid.z = (c->d.n3 + KZ - 1) / KZ;
+  const int kz = march_planes(c, mgrid, c->d.n3, 1, 4);
   const uint3 tiles = {mgrid.x, mgrid.y, mgrid.z};
   if (!br.bt && yv == 1) {  // marching in z
-    FZ_LAUNCH(c, name, (k_youngs_mz<T, KZ>), mgrid, fz_block3(), 0, c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+    FZ_LAUNCH(c, name, (k_youngs_mz<T>), mgrid, fz_block3(), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
               psi, normx, normy, normz, kappa, xper, rflag, tiles);
     FZ_LAUNCHED();
     return FZ_OK;
   }
   if (!br.bt && yv == 3 && rflag) {  // the check-free marching kernel, then the checked one if the flag is raised
-    FZ_LAUNCH(c, name, (k_youngs_mz<T, KZ, 1>), mgrid, fz_block3(), 0, c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+    FZ_LAUNCH(c, name, (k_youngs_mz<T, 1>), mgrid, fz_block3(), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
               psi, normx, normy, normz, kappa, xper, rflag, tiles);
     FZ_LAUNCHED();
     // (a grid-stride launch of at most 512 blocks: 2 per CU)
     const unsigned nt = mgrid.x * mgrid.y * mgrid.z, nb2 = nt < 512u ? nt : 512u;
-    FZ_LAUNCH(c, name, (k_youngs_mz<T, KZ, 2>), dim3(nb2), fz_block3(), 0, c->d, c->dzci, c->dzfi, c->dli[0],
+    FZ_LAUNCH(c, name, (k_youngs_mz<T, 2>), dim3(nb2), fz_block3(), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0],
               c->dli[1], psi, normx, normy, normz, kappa, xper, rflag, tiles);
     FZ_LAUNCHED();
     return FZ_OK;
@@ -2024,7 +2056,7 @@ FZ_MOM_FUSED_KERNEL(k_mom_fused_w5, __attribute__((amdgpu_waves_per_eu(5))), fal
 // stencil reads u, v, w, psi and the three psi fluxes at up to 16 neighbours
 // each; read from HBM/L1 one by one, those loads keep the texture-address
 // unit busy 94 % of the kernel (rocprofv3 TA_TA_BUSY at 256x256x512) while
-// HBM moves 3 TB/s. Here a block of MX x MY cells marches up KZ planes in z
+// HBM moves 3 TB/s. Here a block of MX x MY cells marches up kz planes in z
 // and holds, for each of the seven fields, the planes k-1, k, k+1 of its
 // tile plus a one-cell x/y frame in LDS (a ring of three plane slots); each
 // plane is read from HBM once, in rows, the plane k+2 being loaded into
@@ -2050,9 +2082,9 @@ struct LdsAt {
 // first (first = 0) with no bulk-density term (rho_av = 0), known at compile time
 // (XPER: the cells 1 and n1 also store their new velocity at the periodic
 // x-halo images n1+1 and 0 of their row)
-template <typename PT, typename HT, int KZ, int WPE, bool BT = false, bool STEADY = false, bool XPER = false>
+template <typename PT, typename HT, int WPE, bool BT = false, bool STEADY = false, bool XPER = false>
 __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_per_eu(WPE))) k_mom_lds(
-    fz_dims d, const double *__restrict__ dzci, const double *__restrict__ dzfi, double dxi, double dyi, double rho,
+    fz_dims d, int kz, const double *__restrict__ dzci, const double *__restrict__ dzfi, double dxi, double dyi, double rho,
     double drho, double mu, double dmu, double factor1_v, double factor2_v, int first, double factor12_v,
     double dt_r_v, const double *__restrict__ stc, double surf_factor, double rho0, double bfx, double bfy,
     double bfz, double gx, double gy, double gz, double rax, double ray, double raz, const PT *__restrict__ psiflx_x,
@@ -2100,10 +2132,10 @@ __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_pe
   const double factor1 = stc ? stc[FZ_STC_F1] : factor1_v, factor2 = stc ? stc[FZ_STC_F2] : factor2_v;
   const double factor12 = stc ? stc[FZ_STC_F12] : factor12_v, dt_r = stc ? stc[FZ_STC_DTR] : dt_r_v;
   const int tx = threadIdx.x, ty = threadIdx.y, t = tx + MOM_MX * ty;
-  const int i0 = (int)bx * MOM_MX + 1, j0 = (int)by * MOM_MY + 1, k0 = (int)bz * KZ + 1;
+  const int i0 = (int)bx * MOM_MX + 1, j0 = (int)by * MOM_MY + 1, k0 = (int)bz * kz + 1;
   const int i = i0 + tx, j = j0 + ty;
   const bool act = i <= d.n1 && j <= d.n2;
-  const int kend = min(k0 + KZ - 1, d.n3);
+  const int kend = min(k0 + kz - 1, d.n3);
   const int c = (ty + 1) * MOM_PX + (tx + 1);
   const BufFld<double> GU = buf_fld(u, d), GV = buf_fld(v, d), GW = buf_fld(w, d);
   const BufFld<PT> GPSI = buf_fld(psi, d), GFX = buf_fld(psiflx_x, d), GFY = buf_fld(psiflx_y, d),
@@ -2233,8 +2265,8 @@ int fz_launch_mom_fused(fz_ctx *c, const double rho12[2], const double mu12[2], 
   int variant = c->mom_variant;
   if (variant == 0) variant = 8;
   if (variant == 8) {  // stencil fields staged in LDS
-    constexpr int KZ = 16;
-    const dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY, (c->d.n3 + KZ - 1) / KZ);
+    dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY);
+    const int kz = march_planes<true>(c, grid, c->d.n3, 1, sizeof(PT) == 4 ? 3 : 2);
     // (3 waves per SIMD fit FP32 phase fields' registers, 169 -> 168 VGPRs;
     // FP64 needs 188, and a 3-wave FP64 build spills 36 and runs 2.2x slower)
     // With FP32 phase fields, a step after the first without a bulk-density
@@ -2246,12 +2278,12 @@ int fz_launch_mom_fused(fz_ctx *c, const double rho12[2], const double mu12[2], 
     const bool steady = first == 0 && rho_av[0] == 0.0 && rho_av[1] == 0.0 && rho_av[2] == 0.0;
     // (xper: the x-halo stores, compiled only into the instances that make them)
     constexpr int W = sizeof(PT) == 4 ? 3 : 1;
-    auto kern = sizeof(PT) == 4 && steady ? (xper ? k_mom_lds<PT, HT, KZ, 3, false, true, true>
-                                                  : k_mom_lds<PT, HT, KZ, 3, false, true, false>)
-                                          : (xper ? k_mom_lds<PT, HT, KZ, W, false, false, true>
-                                                  : k_mom_lds<PT, HT, KZ, W, false, false, false>);
+    auto kern = sizeof(PT) == 4 && steady ? (xper ? k_mom_lds<PT, HT, 3, false, true, true>
+                                                  : k_mom_lds<PT, HT, 3, false, true, false>)
+                                          : (xper ? k_mom_lds<PT, HT, W, false, false, true>
+                                                  : k_mom_lds<PT, HT, W, false, false, false>);
     FZ_LAUNCH(c, sizeof(PT) == 4 ? "mom_fused_f32" : "mom_fused", kern,
-              grid, dim3(MOM_MX, MOM_MY), 0, c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1], rho12[1],
+              grid, dim3(MOM_MX, MOM_MY), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], rho12[1],
               rho12[0] - rho12[1], mu12[1], mu12[0] - mu12[1], factor1, factor2, first, factor12, dt_r, stc,
               surf_factor, rho0, bforce[0], bforce[1], bforce[2], gacc[0], gacc[1], gacc[2], rho_av[0], rho_av[1],
               rho_av[2], fx, fy, fz, u, v, w, psi, psio, p, po, kappa, duo, dvo, dwo, un, vn, wn, kNoBRef);
@@ -2806,12 +2838,12 @@ extern "C" int fz_phase_geometry_eval(fz_ctx *c, double seps, const double *psi,
 template <typename T>
 int fz_batch_acdi_step(fz_ctx *c, fz_bref br, int ncase) {
   FZ_TRY(fits_buffers(c, "acdi_step"));
-  constexpr int KZ = 16;
-  dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY, (c->d.n3 + KZ - 1) / KZ);
+  dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY);
+  const int kz = march_planes(c, grid, c->d.n3, ncase, 3);
   br.gz = grid.z;
   grid.z *= (unsigned)ncase;
-  FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", (k_acdi_lds<T, KZ, true>), grid, dim3(ACD_MX, ACD_MY), 0,
-            c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1], (const double *)nullptr, 0.0, 0.0, 0.0, 0.0,
+  FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", (k_acdi_lds<T, true>), grid, dim3(ACD_MX, ACD_MY), 0,
+            c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], (const double *)nullptr, 0.0, 0.0, 0.0, 0.0,
             (const double *)nullptr, 0, (const double *)nullptr, (const double *)nullptr, (const double *)nullptr,
             (const T *)nullptr, (const T *)nullptr, (const T *)nullptr, (const T *)nullptr, (const T *)nullptr,
             (T *)nullptr, (T *)nullptr, (T *)nullptr, (T *)nullptr, (T *)nullptr, br);
@@ -2849,12 +2881,12 @@ int fz_batch_mom(fz_ctx *c, fz_bref br, int ncase) {
       (const double *)nullptr, (const double *)nullptr, (const PT *)nullptr, (HT *)nullptr, (HT *)nullptr,         \
       (HT *)nullptr, (double *)nullptr, (double *)nullptr, (double *)nullptr, br
   if (variant == 8) {
-    constexpr int KZ = 16;
-    dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY, (c->d.n3 + KZ - 1) / KZ);
+    dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY);
+    const int kz = march_planes<true>(c, grid, c->d.n3, ncase, sizeof(PT) == 4 ? 3 : 2);
     br.gz = grid.z;
     grid.z *= (unsigned)ncase;
-    FZ_LAUNCH(c, name, (k_mom_lds<PT, HT, KZ, sizeof(PT) == 4 ? 3 : 1, true, sizeof(PT) == 4>), grid,
-              dim3(MOM_MX, MOM_MY), 0, c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1], FZ_MOM_NULLS);
+    FZ_LAUNCH(c, name, (k_mom_lds<PT, HT, sizeof(PT) == 4 ? 3 : 1, true, sizeof(PT) == 4>), grid,
+              dim3(MOM_MX, MOM_MY), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], FZ_MOM_NULLS);
   } else {
     auto kern = variant == 4   ? k_mom_fused_w4<PT, HT, true>
                 : variant == 5 ? k_mom_fused_w5<PT, HT, true>
@@ -2876,14 +2908,14 @@ template int fz_batch_mom<float, float>(fz_ctx *, fz_bref, int);
 // gamma from its slots
 int fz_batch_correc_gamma(fz_ctx *c, fz_bref br, int ncase, bool gamma) {
   FZ_TRY(fits_buffers(c, "correc_step"));
-  constexpr int KZ = 16;
   const int my = c->correc_my;
-  dim3 grid((c->d.n1 + 2 + COR_MX - 1) / COR_MX, (c->d.n2 + 2 + my - 1) / my, (c->d.n3 + 2 + KZ - 1) / KZ);
+  dim3 grid((c->d.n1 + 2 + COR_MX - 1) / COR_MX, (c->d.n2 + 2 + my - 1) / my);
+  const int kz = march_planes(c, grid, c->d.n3 + 2, ncase, 24 / my);
   fz_bref b = br;
   b.gz = grid.z;
   grid.z *= (unsigned)ncase;
 #define FZ_CORREC_LDS_B(MY)                                                                                        \
-  FZ_LAUNCH(c, "correc_step", (k_correc_lds<KZ, MY, true>), grid, dim3(COR_MX, MY), 0, c->d, c->dzci, 0.0, 0.0, 0.0, \
+  FZ_LAUNCH(c, "correc_step", (k_correc_lds<MY, true>), grid, dim3(COR_MX, MY), 0, c->d, kz, c->dzci, 0.0, 0.0, 0.0, \
             c->dli[0], c->dli[1], (const double *)nullptr, 0.0, (const double *)nullptr, (const double *)nullptr,   \
             (const double *)nullptr, (const double *)nullptr, (const double *)nullptr, (double *)nullptr,          \
             (double *)nullptr, (double *)nullptr, (double *)nullptr, (unsigned long long *)nullptr, b, 0, 0u)
