@@ -16,9 +16,6 @@
 
 enum { K_R2HC = 0, K_HC2R = 1, K_REDFT01 = 4, K_REDFT10 = 5, K_REDFT11 = 6, K_RODFT01 = 8, K_RODFT10 = 9, K_RODFT11 = 10 };
 
-struct RadList {
-  int r[24];
-};
 struct LineMap {  // element e of line (l1,l2) sits at base + l1*s1 + l2*s2 + e*se
   long base, s1, s2, se;
 };
@@ -117,60 +114,6 @@ __device__ inline void bfly4(C *v, R sign) {
   v[3] = csub(d02, r);
 }
 
-// One Stockham pass of radix R over nfft complex lines of length m (LDS to LDS).
-template <typename T>
-__device__ inline void stockham_pass(const typename CT<T>::C *__restrict__ X, typename CT<T>::C *__restrict__ Y,
-                                     int nfft, int m, int R, int Ns, T sign, const typename CT<T>::C *__restrict__ tw) {
-  using C = typename CT<T>::C;
-  const int nb = m / R;
-  const int total = nfft * nb;
-  const int tstride = m / (Ns * R);
-  for (int idx = threadIdx.x; idx < total; idx += blockDim.x) {
-    const int f = idx / nb, b = idx - f * nb;
-    const C *x = X + (long)f * m;
-    C *y = Y + (long)f * m;
-    const int k = b % Ns;
-    const int base = (b / Ns) * Ns * R + k;
-    C v[16];
-    for (int t = 0; t < R; t++) {
-      C xv = x[b + t * nb];
-      if (t > 0 && k > 0) {
-        C w = tw[t * k * tstride];  // exp(-2 pi i j/m); the inverse uses its conjugate
-        if (sign > 0) w.y = -w.y;
-        xv = cmul(xv, w);
-      }
-      v[t] = xv;
-    }
-    if (R == 2) {
-      y[base] = cadd(v[0], v[1]);
-      y[base + Ns] = csub(v[0], v[1]);
-    } else if (R == 4) {
-      bfly4(v, sign);
-      for (int t = 0; t < 4; t++) y[base + t * Ns] = v[t];
-    } else if (R == 3) {
-      const T c3 = (T)0.86602540378443864676;  // sqrt(3)/2
-      const C t1 = cadd(v[1], v[2]);
-      const C t2 = mkc(v[0].x - (T)0.5 * t1.x, v[0].y - (T)0.5 * t1.y);
-      const C d = csub(v[1], v[2]);
-      const C t3 = mkc(-sign * c3 * d.y, sign * c3 * d.x);
-      y[base] = cadd(v[0], t1);
-      y[base + Ns] = cadd(t2, t3);
-      y[base + 2 * Ns] = csub(t2, t3);
-    } else {
-      const int st = m / R;
-      for (int s = 0; s < R; s++) {
-        C acc = v[0];
-        for (int t = 1; t < R; t++) {
-          const C w0 = tw[((t * s) % R) * st];
-          const C w = mkc(w0.x, sign > 0 ? -w0.y : w0.y);
-          acc = cadd(acc, cmul(v[t], w));
-        }
-        y[base + s * Ns] = acc;
-      }
-    }
-  }
-}
-
 // complex input k of packed line f, from the real lines staged in Rw (n values
 // each, rows rs apart)
 template <typename R>
@@ -242,7 +185,7 @@ __device__ inline R post_value(int kind, const ZA &Z, int g, int k, int n, int m
   switch (kind) {
     case K_R2HC: {
       const int kk = (2 * k <= n) ? k : n - k;
-      const C zk = Z(g >> 1, kk), znk = Z(g >> 1, (m - kk) % m);
+      const C zk = Z(g >> 1, kk), znk = Z(g >> 1, kk == 0 ? 0 : m - kk);
       R re, im;
       if ((g & 1) == 0) { re = (R)0.5 * (zk.x + znk.x); im = (R)0.5 * (zk.y - znk.y); }
       else { re = (R)0.5 * (zk.y + znk.y); im = (R)0.5 * (znk.x - zk.x); }
@@ -252,7 +195,7 @@ __device__ inline R post_value(int kind, const ZA &Z, int g, int k, int n, int m
     case K_REDFT10:
     case K_RODFT10: {
       const int kk = (kind == K_REDFT10) ? k : n - 1 - k;
-      const C zk = Z(g >> 1, kk), znk = Z(g >> 1, (m - kk) % m);
+      const C zk = Z(g >> 1, kk), znk = Z(g >> 1, kk == 0 ? 0 : m - kk);
       R re, im;
       if ((g & 1) == 0) { re = (R)0.5 * (zk.x + znk.x); im = (R)0.5 * (zk.y - znk.y); }
       else { re = (R)0.5 * (zk.y + znk.y); im = (R)0.5 * (znk.x - zk.x); }
@@ -293,71 +236,235 @@ __device__ inline void store_out(TO *dst, long a, R val, double scale, int accum
   else dst[a] = (TO)s;
 }
 
-// Batched r2r line transform: G lines per block, all in LDS. R is the
-// arithmetic type, TI/TO the element types of the input and output arrays.
-template <typename R, typename TI, typename TO>
-__global__ void __launch_bounds__(256) k_r2r(const TI *__restrict__ src, LineMap in, TO *__restrict__ dst,
-                                             LineMap out, int L1, int n, int m, int kind, int G, double scale,
-                                             int accum, const typename CT<R>::C *__restrict__ tw,
-                                             const typename CT<R>::C *__restrict__ q,
-                                             const typename CT<R>::C *__restrict__ t2, int nrad, RadList rl,
-                                             Batch bt) {
+// padded position of complex c in an LDS row
+template <int SH>
+__device__ __forceinline__ int lds_pad(int c) {
+  return c + (c >> SH);
+}
+
+// Line transforms of any length (primes up to 13, m <= 2048): the plan of one
+// launch. Divisions by the run-time lengths go through multipliers
+// ceil(2^32 / d) (gen_div; exact for the indices here, below 2^13).
+constexpr int GEN_NT = 256, GEN_NP = 2560, GEN_PASSES = 12;
+struct GenPlan {
+  int G, nfft;          // real lines and packed complex lines per block
+  int mp, rs;           // LDS row strides: padded complex lines, staged real lines
+  int nrad;
+  unsigned md_n, md_G, md_m;
+  struct {
+    int r, ns, nb, ts;  // radix, stride, butterflies per line, twiddle stride
+    unsigned md_nb, md_ns;
+  } p[GEN_PASSES];
+};
+static unsigned gen_magic(int d) { return d == 1 ? 0u : 0xffffffffu / (unsigned)d + 1u; }
+__device__ __forceinline__ int gen_div(int x, unsigned magic) { return magic ? (int)__umulhi((unsigned)x, magic) : x; }
+
+// One Stockham pass of radix R over nfft complex lines in LDS, in place:
+// every thread holds the points of its (at most U) butterflies in registers
+// between the barriers. The radix is fixed at compile time, so the points
+// stay in registers (as a run-time radix they went through scratch memory).
+template <int R, int U, typename T>
+__device__ __forceinline__ void gen_pass(typename CT<T>::C *__restrict__ Z, const GenPlan &gp, int s, T sign,
+                                         const typename CT<T>::C *__restrict__ tw) {
+  using C = typename CT<T>::C;
+  constexpr int SH = sizeof(C) == 16 ? 3 : 4;
+  const int nb = gp.p[s].nb, Ns = gp.p[s].ns, ts = gp.p[s].ts, total = gp.nfft * nb;
+  C v[U][R];
+  int at[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int idx = (int)threadIdx.x + u * GEN_NT;
+    at[u] = 0;
+    if (idx < total) {
+      const int f = gen_div(idx, gp.p[s].md_nb), b = idx - f * nb;
+      const int bq = gen_div(b, gp.p[s].md_ns), k = b - bq * Ns;
+      const C *x = Z + f * gp.mp;
+      at[u] = bq * Ns * R + k;
+#pragma unroll
+      for (int t = 0; t < R; t++) {
+        C xv = x[lds_pad<SH>(b + t * nb)];
+        if (t > 0 && k > 0) {
+          C w = tw[t * k * ts];  // exp(-2 pi i j/m); the inverse uses its conjugate
+          if (sign > 0) w.y = -w.y;
+          xv = cmul(xv, w);
+        }
+        v[u][t] = xv;
+      }
+      if constexpr (R == 2) {
+        const C a = v[u][0], c = v[u][1];
+        v[u][0] = cadd(a, c);
+        v[u][1] = csub(a, c);
+      } else if constexpr (R == 4) {
+        bfly4(v[u], sign);
+      } else if constexpr (R == 3) {
+        const T c3 = (T)0.86602540378443864676;  // sqrt(3)/2
+        const C x0 = v[u][0], t1 = cadd(v[u][1], v[u][2]);
+        const C t2 = mkc(x0.x - (T)0.5 * t1.x, x0.y - (T)0.5 * t1.y);
+        const C d = csub(v[u][1], v[u][2]);
+        const C t3 = mkc(-sign * c3 * d.y, sign * c3 * d.x);
+        v[u][0] = cadd(x0, t1);
+        v[u][1] = cadd(t2, t3);
+        v[u][2] = csub(t2, t3);
+      } else {
+        const int st = nb;  // m / R
+        C o[R];
+#pragma unroll
+        for (int h = 0; h < R; h++) {
+          C acc = v[u][0];
+#pragma unroll
+          for (int t = 1; t < R; t++) {
+            const C w0 = tw[((t * h) % R) * st];
+            acc = cadd(acc, cmul(v[u][t], mkc(w0.x, sign > 0 ? -w0.y : w0.y)));
+          }
+          o[h] = acc;
+        }
+#pragma unroll
+        for (int h = 0; h < R; h++) v[u][h] = o[h];
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int idx = (int)threadIdx.x + u * GEN_NT;
+    if (idx < total) {
+      C *y = Z + gen_div(idx, gp.p[s].md_nb) * gp.mp;
+#pragma unroll
+      for (int t = 0; t < R; t++) y[lds_pad<SH>(at[u] + t * Ns)] = v[u][t];
+    }
+  }
+  __syncthreads();
+}
+
+// Batched r2r line transform of any length: G lines per block in one LDS
+// buffer of complex lines. R is the arithmetic type, TI/TO the element types
+// of the input and output arrays; SRC: the source evaluated in the load (fs).
+// The forward kinds' packing is a permutation and is done by the load; the
+// others stage the real lines and pack from there. The lengths are run-time
+// values, so what bounds this kernel is the index arithmetic and LDS passes
+// of an ordinary grid and one memory latency of a small one: the loads are
+// issued four at a time, and the launcher takes few lines per block. Against
+// a kernel whose butterflies took their radix at run time (points in scratch
+// memory), with two LDS buffers and one load at a time: 90x75x130 46-53 ->
+// 19-22 us a transform, 150x98x126 58-71 -> 29-36 us, 192x192x256 about 280
+// -> 68-73 us (2.2 TB/s).
+template <typename R, typename TI, typename TO, bool SRC>
+__global__ void __launch_bounds__(GEN_NT) k_r2r(const TI *__restrict__ src, LineMap in, TO *__restrict__ dst,
+                                                LineMap out, int L1, int n, int m, int kind, double scale, int accum,
+                                                const typename CT<R>::C *__restrict__ tw,
+                                                const typename CT<R>::C *__restrict__ q,
+                                                const typename CT<R>::C *__restrict__ t2, GenPlan gp, FillSrc fs,
+                                                Batch bt) {
   using C = typename CT<R>::C;
+  constexpr int SH = sizeof(C) == 16 ? 3 : 4;
   if (bt.src) {
     src = (const TI *)bt.src[blockIdx.z];
     dst = (TO *)bt.dst[blockIdx.z];
   }
   extern __shared__ double2 smem_raw[];
-  C *smem = (C *)smem_raw;
-  const bool quarter = kind_is_quarter(kind);
-  const int nfft = quarter ? G : G / 2;
-  C *A = smem;
-  C *B = smem + (long)nfft * m;
-  R *Rw = (R *)B;  // raw staging, G*n values
+  C *Z = (C *)smem_raw;
+  R *Rw = (R *)smem_raw;  // staged real lines, overlaid by the complex lines
+  const int G = gp.G, tid = threadIdx.x;
   const int l1_0 = blockIdx.x * G;
   const long l2 = blockIdx.y;
   const int gcount = min(G, L1 - l1_0);
   const int tot = G * n;
+  const bool direct = kind == K_R2HC || kind == K_REDFT10 || kind == K_RODFT10;
   // 1. load the G lines
-  for (int idx = threadIdx.x; idx < tot; idx += blockDim.x) {
-    int g, e;
-    if (in.se == 1) { g = idx / n; e = idx - g * n; }
-    else { e = idx / G; g = idx - e * G; }
-    Rw[g * n + e] = (g < gcount) ? (R)src[in.base + (long)(l1_0 + g) * in.s1 + l2 * in.s2 + (long)e * in.se] : (R)0.0;
+  double vmax = 0.0;
+  for (int i0 = tid; i0 < tot; i0 += 4 * GEN_NT) {
+    R val[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int idx = i0 + r * GEN_NT;
+      int g, e;
+      if (in.se == 1) { g = gen_div(idx, gp.md_n); e = idx - g * n; }
+      else { e = gen_div(idx, gp.md_G); g = idx - e * G; }
+      val[r] = (R)0.0;
+      if (idx < tot && g < gcount) {
+        const long a = in.base + (long)(l1_0 + g) * in.s1 + l2 * in.s2 + (long)e * in.se;
+        if constexpr (SRC) {
+          const double sv = src_value(fs, a, (int)l2 + 1);
+          vmax = fmax(vmax, fabs(sv));
+          val[r] = (R)sv;
+        } else {
+          val[r] = (R)src[a];
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int idx = i0 + r * GEN_NT;
+      if (idx >= tot) break;
+      int g, e;
+      if (in.se == 1) { g = gen_div(idx, gp.md_n); e = idx - g * n; }
+      else { e = gen_div(idx, gp.md_G); g = idx - e * G; }
+      if (direct) {  // pre_value's packing: element e of line g is a component of complex k of line g/2
+        int k = e;
+        R x = val[r];
+        if (kind != K_R2HC) {
+          k = (e & 1) ? n - 1 - (e >> 1) : e >> 1;
+          if (kind == K_RODFT10 && (e & 1)) x = -x;
+        }
+        ((R *)(Z + (g >> 1) * gp.mp + lds_pad<SH>(k)))[g & 1] = x;
+      } else {
+        Rw[g * gp.rs + e] = val[r];
+      }
+    }
   }
+  if (SRC && fs.rmax) slots_max(fs.rmax, vmax, (blockIdx.x + gridDim.x * blockIdx.y) * (GEN_NT / 64) + tid / 64);
   __syncthreads();
-  // 2. pre-processing into complex lines
-  const int totc = nfft * m;
-  for (int idx = threadIdx.x; idx < totc; idx += blockDim.x) {
-    const int f = idx / m, k = idx - f * m;
-    A[idx] = pre_value<R>(kind, Rw, f, k, n, q, n);
-  }
-  __syncthreads();
-  // 3. complex FFT passes
-  const R sign = kind_is_forward(kind) ? (R)-1.0 : (R)1.0;
-  C *cur = A, *oth = B;
-  int Ns = 1;
-  for (int s = 0; s < nrad; s++) {
-    const int Rd = rl.r[s];
-    stockham_pass<R>(cur, oth, nfft, m, Rd, Ns, sign, tw);
+  // 2. pre-processing of the staged kinds into complex lines
+  if (!direct) {
+    constexpr int U = GEN_NP / GEN_NT;
+    const int totc = gp.nfft * m;
+    C v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int idx = tid + u * GEN_NT;
+      if (idx < totc) {
+        const int f = gen_div(idx, gp.md_m);
+        v[u] = pre_value<R>(kind, Rw, f, idx - f * m, n, q, gp.rs);
+      }
+    }
     __syncthreads();
-    C *t = cur; cur = oth; oth = t;
-    Ns *= Rd;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int idx = tid + u * GEN_NT;
+      if (idx < totc) {
+        const int f = gen_div(idx, gp.md_m);
+        Z[f * gp.mp + lds_pad<SH>(idx - f * m)] = v[u];
+      }
+    }
+    __syncthreads();
   }
-  // 4. post-processing into real lines
-  R *O = (R *)oth;
-  for (int idx = threadIdx.x; idx < tot; idx += blockDim.x) {
-    const int g = idx / n, k = idx - g * n;
-    O[idx] = post_value<R>(kind, [&](int row, int c) { return cur[(long)row * m + c]; }, g, k, n, m, q, t2);
+  // 3. complex FFT passes (at most ceil(GEN_NP / (GEN_NT R)) butterflies a thread)
+  const R sign = kind_is_forward(kind) ? (R)-1.0 : (R)1.0;
+  for (int s = 0; s < gp.nrad; s++) {
+    switch (gp.p[s].r) {
+      case 2: gen_pass<2, 5, R>(Z, gp, s, sign, tw); break;
+      case 3: gen_pass<3, 4, R>(Z, gp, s, sign, tw); break;
+      case 4: gen_pass<4, 3, R>(Z, gp, s, sign, tw); break;
+      case 5: gen_pass<5, 2, R>(Z, gp, s, sign, tw); break;
+      case 7: gen_pass<7, 2, R>(Z, gp, s, sign, tw); break;
+      case 11: gen_pass<11, 1, R>(Z, gp, s, sign, tw); break;
+      default: gen_pass<13, 1, R>(Z, gp, s, sign, tw); break;
+    }
   }
-  __syncthreads();
-  // 5. store
-  for (int idx = threadIdx.x; idx < tot; idx += blockDim.x) {
-    int g, e;
-    if (out.se == 1) { g = idx / n; e = idx - g * n; }
-    else { e = idx / G; g = idx - e * G; }
-    if (g < gcount) store_out(dst, out.base + (long)(l1_0 + g) * out.s1 + l2 * out.s2 + (long)e * out.se, O[g * n + e],
-                              scale, accum);
+  // 4. post-processing and store
+  for (int i0 = tid; i0 < tot; i0 += 4 * GEN_NT) {
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int idx = i0 + r * GEN_NT;
+      int g, e;
+      if (out.se == 1) { g = gen_div(idx, gp.md_n); e = idx - g * n; }
+      else { e = gen_div(idx, gp.md_G); g = idx - e * G; }
+      if (idx < tot && g < gcount) {
+        const R val = post_value<R>(kind, [&](int row, int c) { return Z[row * gp.mp + lds_pad<SH>(c)]; }, g, e, n, m,
+                                    q, t2);
+        store_out(dst, out.base + (long)(l1_0 + g) * out.s1 + l2 * out.s2 + (long)e * out.se, val, scale, accum);
+      }
+    }
   }
 }
 
@@ -406,12 +513,6 @@ struct P2Shape {
   static constexpr size_t LDSR = (size_t)G * RS * sizeof(R);
   static constexpr size_t LDS = LDSC > LDSR ? LDSC : LDSR;
 };
-// padded position of complex c in an LDS row
-template <int SH>
-__device__ __forceinline__ int lds_pad(int c) {
-  return c + (c >> SH);
-}
-
 // (WPE: the waves per SIMD its registers must allow; 8 for array sources, a
 // level the LDS allows too, 1 (no cap) for computed sources, whose loads
 // need more registers: only the WPE 1 instances read fs. KIND: the r2r kind
@@ -1081,8 +1182,8 @@ __global__ void __launch_bounds__(64) k_thomas_periodic_pc(T *__restrict__ W, do
   }
 }
 
-// the source of a forward x transform evaluated into x lines of W (the
-// general path for lengths k_r2r_p2 does not cover)
+// a transform's source evaluated into x lines of W, and the maximum of its
+// magnitude (the residual of a finished solve)
 template <typename T>
 __global__ void k_src_lines(fz_dims d, FillSrc fs, T *__restrict__ W) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
@@ -1430,6 +1531,61 @@ extern "C" int fz_initsolver(fz_ctx *ctx, const double bcpre[6], double *lambdax
   return FZ_OK;
 }
 
+// The lines of one block of k_r2r: at most GEN_NP complex points. Lines
+// strided in memory take 128 bytes of adjacent lines where those fit (a
+// narrower row segment wastes the rest of its cache lines), contiguous ones
+// about a thousand points; both fewer where the launch would not give every
+// CU two blocks, since a block's chain of passes is then all that counts.
+// (lines are packed in pairs, so G is even and pairs are those of any G)
+template <typename R>
+static GenPlan gen_plan(const fz_ctx *ctx, const fz_fftplan &P, int kind, bool strided, int L1, int L2, int nbatch) {
+  const bool quarter = kind_is_quarter(kind);
+  const int step = quarter ? 1 : 2, per = quarter ? P.m : P.m / 2;  // complex points a line adds
+  auto fit = [&](int g) { g -= g % step; return g < step ? step : g; };
+  int most = quarter ? GEN_NP / P.m : 2 * (GEN_NP / P.m);
+  if (most > 64) most = 64;
+  int G = strided ? 128 / (int)sizeof(R) : 1024 / (per > 0 ? per : 1);
+  G = fit(G < most ? G : most);
+  if (strided && P.m <= 16) G = fit(most);
+  const long want = 2L * ctx->ncu, low = strided ? 64 / (long)sizeof(R) : step;
+  while (G / 2 >= low && (long)((L1 + G - 1) / G) * L2 * nbatch < want && G * per > 256) G = fit(G / 2);
+  GenPlan gp;
+  memset(&gp, 0, sizeof(gp));
+  constexpr int SH = sizeof(typename CT<R>::C) == 16 ? 3 : 4;
+  gp.G = G;
+  gp.nfft = quarter ? G : G / 2;
+  gp.mp = (P.m + (P.m >> SH)) | 1;
+  gp.rs = P.n | 1;
+  gp.nrad = P.nrad;
+  gp.md_n = gen_magic(P.n);
+  gp.md_G = gen_magic(G);
+  gp.md_m = gen_magic(P.m);
+  int ns = 1;
+  for (int s = 0; s < P.nrad; s++) {
+    const int r = P.rad[s];
+    gp.p[s].r = r;
+    gp.p[s].ns = ns;
+    gp.p[s].nb = P.m / r;
+    gp.p[s].ts = P.m / (ns * r);
+    gp.p[s].md_nb = gen_magic(P.m / r);
+    gp.p[s].md_ns = gen_magic(ns);
+    ns *= r;
+  }
+  return gp;
+}
+template <typename R, typename TI, typename TO, bool SRC>
+static void launch_gen(fz_ctx *ctx, const char *name, const fz_fftplan &P, int kind, const TI *src, LineMap in,
+                       TO *dst, LineMap out, int L1, int L2, double scale, int accum, const FillSrc &fs,
+                       const Batch &bt) {
+  const int nbatch = bt.src ? bt.n : 1;
+  const GenPlan gp = gen_plan<R>(ctx, P, kind, in.se != 1 || out.se != 1, L1, L2, nbatch);
+  const size_t lc = (size_t)gp.nfft * gp.mp * sizeof(typename CT<R>::C), lr = (size_t)gp.G * gp.rs * sizeof(R);
+  const dim3 grid((L1 + gp.G - 1) / gp.G, L2, nbatch);
+  const PlanTabs<R> t = tabs_of(P, R());
+  FZ_LAUNCH(ctx, name, (k_r2r<R, TI, TO, SRC>), grid, dim3(GEN_NT), lc > lr ? lc : lr, src, in, dst, out, L1, P.n,
+            P.m, kind, scale, accum, t.tw, t.q, t.t2, gp, fs, bt);
+}
+
 template <typename R, typename TI, typename TO>
 static int launch_r2r(fz_ctx *ctx, const char *name, const fz_fftplan &P, int kind, const TI *src, LineMap in,
                       TO *dst, LineMap out, int L1, int L2, double scale, int accum = 0,
@@ -1446,26 +1602,7 @@ static int launch_r2r(fz_ctx *ctx, const char *name, const fz_fftplan &P, int ki
       return FZ_OK;
     }
   }
-  int G;
-  size_t lds;
-  if (quarter) {
-    G = 2048 / P.m;
-    if (G < 1) G = 1;
-    if (G > 64) G = 64;
-    lds = (size_t)G * P.m * sizeof(typename CT<R>::C) * 2;
-  } else {
-    G = 4096 / P.m;
-    if (G < 2) G = 2;
-    if (G > 64) G = 64;
-    G &= ~1;
-    lds = (size_t)(G / 2) * P.m * sizeof(typename CT<R>::C) * 2;
-  }
-  RadList rl;
-  for (int s = 0; s < 24; s++) rl.r[s] = P.rad[s];
-  dim3 grid((L1 + G - 1) / G, L2, bt.src ? bt.n : 1);
-  const PlanTabs<R> t = tabs_of(P, R());
-  FZ_LAUNCH(ctx, name, (k_r2r<R, TI, TO>), grid, dim3(256), lds, src, in, dst, out, L1, P.n, P.m, kind, G, scale,
-            accum, t.tw, t.q, t.t2, P.nrad, rl, bt);
+  launch_gen<R, TI, TO, false>(ctx, name, P, kind, src, in, dst, out, L1, L2, scale, accum, FillSrc(), bt);
   FZ_LAUNCHED();
   return FZ_OK;
 }
@@ -1516,14 +1653,14 @@ static FillSrc fill_src(fz_ctx *ctx, double dti, double rho0, const double *u, c
 
 // fillps + updt_rhs_b + solver (src/main.f90:492-496). When every boundary
 // right-hand side is zero, updt_rhs_b adds exact zeros and is skipped, and
-// fillps is evaluated inside the load of the forward x transform (power-of-two
-// x lengths); p then receives the correction pressure only. Otherwise the
-// three routines run as they are.
+// fillps is evaluated inside the load of the forward x transform (all but the
+// quarter-wave kinds); p then receives the correction pressure only. Otherwise
+// the three routines run as they are.
 int fz_projection_rhs_solve(fz_ctx *ctx, double dti, double rho0, const double *u, const double *v, const double *w,
                             double *p, const double *stc) {
   fz_poisson *P = ctx->pois;
   if (!P) return fz_set_error(FZ_ERR_STATE, "fz_solver: fz_initsolver has not been called");
-  if (!P->rhsb_zero || !p2_length(P->px.m) || kind_is_quarter(P->px.kind_f)) {
+  if (!P->rhsb_zero || kind_is_quarter(P->px.kind_f)) {
     if (stc) return fz_set_error(FZ_ERR_STATE, "fz_projection_rhs_solve: device scalars need the fused path");
     FZ_TRY(fz_fillps(ctx, dti, rho0, u, v, w, p));
     FZ_TRY(fz_updt_rhs_b(ctx, p));
@@ -1536,8 +1673,12 @@ int fz_projection_rhs_solve(fz_ctx *ctx, double dti, double rho0, const double *
   const LineMap w_x = {0, n1, ps, 1};
   FillSrc fs = fill_src(ctx, dti, rho0, u, v, w);
   fs.stc = stc;
-  dispatch_p2<false, double, double, double>(ctx, "fillps_fft_x_fwd", P->px, P->px.kind_f, (const double *)nullptr,
-                                             p_x, P->work, w_x, n2, n3, 1.0, 0, fs);
+  if (p2_length(P->px.m))
+    dispatch_p2<false, double, double, double>(ctx, "fillps_fft_x_fwd", P->px, P->px.kind_f, (const double *)nullptr,
+                                               p_x, P->work, w_x, n2, n3, 1.0, 0, fs);
+  else
+    launch_gen<double, double, double, true>(ctx, "fillps_fft_x_fwd", P->px, P->px.kind_f, (const double *)nullptr,
+                                             p_x, P->work, w_x, n2, n3, 1.0, 0, fs, kNoBatch);
   FZ_LAUNCHED();
   return solver_rest<double>(ctx, P->work, p, 0);
 }
@@ -1630,7 +1771,7 @@ static int mixed_buffers(fz_ctx *ctx) {
 }
 
 // one FP32 solve of the source fs: forward x transform of the source (fused
-// into the load for power-of-two lengths), the rest in FP32; the result is
+// into the load), the rest in FP32; the result is
 // written into p (accum 0) or added to it (accum 1)
 static int mixed_pass(fz_ctx *ctx, const FillSrc &fs, double *p, int accum) {
   fz_poisson *P = ctx->pois;
@@ -1641,20 +1782,16 @@ static int mixed_pass(fz_ctx *ctx, const FillSrc &fs, double *p, int accum) {
   const LineMap w_x = {0, n1, ps, 1};
   float *W = P->work32;
   const char *name = fs.on == SRC_FILLPS ? "fillps_fft_x_fwd_f32" : (fs.on == SRC_B ? "fft_x_fwd_f32" : "residual_fft_x_fwd_f32");
-  bool fused = false;
-  if (p2_length(P->px.m)) {
-    fused = kind_is_quarter(P->px.kind_f)
-                ? dispatch_p2<true, float, double, float>(ctx, name, P->px, P->px.kind_f, (const double *)nullptr, p_x,
-                                                          W, w_x, n2, n3, 1.0, 0, fs)
-                : dispatch_p2<false, float, double, float>(ctx, name, P->px, P->px.kind_f, (const double *)nullptr,
-                                                           p_x, W, w_x, n2, n3, 1.0, 0, fs);
-    FZ_LAUNCHED();
-  }
-  if (!fused) {
-    FZ_LAUNCH(ctx, "src_lines_f32", k_src_lines<float>, fz_grid_interior(ctx->d), fz_block3(), 0, ctx->d, fs, W);
-    FZ_LAUNCHED();
-    FZ_TRY((launch_r2r<float, float, float>(ctx, "fft_x_fwd_f32", P->px, P->px.kind_f, W, w_x, W, w_x, n2, n3, 1.0)));
-  }
+  if (!p2_length(P->px.m))
+    launch_gen<float, double, float, true>(ctx, name, P->px, P->px.kind_f, (const double *)nullptr, p_x, W, w_x, n2,
+                                           n3, 1.0, 0, fs, kNoBatch);
+  else if (kind_is_quarter(P->px.kind_f))
+    dispatch_p2<true, float, double, float>(ctx, name, P->px, P->px.kind_f, (const double *)nullptr, p_x, W, w_x, n2,
+                                            n3, 1.0, 0, fs);
+  else
+    dispatch_p2<false, float, double, float>(ctx, name, P->px, P->px.kind_f, (const double *)nullptr, p_x, W, w_x, n2,
+                                             n3, 1.0, 0, fs);
+  FZ_LAUNCHED();
   return solver_rest<float>(ctx, W, p, accum);
 }
 
@@ -1700,7 +1837,7 @@ int fz_projection_device_scalars_ok(fz_ctx *ctx, int mixed) {
   fz_poisson *P = ctx->pois;
   if (!P) return 0;
   if (mixed) return 1;
-  return P->rhsb_zero && p2_length(P->px.m) && !kind_is_quarter(P->px.kind_f);
+  return P->rhsb_zero && !kind_is_quarter(P->px.kind_f);
 }
 
 __global__ void k_slots_max(unsigned long long *__restrict__ slots, double *__restrict__ out) {
