@@ -87,6 +87,12 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
   // below that, the FP64 solve of a non-periodic z reads pivots made once at
   // set-up (two more N-element arrays; 294 against 330 us at 256x256x512)
   c->thomas_pre = c->thomas_rc ? 0 : 1;
+  // (a chunked kernel asked for by name is the one that runs)
+  if (getenv("FZ_THOMAS_RC") || getenv("FZ_THOMAS_PRE") || getenv("FZ_THOMAS_ROWS64") || getenv("FZ_THOMAS_ROWS32")) {
+    c->thomas_reg = 0;
+    c->tk64 = 16;
+    c->tk32 = -8;
+  }
   if (const char *e = getenv("FZ_THOMAS_RC")) c->thomas_rc = atoi(e);
   if (const char *e = getenv("FZ_THOMAS_PRE")) c->thomas_pre = atoi(e);
   if (const char *e = getenv("FZ_THOMAS_ROWS32")) c->tk32 = atoi(e);

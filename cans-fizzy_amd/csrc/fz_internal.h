@@ -54,6 +54,7 @@ struct fz_poisson {
   double normfft = 1.0;
   double *lambdaxy = nullptr;  // device n1*n2
   double *a = nullptr, *b = nullptr, *c = nullptr;  // device n3
+  double *apad = nullptr, *cpad = nullptr;          // a and c padded for k_thomas_reg
   double *rhsbx = nullptr, *rhsby = nullptr, *rhsbz = nullptr;  // device
   double *work = nullptr;   // spectral buffer, n1*n2*n3
   double *piv = nullptr;    // Thomas pivots, n1*n2*n3
@@ -61,6 +62,7 @@ struct fz_poisson {
   double *zpre = nullptr;   // non-periodic z with precomputed pivots: 1/pivot and d of every row, n1*n2*n3
   double *dpre = nullptr;   // each
   int periodic_z = 0;
+  int zper = 0;        // periodic z: piv holds the reciprocal pivots of the first n3-1 rows (k_thomas_reg)
   int rhsb_zero = 0;  // all boundary right-hand sides vanish (homogeneous pressure BCs)
   long null_col = -1;  // spectral column of the operator's null mode, or -1
   float *work32 = nullptr;              // FP32 spectral buffer of the mixed-precision solve
@@ -101,9 +103,11 @@ struct fz_ctx {
   // launch parameters (defaults, environment overrides, or fz_case_autotune)
   int mom_variant = 0;  // momentum kernel: 0 the default (8), 1 staged
                         // loads, 2 plain, 4 or 5 waves per EU, 8 stencil fields in LDS (k_mom_lds)
-  int tk64 = 16;        // rows per chunk of the FP64 Thomas kernel: 8, 16 or 32
-  int tk32 = -8;        // the same for the FP32 one; negative: two columns per lane, -8 or -16 (the default,
-                        // -8, is the tuner's choice at 256x256x512 and 256^3)
+  int tk64 = 0;         // FP64 Thomas kernel: 0 the columns in registers (k_thomas_reg, where they fit and the
+                        // pivots are made at set-up, else 16), or 8, 16 or 32 rows per chunk
+  int tk32 = 0;         // the same for the FP32 one; negative: two columns per lane, -8 or -16 rows per chunk
+                        // (-8 where the columns do not fit in registers)
+  int thomas_reg = 1;   // 0: periodic z keeps its chunked kernel too
   int acdi_variant = 0;  // ACDI step: 0 the default (3), 1 fields staged in LDS, 2 one cell per thread, 3 each face once
   int youngs_variant = 0;  // Youngs kernel: 0 the default (FP32 1, FP64 3), 1 marching in z, 2 one cell per thread,
                            // 3 marching without range checks when the range flag allows, else one cell per thread

@@ -946,7 +946,7 @@ __global__ void k_piv_pre(double *__restrict__ Z, double *__restrict__ D, const 
     const double z = l == 0 ? 1.0 / (bb + FZ_EPS) : 1.0 / (bb - a[l] * d + FZ_EPS);
     d = (l == 0 ? c[0] : c[l]) * z;
     Z[idx + (long)l * ps] = z;
-    D[idx + (long)l * ps] = d;
+    if (D) D[idx + (long)l * ps] = d;
   }
 }
 
@@ -1182,6 +1182,183 @@ __global__ void __launch_bounds__(64) k_thomas_periodic_pc(T *__restrict__ W, do
   }
 }
 
+// an array of n elements through a buffer resource (an access takes one 32-bit
+// offset instead of a 64-bit address)
+template <typename T>
+struct ColBuf {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ T get(unsigned e) const {
+    if constexpr (sizeof(T) == 8)
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, e * 8u, 0u, 0));
+    else
+      return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, e * 4u, 0u, 0));
+  }
+  __device__ __forceinline__ void put(unsigned e, T v) const {
+    if constexpr (sizeof(T) == 8)
+      __builtin_amdgcn_raw_buffer_store_b64(
+          __builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b64(r, 0u, 0u, 0)), v), r, e * 8u, 0u, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b32(
+          __builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b32(r, 0u, 0u, 0)), v), r, e * 4u, 0u, 0);
+  }
+};
+template <typename T>
+__device__ __forceinline__ ColBuf<T> col_buf(const T *p, long n) {
+  return ColBuf<T>{__builtin_amdgcn_make_buffer_rsrc((void *)p, (short)0, (int)(unsigned)(n * (long)sizeof(T)),
+                                                     0x00020000)};
+}
+
+// The line solves with a block's columns held in registers: each value of W
+// is read once and written once, and the reciprocal pivots Z (k_piv_pre, made
+// at set-up) are read once, 24 bytes a row where k_thomas_pre moves 48. CB
+// adjacent columns to a block (row segments of 128 bytes), thread (g, col)
+// holding the RPT rows from g*RPT of column col and their pivots, all loaded
+// together. The elimination then runs through the groups in turn, by a shuffle
+// inside a wave and through LDS from wave to wave, and the substitution runs
+// back the same way; the other blocks of the CU load meanwhile. The chain is
+// three dependent operations a row forward and two back, the products
+// d = c z being made beside it, and everything it reads is in registers before
+// its turn (ap and cp are a and c, -1 past the end, where a row passes the
+// running value on, (0 - -1 p) 1 and 0 - -1 p, so that the chain has no
+// conditions). The arithmetic is k_thomas_pre's, and so k_thomas's, exactly:
+// eliminated values are rounded to T, and the last one starts the
+// substitution unrounded.
+// PER: gaussel_periodic with the second solve P2 made at set-up, as
+// k_thomas_periodic_pc (32 bytes a row against 88): the first n3-1 rows, then
+// the cyclic unknown and the update on the values in registers.
+// What bounds it: the bytes where the columns fill the device (256x256x512
+// 207 us against 287 for k_thomas_pre, 3.9 TB/s; 256^3 periodic 112 against
+// 212; FP32 256^3 77 against 95), the chain of a block elsewhere
+// (64x64x128 10 against 27 us, 128x128x256 FP32 25 against 69, sixteen 64^3
+// in a batch 18 against 35, whose kernel k_thomas divides per row). The
+// coefficients read from memory inside the chain instead: 313 us at
+// 256x256x512.
+template <typename T, int CB, int RPT, bool PER>
+__global__ void __launch_bounds__(1024 / (RPT / 16)) k_thomas_reg(T *__restrict__ W, const double *__restrict__ Z,
+                                                                  const double *__restrict__ P2,
+                                                                  const double *__restrict__ lambdaxy,
+                                                                  const double *__restrict__ a,
+                                                                  const double *__restrict__ b,
+                                                                  const double *__restrict__ c,
+                                                                  const double *__restrict__ ap,
+                                                                  const double *__restrict__ cp, long ps, int n3,
+                                                                  long gauge, Batch bt) {
+  constexpr int SUB = 64 / CB;  // groups of a wave
+  if (bt.src) W = (T *)bt.src[blockIdx.y];
+  __shared__ double hand[CB], last[CB];
+  const int m = PER ? n3 - 1 : n3;
+  const int tid = threadIdx.x, col = tid % CB, sub = (tid & 63) / CB, nw = (int)blockDim.x >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l0 = tid / CB * RPT;
+  const long idx = (long)fz_xcd_block(blockIdx.x, gridDim.x) * CB + col;
+  const bool on = idx < ps;
+  // (byte offsets of 32 bits, which the launcher checks; rows and columns past
+  // the last read the last, and are not written)
+  const ColBuf<T> BW = col_buf(W, ps * n3);
+  const ColBuf<double> BZ = col_buf(Z, ps * n3), BP = col_buf(P2, ps * n3);
+  const unsigned pb = (unsigned)ps, ec = (unsigned)(on ? idx : ps - 1);
+  auto at = [&](int t) { return ec + (unsigned)min(l0 + t, m - 1) * pb; };
+  T r[RPT];
+  double z[RPT];
+#pragma unroll
+  for (int t = 0; t < RPT; t++) r[t] = BW.get(at(t));
+#pragma unroll
+  for (int t = 0; t < RPT; t++) z[t] = BZ.get(at(t));
+  if (l0 + RPT > m) {
+#pragma unroll
+    for (int t = 0; t < RPT; t++) {
+      r[t] = l0 + t < m ? r[t] : (T)0;
+      z[t] = l0 + t < m ? z[t] : 1.0;
+    }
+  }
+  double wm = 0.0, q0 = 0.0, qm = 0.0, lam = 0.0;
+  if (PER && on) {
+    wm = (double)W[idx + (long)m * ps];
+    q0 = P2[idx];
+    qm = P2[idx + (long)(m - 1) * ps];
+    lam = lambdaxy[idx];
+  }
+  // the coefficients of the thread's rows, a for its elimination, then c; held
+  // in registers before its turn comes (the empty statement keeps the loads here)
+  double co[RPT];
+#pragma unroll
+  for (int t = 0; t < RPT; t++) co[t] = ap[l0 + t];
+  if (tid < CB) hand[tid] = 0.0;
+#pragma unroll
+  for (int t = 0; t < RPT; t++) asm volatile("" : "+v"(co[t]));
+  __syncthreads();
+  for (int w = 0; w < nw; w++) {
+    if (wave == w) {
+      double p = hand[col];
+#pragma unroll 1
+      for (int h = 0; h < SUB; h++) {
+        if (sub == h) {
+#pragma unroll
+          for (int t = 0; t < RPT; t++) {
+            p = ((double)r[t] - co[t] * p) * z[t];
+            r[t] = (T)p;
+          }
+        }
+        const double up = __shfl_up(p, CB, 64);
+        if (sub == h + 1) p = up;
+      }
+      if (sub == SUB - 1) hand[col] = p;
+#pragma unroll
+      for (int t = 0; t < RPT; t++) co[t] = cp[l0 + t];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int t = 0; t < RPT; t++) z[t] = co[t] * z[t];  // d
+  if (l0 + RPT >= m) {  // the last row takes the running value itself (it starts the substitution unrounded),
+                        // and so do the rows past it
+#pragma unroll
+    for (int t = 0; t < RPT; t++)
+      if (l0 + t >= m - 1) {
+        r[t] = (T)0;
+        z[t] = -1.0;
+      }
+  }
+  for (int w = nw - 1; w >= 0; w--) {
+    if (wave == w) {
+      double p = hand[col];
+      if (!PER && w == nw - 1 && idx == gauge) p = 0.0;  // (the mixed solve's pinned unknown, see k_thomas)
+      if (PER && w == nw - 1 && sub == SUB - 1) last[col] = p;
+#pragma unroll 1
+      for (int h = SUB - 1; h >= 0; h--) {
+        if (sub == h) {
+#pragma unroll
+          for (int t = RPT - 1; t >= 0; t--) {
+            p = (double)r[t] - z[t] * p;
+            r[t] = (T)p;
+          }
+        }
+        const double dn = __shfl_down(p, CB, 64);
+        if (sub == h - 1) p = dn;
+      }
+      if (sub == 0) hand[col] = p;
+      if constexpr (PER) {
+#pragma unroll
+        for (int t = 0; t < RPT; t++) z[t] = BP.get(at(t));
+      } else {
+#pragma unroll
+        for (int t = 0; t < RPT; t++)
+          if (on && l0 + t < m) BW.put(at(t), r[t]);
+      }
+    }
+    __syncthreads();
+  }
+  if constexpr (PER) {
+    const double p0 = (double)(T)hand[col], pm = (double)(T)last[col];
+    double pn = (wm - c[m] * p0 - a[m] * pm) / (b[m] + lam + c[m] * q0 + a[m] * qm + FZ_EPS);
+    if (idx == gauge) pn = 0.0;
+    if (on && l0 == 0) W[idx + (long)m * ps] = (T)pn;
+#pragma unroll
+    for (int t = 0; t < RPT; t++)
+      if (on && l0 + t < m) BW.put(at(t), (T)((double)r[t] + z[t] * pn));
+  }
+}
+
 // a transform's source evaluated into x lines of W, and the maximum of its
 // magnitude (the residual of a finished solve)
 template <typename T>
@@ -1400,8 +1577,8 @@ int fz_poisson_destroy(fz_poisson *p) {
   if (!p) return FZ_OK;
   fftplan_free(&p->px);
   fftplan_free(&p->py);
-  double *bufs[9] = {p->lambdaxy, p->a, p->b, p->c, p->rhsbx, p->rhsby, p->rhsbz, p->work, p->piv};
-  for (int q = 0; q < 9; q++)
+  double *bufs[11] = {p->lambdaxy, p->a, p->b, p->c, p->rhsbx, p->rhsby, p->rhsbz, p->work, p->piv, p->apad, p->cpad};
+  for (int q = 0; q < 11; q++)
     if (bufs[q]) (void)hipFree(bufs[q]);
   if (p->aux) (void)hipFree(p->aux);
   if (p->zpre) (void)hipFree(p->zpre);
@@ -1413,6 +1590,10 @@ int fz_poisson_destroy(fz_poisson *p) {
   delete p;
   return FZ_OK;
 }
+
+template <typename T>
+static bool reg_fits(const fz_ctx *ctx);
+constexpr int REG_PAD = 128;  // a k_thomas_reg block's rows past the last one are fewer
 
 extern "C" int fz_initsolver(fz_ctx *ctx, const double bcpre[6], double *lambdaxy_h, double *a_h, double *b_h,
                              double *c_h, double *normfft_h, double *rhsbx_h, double *rhsby_h, double *rhsbz_h) {
@@ -1494,13 +1675,18 @@ extern "C" int fz_initsolver(fz_ctx *ctx, const double bcpre[6], double *lambdax
     return rc;
   }
   const size_t N = (size_t)n1 * n2 * n3;
+  // a and c for k_thomas_reg: of the rows it eliminates, then -1 to the end of a block's groups
+  const int mreg = P->periodic_z ? n3 - 1 : n3;
+  std::vector<double> apad(a.begin(), a.begin() + mreg), cpad(c.begin(), c.begin() + mreg - 1);
+  apad.resize(mreg + REG_PAD, -1.0);
+  cpad.resize(mreg + REG_PAD, -1.0);
   struct {
     double **d;
     const std::vector<double> *h;
-  } up[7] = {{&P->lambdaxy, &lxy}, {&P->a, &a}, {&P->b, &b}, {&P->c, &c}, {&P->rhsbx, &rbx}, {&P->rhsby, &rby},
-             {&P->rhsbz, &rbz}};
+  } up[9] = {{&P->lambdaxy, &lxy}, {&P->a, &a}, {&P->b, &b}, {&P->c, &c}, {&P->rhsbx, &rbx}, {&P->rhsby, &rby},
+             {&P->rhsbz, &rbz}, {&P->apad, &apad}, {&P->cpad, &cpad}};
   hipError_t e = hipSuccess;
-  for (int q = 0; q < 7 && e == hipSuccess; q++) {
+  for (int q = 0; q < 9 && e == hipSuccess; q++) {
     e = hipMalloc((void **)up[q].d, sizeof(double) * up[q].h->size());
     if (e == hipSuccess) e = hipMemcpy(*up[q].d, up[q].h->data(), sizeof(double) * up[q].h->size(), hipMemcpyHostToDevice);
   }
@@ -1527,6 +1713,12 @@ extern "C" int fz_initsolver(fz_ctx *ctx, const double bcpre[6], double *lambdax
     FZ_LAUNCH(ctx, "periodic_p2", k_periodic_p2, dim3((int)((ps + 255) / 256)), dim3(256), 0, P->piv, P->aux,
               P->lambdaxy, P->a, P->b, P->c, n1, n2, n3);
     FZ_LAUNCHED();
+    P->zper = ctx->thomas_reg && reg_fits<float>(ctx);  // (FP64 and FP32 solves alike)
+    if (P->zper) {  // the pivots of its n3 - 1 rows in place of the per-solve ones
+      FZ_LAUNCH(ctx, "piv_pre", k_piv_pre, dim3((int)((ps + 255) / 256)), dim3(256), 0, P->piv, (double *)nullptr,
+                P->lambdaxy, P->a, P->b, P->c, n1, n2, n3 - 1);
+      FZ_LAUNCHED();
+    }
   }
   return FZ_OK;
 }
@@ -1605,6 +1797,32 @@ static int launch_r2r(fz_ctx *ctx, const char *name, const fz_fftplan &P, int ki
   launch_gen<R, TI, TO, false>(ctx, name, P, kind, src, in, dst, out, L1, L2, scale, accum, FillSrc(), bt);
   FZ_LAUNCHED();
   return FZ_OK;
+}
+
+// whether k_thomas_reg takes columns of T: its blocks hold 1024 FP64 or 512
+// FP32 rows, and the array's byte offsets fit in 32 bits
+template <typename T>
+static bool reg_fits(const fz_ctx *ctx) {
+  return ctx->d.n3 <= (sizeof(T) == 8 ? 1024 : 512) && ctx->ni * (long)sizeof(double) < (1L << 32);
+}
+// (32 rows to a thread from 256 rows: half the turns, 213 -> 207 us at
+// 256x256x512, 124 -> 112 us at 256^3 periodic; 16 below, where the waves
+// count: 16 solves of 64^3 26 -> 18 us, 64x2x64 9 -> 7 us)
+template <typename T, bool PER>
+static void launch_thomas_reg(fz_ctx *ctx, const char *name, T *W, const double *Z, long gauge, const Batch &bt) {
+  const fz_poisson *P = ctx->pois;
+  const int n3 = ctx->d.n3, m = PER ? n3 - 1 : n3;
+  const long ps = (long)ctx->d.n1 * ctx->d.n2;
+  constexpr int CB = 128 / (int)sizeof(T);
+  const int rpt = n3 >= 256 ? 32 : 16;
+  const int nt = (CB * ((m + rpt - 1) / rpt) + 63) / 64 * 64;
+  const dim3 grid((unsigned)((ps + CB - 1) / CB), bt.src ? bt.n : 1);
+  if (rpt == 32)
+    FZ_LAUNCH(ctx, name, (k_thomas_reg<T, CB, 32, PER>), grid, dim3(nt), 0, W, Z, P->aux, P->lambdaxy, P->a, P->b,
+              P->c, P->apad, P->cpad, ps, n3, gauge, bt);
+  else
+    FZ_LAUNCH(ctx, name, (k_thomas_reg<T, CB, 16, PER>), grid, dim3(nt), 0, W, Z, P->aux, P->lambdaxy, P->a, P->b,
+              P->c, P->apad, P->cpad, ps, n3, gauge, bt);
 }
 
 // everything after the forward x transform: y transform, z solve, inverses
@@ -1696,15 +1914,17 @@ static int solver_rest(fz_ctx *ctx, T *W, double *p, int accum) {
   const LineMap w_y = {0, 1, ps, n1};
   FZ_TRY((launch_r2r<T, T, T>(ctx, mixed ? "fft_y_fwd_f32" : "fft_y_fwd", P->py, P->py.kind_f, W, w_y, W, w_y, n1, n3,
                               1.0)));
-  const int tpb = 256;
-  const int nb = (int)((ps + tpb - 1) / tpb);
   if (!P->periodic_z) {
     // rows per chunk: the context's choice (FP32 columns move half the
     // bytes per load, so their default keeps twice the rows in flight)
-    const int tk = mixed ? ctx->tk32 : ctx->tk64;
+    int tk = mixed ? ctx->tk32 : ctx->tk64;
+    const bool reg = tk == 0 && P->zpre && reg_fits<T>(ctx);
+    if (tk == 0) tk = mixed ? -8 : 16;
     const dim3 grid((int)((ps + 63) / 64)), blk(64);
     const char *name = mixed ? "thomas_f32" : "thomas";
-    if (P->zpre && tk > 0) {  // pivots made at set-up
+    if (reg) {  // columns in registers
+      launch_thomas_reg<T, false>(ctx, name, W, P->zpre, gauge, kNoBatch);
+    } else if (P->zpre && tk > 0) {  // pivots made at set-up
       if (tk == 8) FZ_LAUNCH(ctx, name, (k_thomas_pre<8, T>), grid, blk, 0, W, P->zpre, P->dpre, P->a, n1, n2, n3,
                              gauge);
       else FZ_LAUNCH(ctx, name, (k_thomas_pre<16, T>), grid, blk, 0, W, P->zpre, P->dpre, P->a, n1, n2, n3, gauge);
@@ -1734,9 +1954,9 @@ static int solver_rest(fz_ctx *ctx, T *W, double *p, int accum) {
     else FZ_LAUNCH(ctx, name, (k_thomas<16, T>), grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3,
                    gauge, kNoBatch);
   } else {
-    (void)nb;
-    (void)tpb;
-    if (mixed && ctx->tk32 < 0 && ps % 2 == 0)  // two FP32 columns per lane
+    if (P->zper)  // columns in registers
+      launch_thomas_reg<T, true>(ctx, mixed ? "thomas_periodic_f32" : "thomas_periodic", W, P->piv, gauge, kNoBatch);
+    else if (mixed && ctx->tk32 <= 0 && ps % 2 == 0)  // two FP32 columns per lane
       FZ_LAUNCH(ctx, "thomas_periodic_f32", k_thomas_periodic_x2<16>, dim3((int)((ps / 2 + 63) / 64)), dim3(64), 0,
                 (float *)(void *)W, P->piv, P->aux, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3, gauge);
     else
@@ -1985,9 +2205,12 @@ int fz_batch_solve(fz_ctx *c0, void **dptrs, int n) {
                                              p_x, (double *)nullptr, w_x, n2, n3, 1.0, 0, p_w)));
   FZ_TRY((launch_r2r<double, double, double>(c0, "fft_y_fwd_batch", P->py, P->py.kind_f, (const double *)nullptr,
                                              w_y, (double *)nullptr, w_y, n1, n3, 1.0, 0, w_w)));
-  const dim3 grid((int)((ps1 + 63) / 64), n), blk(64);
-  FZ_LAUNCH(c0, "thomas_batch", (k_thomas<16, double>), grid, blk, 0, (double *)nullptr, (double *)nullptr,
-            P->lambdaxy, P->a, P->b, P->c, n1, n2, n3, -1L, w_d);
+  // (the cases share the operator, so the first one's pivots serve all)
+  if (c0->tk64 == 0 && P->zpre && reg_fits<double>(c0))
+    launch_thomas_reg<double, false>(c0, "thomas_batch", (double *)nullptr, P->zpre, -1L, w_d);
+  else
+    FZ_LAUNCH(c0, "thomas_batch", (k_thomas<16, double>), dim3((int)((ps1 + 63) / 64), n), dim3(64), 0,
+              (double *)nullptr, (double *)nullptr, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3, -1L, w_d);
   FZ_LAUNCHED();
   FZ_TRY((launch_r2r<double, double, double>(c0, "fft_y_bwd_batch", P->py, P->py.kind_b, (const double *)nullptr,
                                              w_y, (double *)nullptr, w_y, n1, n3, 1.0, 0, w_w)));

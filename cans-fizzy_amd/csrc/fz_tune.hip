@@ -5,8 +5,9 @@
 //  - tile_y: rows of blocks per z-marching pencil in the stencil block order;
 //  - the variant of the fused momentum kernel (occupancy, staged loads,
 //    stencil fields staged in LDS);
-//  - rows per chunk of the Thomas kernel (FP64, or FP32 in mixed cases,
-//    where two columns per lane are a candidate too);
+//  - the Thomas kernel: the columns in registers, or chunks of 8, 16 or 32
+//    rows (FP64, or FP32 in mixed cases, where two columns per lane are a
+//    candidate too);
 //  - for a non-periodic z, the Thomas kernel without a pivot array (it
 //    reads a column twice instead of storing and reloading pivots).
 // A scratch case with the same parameters (dt checks off, so every trial
@@ -94,7 +95,7 @@ extern "C" int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size
     if (rc == FZ_OK) rc = fz_case_init(sc);
     if (rc == FZ_OK && hipEventCreate(&a) != hipSuccess) rc = fz_set_error(FZ_ERR_HIP, "hipEventCreate");
     if (rc == FZ_OK && hipEventCreate(&b) != hipSuccess) rc = fz_set_error(FZ_ERR_HIP, "hipEventCreate");
-    best = {c ? c->d.tile_y : 8, c ? c->mom_variant : 0, proj32 ? (c ? c->tk32 : -8) : (c ? c->tk64 : 16),
+    best = {c ? c->d.tile_y : 8, c ? c->mom_variant : 0, c ? (proj32 ? c->tk32 : c->tk64) : 0,
             c ? c->thomas_rc : 0, 0.0f};
     if (rc == FZ_OK) rc = trial(sc, c, best, proj32, trial_steps, a, b, &best.ms);
     const int tiles[] = {0, 2, 4, 8, 16};
@@ -105,7 +106,7 @@ extern "C" int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size
     for (int dim = 0; dim < 4 && rc == FZ_OK; dim++) {
       const int *cand = dim == 0 ? tiles : (dim == 1 ? moms : (dim == 2 ? tks : rcs));
       int ncand = dim == 0 ? 5 : (dim == 1 ? 5 : (dim == 2 ? (proj32 ? 5 : 3) : 2));
-      if (dim == 3 && (periodic_z || best.tk < 0)) ncand = 0;  // no such kernel there
+      if (dim == 3 && (periodic_z || best.tk <= 0)) ncand = 0;  // no such kernel there
       for (int q = 0; q < ncand && rc == FZ_OK; q++) {
         Tuned t = best;
         int &field = dim == 0 ? t.tile_y : (dim == 1 ? t.mom_variant : (dim == 2 ? t.tk : t.rc));
@@ -126,7 +127,7 @@ extern "C" int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size
   fz_case_drop_graphs(cs);  // captured launches carry the old parameters
   if (report && cap > 0)
     snprintf(report, cap, "tile_y=%d mom_variant=%d thomas_rows=%d%s ms_per_step=%.4f%s", best.tile_y,
-             best.mom_variant, best.tk < 0 ? -best.tk : best.tk, best.tk < 0 ? "x2" : (best.rc ? "rc" : ""), best.ms,
+             best.mom_variant, best.tk < 0 ? -best.tk : (best.tk ? best.tk : 16), best.tk < 0 ? "x2" : (best.rc ? "rc" : ""), best.ms,
              cached ? " (cached)" : "");
   return FZ_OK;
 }

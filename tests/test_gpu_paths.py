@@ -3,6 +3,8 @@
 The z-marching kernels (momentum, ACDI step, correction, normals) take their
 planes per block from the grid; FZ_MARCH_PLANES, read when a context is made,
 fixes the number. Every number gives the same fields bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -94,3 +96,39 @@ def test_ragged_steps_match_the_oracle(name, graphs):
             assert max(errs.values()) <= 1e-12, (step, errs)
     finally:
         dc.close()
+
+
+def solve(n, cbc, f, mixed, count=1):
+    ctxs = [F.Context(n, [1.0, 0.9, 1.7], cbc, gr=0.6 if cbc[4:] != "PP" else 0.0) for _ in range(count)]
+    try:
+        ds = []
+        for c in ctxs:
+            F.call("fz_initsolver", c.h, None, None, None, None, None, None, None, None, None)
+            ds.append(c.halo(f))
+        if count > 1:
+            F.call("fz_solver_batched", (C.c_void_p * count)(*[c.h.value for c in ctxs]),
+                   (C.c_void_p * count)(*[d.ptr.value for d in ds]), count)
+        elif mixed:
+            F.call("fz_solver_mixed", ctxs[0].h, ds[0].ptr, 0.0, 2, C.byref(C.c_int()), None)
+        else:
+            F.call("fz_solver", ctxs[0].h, ds[0].ptr)
+        return ds[-1].download()[1:-1, 1:-1, 1:-1]
+    finally:
+        for c in ctxs:
+            c.close()
+
+
+@pytest.mark.parametrize("n3", [2, 3, 15, 16, 17, 32, 33, 64, 65, 127, 255, 256, 257, 258, 511, 512, 513, 1024, 1025])
+@pytest.mark.parametrize("cbc", ["PPPPNN", "NNPPDD", "PPPPPP"])
+def test_columns_in_registers_match_the_chunked_kernels(n3, cbc, rng, monkeypatch):
+    """Both sides of a thread's, a wave's and a block's rows, and column
+    counts that are no multiple of a block's, in FP64, mixed precision and
+    (non-periodic z) as a batch, against the chunked kernels bit for bit."""
+    for n in ([6, 5, n3], [16, 4, n3]):
+        f = np.asfortranarray(rng.uniform(-1.0, 1.0, [x + 2 for x in n]))
+        kinds = [(False, 1), (True, 1)] + ([(False, 3)] if cbc != "PPPPPP" else [])
+        for mixed, count in kinds:
+            monkeypatch.delenv("FZ_THOMAS_ROWS64", raising=False)
+            got = solve(n, cbc, f, mixed, count)
+            monkeypatch.setenv("FZ_THOMAS_ROWS64", "16")
+            assert np.array_equal(got, solve(n, cbc, f, mixed, count), equal_nan=True), (n, mixed, count)
