@@ -22,6 +22,16 @@ int fz_launch_rk_mom(fz_ctx *c, double f1, double f2, const double rho12[2], con
                      const double *dwo, double *u, double *v, double *w);
 int fz_launch_rk_oth(fz_ctx *c, double f12, const double rho12[2], const double *psi, const double *du,
                      const double *dv, const double *dw, double *u, double *v, double *w);
+int fz_launch_rk_fused(fz_ctx *c, const double rho12[2], const double mu12[2], double factor1, double factor2,
+                       int first, double dt_r, double sigma, double rho0, const double bforce[3],
+                       const double gacc[3], const double rho_av[3], const double *fx, const double *fy,
+                       const double *fz, const double *psi, const double *psio, const double *p, const double *pn,
+                       const double *po, const double *kappa, double *duo, double *dvo, double *dwo, double *un,
+                       double *vn, double *wn, double *u, double *v, double *w);
+int fz_launch_rk_2fl_fused(fz_ctx *c, double factor1, double factor2, int first, double gam, double seps,
+                           double beta, int vof, const double *u, const double *v, const double *w, const double *nx,
+                           const double *ny, const double *nz, const double *phi, double *dpsio, double *ps,
+                           double *psi, double *fx, double *fy, double *fz);
 template <typename PT, typename HT>
 int fz_launch_mom_fused(fz_ctx *c, const double rho12[2], const double mu12[2], double factor1, double factor2,
                         int first, double factor12, double dt_r, const double *stc, double sigma, double rho0,
@@ -854,6 +864,17 @@ extern "C" int fz_rk(fz_ctx *c, fz_rk_state *s, const double rkpar[2], double dt
   if (!c || !s || !rkpar || s->ctx != c) return fz_set_error(FZ_ERR_ARG, "fz_rk: bad argument");
   const double factor1 = rkpar[0] * dt, factor2 = rkpar[1] * dt, factor12 = factor1 + factor2;
   const long bi = sizeof(double) * c->ni;
+  if (!rho12 || !mu12 || !psiflx_x || !psiflx_y || !psiflx_z || !u || !v || !w || !psi || !psio || !bforce || !gacc ||
+      !rho_av || !p || !kappa || !pn || !po)
+    return fz_set_error(FZ_ERR_ARG, "fz_rk: null argument");
+  // (the history is updated in place; du, dv, dw are the kernel's output)
+  const int rc = fz_launch_rk_fused(c, rho12, mu12, factor1, factor2, s->first_mom ? 1 : 0, dt_r, sigma, rho0, bforce,
+                                    gacc, rho_av, psiflx_x, psiflx_y, psiflx_z, psi, psio, p, pn, po, kappa, s->duo,
+                                    s->dvo, s->dwo, s->du, s->dv, s->dw, u, v, w);
+  if (rc != 1) {
+    if (rc == FZ_OK) s->first_mom = false;
+    return rc;
+  }
   FZ_TRY(fz_mom_xyz_ad(c, rho12, mu12, psiflx_x, psiflx_y, psiflx_z, u, v, w, psi, s->du, s->dv, s->dw));
   if (s->first_mom) {
     FZ_HIP(hipMemcpyAsync(s->duo, s->du, bi, hipMemcpyDeviceToDevice, c->st));
@@ -876,6 +897,16 @@ extern "C" int fz_rk_2fl(fz_ctx *c, fz_rk_state *s, const double rkpar[2], doubl
                          double *psiflx_y, double *psiflx_z) {
   if (!c || !s || !rkpar || s->ctx != c) return fz_set_error(FZ_ERR_ARG, "fz_rk_2fl: bad argument");
   const double factor1 = rkpar[0] * dt, factor2 = rkpar[1] * dt;
+  if (!u || !v || !w || !normx || !normy || !normz || !phi || !psi || !psiflx_x || !psiflx_y || !psiflx_z)
+    return fz_set_error(FZ_ERR_ARG, "fz_rk_2fl: null argument");
+  // (the history is updated in place; dpsi is the kernel's output)
+  const int rc = fz_launch_rk_2fl_fused(c, factor1, factor2, s->first_psi ? 1 : 0, gam, seps, beta, vof, u, v, w,
+                                        normx, normy, normz, phi, s->dpsio, s->dpsi, psi, psiflx_x, psiflx_y,
+                                        psiflx_z);
+  if (rc != 1) {
+    if (rc == FZ_OK) s->first_psi = false;
+    return rc;
+  }
   if (!vof) FZ_TRY(fz_acdi_transport_pf(c, gam, seps, u, v, w, normx, normy, normz, phi, psi, s->dpsi, psiflx_x,
                                         psiflx_y, psiflx_z));
   else FZ_TRY(fz_vof_thinc_transport_psi(c, beta, u, v, w, normx, normy, normz, phi, psi, s->dpsi, psiflx_x, psiflx_y,

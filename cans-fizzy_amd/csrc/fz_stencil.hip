@@ -935,7 +935,8 @@ __device__ __forceinline__ void acdi_face(T psa, T psb, T pha, T phb, T nxa, T n
 // right-hand side from its six faces in acdi_cell's order, so the results
 // are those of k_acdi_lds bit for bit. The velocities are read at the cell
 // only (and below the tile's edges), straight from memory.
-template <typename T, bool XPER = false, int MY = ACD_MY>
+// (RK: psi_out is an interior array)
+template <typename T, bool XPER = false, int MY = ACD_MY, bool RK = false>
 __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const double *__restrict__ dzci,
                                                            const double *__restrict__ dzfi, double dxi_d,
                                                            double dyi_d, const double *__restrict__ d_gam,
@@ -1074,7 +1075,7 @@ __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const
       flux_z[q] = fz;
       const T pn = pso + (T)factor1 * R + (T)factor2 * Ro;
       const T ps = fmin(fmax((T)0.0, pn), (T)1.0);
-      psi_out[q] = ps;
+      psi_out[RK ? r : q] = ps;
       if (XPER && xper && (i == 1 || i == d.n1)) {  // the periodic x halo of the row
         const XHalo xh = xhalo_of(d, i);
         xhalo_put(xh, (unsigned)q, buf_out(flux_x, d), fx);
@@ -1227,7 +1228,7 @@ __device__ __forceinline__ T vof_face_flux(const fz_dims &d, int dir, long f, T 
 // history dpsio is read and replaced by R in place (on the first step the
 // history is R itself). Fluxes of the faces at index 0 are left to the
 // boundary update that follows, which sets every halo face.
-template <typename T>
+template <typename T, bool RK = false>  // (RK: psi_out is an interior array)
 __global__ void __launch_bounds__(256) k_vof_step(fz_dims d, const double *__restrict__ dzfi, double dxi_d,
                                                   double dyi_d, double beta_d, double factor1_v, double factor2_v,
                                                   const double *__restrict__ stc, int first,
@@ -1253,7 +1254,7 @@ __global__ void __launch_bounds__(256) k_vof_step(fz_dims d, const double *__res
   const T Ro = first ? R : dpsio[r];
   dpsio[r] = R;
   const T pn = psio[q] + (T)factor1 * R + (T)factor2 * Ro;
-  psi_out[q] = fmin(fmax((T)0.0, pn), (T)1.0);
+  psi_out[RK ? r : q] = fmin(fmax((T)0.0, pn), (T)1.0);
 }
 
 template <typename T>
@@ -2081,8 +2082,11 @@ struct LdsAt {
 // WPE: waves per SIMD the registers must allow; STEADY: a step after the
 // first (first = 0) with no bulk-density term (rho_av = 0), known at compile time
 // (XPER: the cells 1 and n1 also store their new velocity at the periodic
-// x-halo images n1+1 and 0 of their row)
-template <typename PT, typename HT, int WPE, bool BT = false, bool STEADY = false, bool XPER = false>
+// x-halo images n1+1 and 0 of their row; RK: rk as a routine of its own, with
+// the pressure of the step before the last in pn instead of p, and the new
+// velocity written to interior arrays)
+template <typename PT, typename HT, int WPE, bool BT = false, bool STEADY = false, bool XPER = false,
+          bool RK = false>
 __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_per_eu(WPE))) k_mom_lds(
     fz_dims d, int kz, const double *__restrict__ dzci, const double *__restrict__ dzfi, double dxi, double dyi, double rho,
     double drho, double mu, double dmu, double factor1_v, double factor2_v, int first, double factor12_v,
@@ -2090,9 +2094,9 @@ __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_pe
     double bfz, double gx, double gy, double gz, double rax, double ray, double raz, const PT *__restrict__ psiflx_x,
     const PT *__restrict__ psiflx_y, const PT *__restrict__ psiflx_z, const double *__restrict__ u,
     const double *__restrict__ v, const double *__restrict__ w, const PT *__restrict__ psi,
-    const PT *__restrict__ psio, const double *__restrict__ p, const double *__restrict__ po,
-    const PT *__restrict__ kappa, HT *__restrict__ duo, HT *__restrict__ dvo, HT *__restrict__ dwo,
-    double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn, fz_bref br) {
+    const PT *__restrict__ psio, const double *__restrict__ p, const double *__restrict__ pn,
+    const double *__restrict__ po, const PT *__restrict__ kappa, HT *__restrict__ duo, HT *__restrict__ dvo,
+    HT *__restrict__ dwo, double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn, fz_bref br) {
   constexpr int NT = MOM_MX * MOM_MY, PL = MOM_PL;
   constexpr int NPT = (PL + NT - 1) / NT;  // plane positions per thread
   // u, v, w, psi and the z flux are read at k-1, k, k+1 (three plane slots);
@@ -2213,7 +2217,7 @@ __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_pe
       dvo[r] = rv;
       dwo[r] = rw;
       const BufAt<PT> PSIO = buf_at(psio, d, q), KAP = buf_at(kappa, d, q);
-      const BufAt<double> P = buf_at(p, d, q), PO = buf_at(po, d, q);
+      const BufAt<double> P = buf_at(p, d, q), PN = buf_at(RK ? pn : p, d, q), PO = buf_at(po, d, q);
       const double rhox_n = rho + drho * 0.5 * ((double)PSIO(0, 0, 0) + (double)PSIO(1, 0, 0));
       const double rhoy_n = rho + drho * 0.5 * ((double)PSIO(0, 0, 0) + (double)PSIO(0, 1, 0));
       const double rhoz_n = rho + drho * 0.5 * ((double)PSIO(0, 0, 0) + (double)PSIO(0, 0, 1));
@@ -2224,13 +2228,13 @@ __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_pe
       const double nv1 = V(0, 0, 0) * rhoy_n, nv2 = factor1 * rv + factor2 * rvo;
       const double nw1 = W(0, 0, 0) * rhoz_n, nw2 = factor1 * rw + factor2 * rwo;
       mom_oth_cell(k, dzci, dxi, dyi, dt_r, rho, drho, surf_factor, rho0, bfx, bfy, bfz, gx, gy, gz, rax, ray, raz,
-                   P, PSI, KAP, P, PO, ru, rv, rw);
+                   P, PSI, KAP, PN, PO, ru, rv, rw);
       double uo, vo, wo;
       mom_update(nu1, nu2, factor12 * ru, rhox_p, nv1, nv2, factor12 * rv, rhoy_p, nw1, nw2, factor12 * rw, rhoz_p, uo,
                  vo, wo);
-      un[q] = uo;
-      vn[q] = vo;
-      wn[q] = wo;
+      un[RK ? r : q] = uo;
+      vn[RK ? r : q] = vo;
+      wn[RK ? r : q] = wo;
       if constexpr (XPER) {  // (plain stores: buffer resources for three more fields spill scalar registers)
         if (i == d.n1) {
           un[q - d.n1] = uo;
@@ -2286,7 +2290,7 @@ int fz_launch_mom_fused(fz_ctx *c, const double rho12[2], const double mu12[2], 
               grid, dim3(MOM_MX, MOM_MY), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], rho12[1],
               rho12[0] - rho12[1], mu12[1], mu12[0] - mu12[1], factor1, factor2, first, factor12, dt_r, stc,
               surf_factor, rho0, bforce[0], bforce[1], bforce[2], gacc[0], gacc[1], gacc[2], rho_av[0], rho_av[1],
-              rho_av[2], fx, fy, fz, u, v, w, psi, psio, p, po, kappa, duo, dvo, dwo, un, vn, wn, kNoBRef);
+              rho_av[2], fx, fy, fz, u, v, w, psi, psio, p, p, po, kappa, duo, dvo, dwo, un, vn, wn, kNoBRef);
     FZ_LAUNCHED();
     return FZ_OK;
   }
@@ -2351,6 +2355,31 @@ __global__ void k_rk_mom_oth(fz_dims d, double factor12, double rho, double drho
   u[q] = u[q] + factor12 * dudt[r] / rhox_p;
   v[q] = v[q] + factor12 * dvdt[r] / rhoy_p;
   w[q] = w[q] + factor12 * dwdt[r] / rhoz_p;
+}
+
+// the velocity of rk's fused kernel (interior arrays) into the fields
+__global__ void __launch_bounds__(256) k_rk_mom_back(fz_dims d, const double *__restrict__ a,
+                                                     const double *__restrict__ b, const double *__restrict__ c,
+                                                     double *__restrict__ u, double *__restrict__ v,
+                                                     double *__restrict__ w) {
+  CELL_IJK(d);
+  u[q] = a[r];
+  v[q] = b[r];
+  w[q] = c[r];
+}
+// the psi of rk_2fl's fused kernels into the field, whose halo cells are
+// clipped as clip_field does (the interior ones are); the cells 1 and n1 of a
+// row take its halo cells along, so that the rows stay aligned with the blocks
+__global__ void __launch_bounds__(256) k_rk_psi_back(fz_dims d, const double *__restrict__ a,
+                                                     double *__restrict__ psi) {
+  FZ_BLOCK_XYZ(d, bx, by, k);
+  const int i = (int)(bx * blockDim.x + threadIdx.x) + 1, j = (int)(by * blockDim.y + threadIdx.y);
+  if (i > d.n1 || j > d.n2 + 1) return;
+  const long q = i + d.sy * j + d.sz * (long)k;
+  const bool in = j >= 1 && j <= d.n2 && k >= 1 && (int)k <= d.n3;
+  psi[q] = in ? a[(i - 1) + (long)d.n1 * ((j - 1) + (long)d.n2 * ((int)k - 1))] : fmin(fmax(0.0, psi[q]), 1.0);
+  if (i == 1) psi[q - 1] = fmin(fmax(0.0, psi[q - 1]), 1.0);
+  if (i == d.n1) psi[q + 1] = fmin(fmax(0.0, psi[q + 1]), 1.0);
 }
 
 // src/rk.f90:240-247
@@ -2510,6 +2539,7 @@ extern "C" int fz_updatep(fz_ctx *c, const double *pp, double *p) {
 extern "C" int fz_updt_rhs_b(fz_ctx *c, double *p) {
   if (!c || !p) return fz_set_error(FZ_ERR_ARG, "fz_updt_rhs_b: null argument");
   if (!c->pois) return fz_set_error(FZ_ERR_STATE, "fz_updt_rhs_b: fz_initsolver has not been called");
+  if (c->pois->rhsb_zero) return FZ_OK;  // every boundary term is zero
   const fz_dims &d = c->d;
   // x is a boundary direction of the x-pencil; y and z when not periodic
   const double *rb[3] = {c->pois->rhsbx, c->pois->rhsby, c->pois->rhsbz};
@@ -2695,6 +2725,59 @@ extern "C" int fz_lscale_forcing(fz_ctx *c, int ftype, double alpha, double dt, 
 }
 
 // rk_2fl / rk AB2 kernels for the case driver and fz_rk / fz_rk_2fl
+// rk (src/rk.f90:72-130) in one pass of the momentum kernel into the interior
+// arrays un, vn, wn, then into u, v, w: 160 + 48 bytes a cell where mom_ad,
+// the AB2 update, mom_oth and its update move 336 (128x128x256: 378 -> 194
+// + 37 us). The same values: k_mom_lds has these kernels' expressions. Fields
+// past the kernel's 32-bit offsets keep the four kernels (returns 1).
+int fz_launch_rk_fused(fz_ctx *c, const double rho12[2], const double mu12[2], double factor1, double factor2,
+                       int first, double dt_r, double sigma, double rho0, const double bforce[3],
+                       const double gacc[3], const double rho_av[3], const double *fx, const double *fy,
+                       const double *fz, const double *psi, const double *psio, const double *p, const double *pn,
+                       const double *po, const double *kappa, double *duo, double *dvo, double *dwo, double *un,
+                       double *vn, double *wn, double *u, double *v, double *w) {
+  if (fits_buffers(c, "rk") != FZ_OK) return 1;
+  dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY);
+  const int kz = march_planes<true>(c, grid, c->d.n3, 1, 2);
+  FZ_LAUNCH(c, "rk_mom", (k_mom_lds<double, double, 1, false, false, false, true>), grid, dim3(MOM_MX, MOM_MY), 0,
+            c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], rho12[1], rho12[0] - rho12[1], mu12[1],
+            mu12[0] - mu12[1], factor1, factor2, first, factor1 + factor2, dt_r, (const double *)nullptr,
+            sigma * 2.0 / (rho12[0] + rho12[1]), rho0, bforce[0], bforce[1], bforce[2], gacc[0], gacc[1], gacc[2],
+            rho_av[0], rho_av[1], rho_av[2], fx, fy, fz, u, v, w, psi, psio, p, pn, po, kappa, duo, dvo, dwo, un, vn,
+            wn, kNoBRef);
+  FZ_LAUNCHED();
+  FZ_LAUNCH(c, "rk_mom_back", k_rk_mom_back, fz_grid_interior(c->d), fz_block3(), 0, c->d, un, vn, wn, u, v, w);
+  FZ_LAUNCHED();
+  return FZ_OK;
+}
+// rk_2fl (src/rk.f90:216-252) in one pass of the step's transport kernel into
+// the interior array ps, then into psi: 112 + 16 bytes a cell where transport,
+// AB2 update and clip move 144, and each ACDI face evaluated once
+// (128x128x256: 188 -> 133 + 26 us). The same values; returns 1 as above.
+int fz_launch_rk_2fl_fused(fz_ctx *c, double factor1, double factor2, int first, double gam, double seps,
+                           double beta, int vof, const double *u, const double *v, const double *w, const double *nx,
+                           const double *ny, const double *nz, const double *phi, double *dpsio, double *ps,
+                           double *psi, double *fx, double *fy, double *fz) {
+  if (fits_buffers(c, "rk_2fl") != FZ_OK) return 1;
+  const double *stc = nullptr, *d_gam = nullptr;
+  if (vof) {
+    FZ_LAUNCH(c, "rk_vof", (k_vof_step<double, true>), fz_grid_interior(c->d), fz_block3(), 0, c->d, c->dzfi,
+              c->dli[0], c->dli[1], beta, factor1, factor2, stc, first, u, v, w, nx, ny, nz, phi, psi, dpsio, ps, fx,
+              fy, fz);
+  } else {
+    dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY);
+    const int kz = march_planes(c, grid, c->d.n3, 1, 3);
+    FZ_LAUNCH(c, "rk_acdi", (k_acdi_sf<double, false, ACD_MY, true>), grid, dim3(ACD_MX, ACD_MY), 0, c->d, kz,
+              c->dzci, c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc, first, u, v, w, nx, ny,
+              nz, phi, psi, dpsio, ps, fx, fy, fz, 0);
+  }
+  FZ_LAUNCHED();
+  const dim3 rows((c->d.n1 + 63) / 64, (c->d.n2 + 2 + 3) / 4, c->d.n3 + 2);
+  FZ_LAUNCH(c, "rk_psi_back", k_rk_psi_back, rows, fz_block3(), 0, c->d, ps, psi);
+  FZ_LAUNCHED();
+  return FZ_OK;
+}
+
 int fz_launch_rk_psi(fz_ctx *c, double f1, double f2, const double *dpsidt, const double *dpsidto, double *psi) {
   FZ_LAUNCH(c, "rk_psi_ab2", k_rk_psi_ab2, fz_grid_interior(c->d), fz_block3(), 0, c->d, f1, f2, dpsidt, dpsidto, psi);
   FZ_LAUNCHED();
@@ -2874,11 +2957,12 @@ int fz_batch_mom(fz_ctx *c, fz_bref br, int ncase) {
   int variant = c->mom_variant;
   if (variant == 0) variant = 8;
   const char *name = sizeof(PT) == 4 ? "mom_fused_f32" : "mom_fused";
-#define FZ_MOM_NULLS                                                                                              \
+#define FZ_COMMA ,
+#define FZ_MOM_NULLS(PN)                                                                                           \
   0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0, 0.0, 0.0, (const double *)nullptr, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, \
       0.0, 0.0, (const PT *)nullptr, (const PT *)nullptr, (const PT *)nullptr, (const double *)nullptr,            \
       (const double *)nullptr, (const double *)nullptr, (const PT *)nullptr, (const PT *)nullptr,                  \
-      (const double *)nullptr, (const double *)nullptr, (const PT *)nullptr, (HT *)nullptr, (HT *)nullptr,         \
+      (const double *)nullptr, PN (const double *)nullptr, (const PT *)nullptr, (HT *)nullptr, (HT *)nullptr,      \
       (HT *)nullptr, (double *)nullptr, (double *)nullptr, (double *)nullptr, br
   if (variant == 8) {
     dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY);
@@ -2886,7 +2970,8 @@ int fz_batch_mom(fz_ctx *c, fz_bref br, int ncase) {
     br.gz = grid.z;
     grid.z *= (unsigned)ncase;
     FZ_LAUNCH(c, name, (k_mom_lds<PT, HT, sizeof(PT) == 4 ? 3 : 1, true, sizeof(PT) == 4>), grid,
-              dim3(MOM_MX, MOM_MY), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], FZ_MOM_NULLS);
+              dim3(MOM_MX, MOM_MY), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+              FZ_MOM_NULLS((const double *)nullptr FZ_COMMA));
   } else {
     auto kern = variant == 4   ? k_mom_fused_w4<PT, HT, true>
                 : variant == 5 ? k_mom_fused_w5<PT, HT, true>
@@ -2895,9 +2980,10 @@ int fz_batch_mom(fz_ctx *c, fz_bref br, int ncase) {
     dim3 grid = fz_grid_interior(c->d);
     br.gz = grid.z;
     grid.z *= (unsigned)ncase;
-    FZ_LAUNCH(c, name, kern, grid, fz_block3(), 0, c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1], FZ_MOM_NULLS);
+    FZ_LAUNCH(c, name, kern, grid, fz_block3(), 0, c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1], FZ_MOM_NULLS());
   }
 #undef FZ_MOM_NULLS
+#undef FZ_COMMA
   FZ_LAUNCHED();
   return FZ_OK;
 }

@@ -132,3 +132,72 @@ def test_columns_in_registers_match_the_chunked_kernels(n3, cbc, rng, monkeypatc
             got = solve(n, cbc, f, mixed, count)
             monkeypatch.setenv("FZ_THOMAS_ROWS64", "16")
             assert np.array_equal(got, solve(n, cbc, f, mixed, count), equal_nan=True), (n, mixed, count)
+
+
+@pytest.mark.parametrize("n", [[5, 3, 2], [33, 7, 9], [64, 8, 17], [70, 13, 40]], ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("vof", [0, 1], ids=["acdi", "thinc"])
+def test_integrators_match_their_parts(n, vof, rng):
+    """rk and rk_2fl (one pass each and a copy back) against transport,
+    momentum terms and clip called by themselves with the AB2 updates of
+    src/rk.f90:86-130 and :232-252 between them, over three calls."""
+    ctx = F.Context(n, [1.0, 0.9, 1.7], "PPPPNN", gr=0.5)
+    try:
+        rand = lambda lo=-1.0, hi=1.0: np.asfortranarray(rng.uniform(lo, hi, [x + 2 for x in n]))  # noqa: E731
+        h = {q: ctx.halo(rand()) for q in ("u", "v", "w", "nx", "ny", "nz", "phi", "p", "pn", "po", "kappa")}
+        h.update(psi=ctx.halo(rand(-0.2, 1.2)), fx=ctx.halo(rand()), fy=ctx.halo(rand()), fz=ctx.halo(rand()))
+        h["psio"] = ctx.halo(rand(0.0, 1.0))
+        part = {q: ctx.interior() for q in ("r", "du", "dv", "dw", "au", "av", "aw")}
+        st = C.c_void_p()
+        F.call("fz_rk_state_create", ctx.h, C.byref(st))
+        rho12, mu12 = (C.c_double * 2)(50.0, 1.0), (C.c_double * 2)(0.3, 0.02)
+        three = [(C.c_double * 3)(*v) for v in ([0.1, 0.0, -0.2], [0.0, 0.3, -0.98], [0.0, 0.5, 3.0])]
+        gam, seps, beta, dt, dt_r = 0.7, 0.02, 40.0, 1e-3, 1.2
+        tm = (C.c_double * 2)(1.0 + 0.5 * dt_r, -0.5 * dt_r)
+        f1, f2 = tm[0] * dt, tm[1] * dt
+        inner = (slice(1, -1),) * 3
+        hist, vel_hist = None, None
+        P = {q: a.ptr for q, a in h.items()}
+        for _ in range(3):
+            psi = h["psi"].download()
+            args = [P[q] for q in ("u", "v", "w", "nx", "ny", "nz", "phi", "psi")]
+            name, par = ("fz_vof_thinc_transport_psi", [beta]) if vof else ("fz_acdi_transport_pf", [gam, seps])
+            F.call(name, ctx.h, *par, *args, part["r"].ptr, P["fx"], P["fy"], P["fz"])
+            flux = [h[q].download() for q in ("fx", "fy", "fz")]
+            r = part["r"].download()
+            hist = r if hist is None else hist
+            ref = psi.copy(order="F")
+            ref[inner] = psi[inner] + f1 * r + f2 * hist
+            ref = np.minimum(np.maximum(0.0, ref), 1.0)
+            hist = r
+            F.call("fz_rk_2fl", ctx.h, st, tm, dt, gam, seps, beta, vof, *args, P["fx"], P["fy"], P["fz"])
+            assert np.array_equal(h["psi"].download(), ref)
+            for q, f in zip(("fx", "fy", "fz"), flux):
+                assert np.array_equal(h[q].download()[inner], f[inner]), q
+            # momentum
+            F.call("fz_mom_xyz_ad", ctx.h, rho12, mu12, P["fx"], P["fy"], P["fz"], P["u"], P["v"], P["w"], P["psi"],
+                   part["du"].ptr, part["dv"].ptr, part["dw"].ptr)
+            F.call("fz_mom_xyz_oth", ctx.h, dt_r, rho12, rho12, three[0], three[1], 24.5, 1.0, three[2], P["p"],
+                   P["psi"], P["kappa"], P["pn"], P["po"], part["au"].ptr, part["av"].ptr, part["aw"].ptr)
+            now = [part[q].download() for q in ("du", "dv", "dw")]
+            vel_hist = now if vel_hist is None else vel_hist
+            pn_, po_ = h["psi"].download(), h["psio"].download()
+            refs = []
+            for d, q in enumerate("uvw"):
+                up = [slice(1, -1)] * 3
+                up[d] = slice(2, None)
+                up = tuple(up)
+                rn = 1.0 + 49.0 * 0.5 * (po_[inner] + po_[up])
+                rp = 1.0 + 49.0 * 0.5 * (pn_[inner] + pn_[up])
+                a = h[q].download()
+                b = a[inner] * rn / rp + (f1 * now[d] + f2 * vel_hist[d]) / rp
+                a[inner] = b + (f1 + f2) * part["a" + q].download() / rp
+                refs.append(a)
+            vel_hist = now
+            F.call("fz_rk", ctx.h, st, tm, dt, dt_r, three[0], three[1], 24.5, three[2], rho12, mu12, rho12, 1.0,
+                   P["psi"], P["kappa"], P["p"], P["pn"], P["po"], P["psio"], P["fx"], P["fy"], P["fz"], P["u"],
+                   P["v"], P["w"])
+            for q, a in zip("uvw", refs):
+                assert np.array_equal(h[q].download(), a), q
+        F.lib().fz_rk_state_destroy(st)
+    finally:
+        ctx.close()
