@@ -486,10 +486,9 @@ struct P2Shape {
   static constexpr int N = QUARTER ? M / 2 : M;  // real line length
   static constexpr int G0 = QUARTER ? (2048 / M < 64 ? 2048 / M : 64) : (4096 / M < 64 ? (4096 / M > 2 ? 4096 / M : 2) : 64);
   // strided lines (GDIV 1, the y lines) whose row segments of G0 values would
-  // span less than 128 bytes take twice the lines (up to 1024 threads): 512
-  // FP64 y lines 702 and 688 -> 675 and 656 us, FP32 ones 608 and 620 -> 530
-  // and 529 us, FP32 256 lines 115 -> 102 us backward; 256 FP64 lines, whose
-  // 16-line segments are 128 bytes already, measured slower doubled
+  // span less than 128 bytes take twice the lines (up to 1024 threads; the
+  // long ones run k_r2r_p16 instead); 256 FP64 lines, whose 16-line segments
+  // are 128 bytes already, measured slower doubled
   static constexpr int G64 =
       GDIV == 1 && !QUARTER && G0 * (int)sizeof(R) < 128 && G0 * M / 4 <= 1024 ? 2 * G0 : G0;
   // lines whose elements are contiguous in the source and the destination
@@ -625,6 +624,27 @@ __global__ void __launch_bounds__((P2Shape<M, QUARTER, R, GDIV>::NT)) __attribut
                            t2);
   }
   if (out.se == 1) {
+    // (an FP32 correction added to an FP64 solution reads the solution first:
+    // its loads go together instead of each waiting for the store before it)
+    if constexpr (sizeof(TO) > sizeof(R)) {
+      if (accum) {
+        TO held[PER];
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+          const int idx = tid + r * NT;
+          const int g = idx / N, e = idx - g * N;
+          held[r] = g < gcount ? dst[out.base + (long)(l1_0 + g) * out.s1 + l2 * out.s2 + e] : (TO)0;
+        }
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+          const int idx = tid + r * NT;
+          const int g = idx / N, e = idx - g * N;
+          const double sv = (double)val[r] * scale;
+          if (g < gcount) dst[out.base + (long)(l1_0 + g) * out.s1 + l2 * out.s2 + e] = (TO)((double)held[r] + sv);
+        }
+        return;
+      }
+    }
 #pragma unroll
     for (int r = 0; r < PER; r++) {
       const int idx = tid + r * NT;
@@ -648,6 +668,289 @@ __global__ void __launch_bounds__((P2Shape<M, QUARTER, R, GDIV>::NT)) __attribut
     if (g < gcount)
       store_out(dst, out.base + (long)(l1_0 + g) * out.s1 + l2 * out.s2 + (long)e * out.se, Rw[g * RS + e], scale,
                 accum);
+  }
+}
+
+// Long lines strided in memory (complex length M = 2^p, 256 <= M <= 2048, not
+// the quarter-wave kinds): the transform of k_r2r_p2 with sixteen points a
+// thread, which runs two passes on them before it exchanges through LDS. With
+// stride Ns the points b + j M/16 (j < 16) are the inputs of the four
+// butterflies b + u M/16 of one radix-4 pass, and their outputs are those of
+// four butterflies of the next; what is left after two such pairs (a radix 2,
+// a radix 4 or both) works in place on the same points. The arithmetic is
+// k_r2r_p2's, so the results are its bit for bit. Adjacent lanes take adjacent
+// lines, and the points a thread transforms first and last are elements
+// b + j M/16 of its two lines, so the packing of the forward kinds and the
+// unpacking of the backward ones, which are permutations, happen in the loads
+// and stores themselves; the other side goes through LDS. A quarter of the LDS
+// round trips and barriers, for a quarter of the waves: it pays where a block
+// of k_r2r_p2 needs 1024 threads for row segments of 128 bytes (512^3 FP64 y
+// lines 663 and 632 -> 578 and 539 us forward and backward; 256^3 FP32 ones 53
+// and 50 -> 37 and 38 us), not below (FP64 lines of 256 backward 132 against
+// 141 us) nor for contiguous lines (512^3 backward 505 against 551 us).
+template <int M, typename R>
+struct P16Shape {
+  static constexpr int LG = __builtin_ctz(M);
+  // threads of a block: its lines' row segments span 128 bytes (to 256 threads, 512 in FP32)
+  static constexpr int NT = M / 2 * 8 / (int)sizeof(R) < (sizeof(R) == 8 ? 256 : 512) ? M / 2 * 8 / (int)sizeof(R)
+                                                                                   : (sizeof(R) == 8 ? 256 : 512);
+  static constexpr int NFFT = NT * 16 / M;       // complex lines
+  static constexpr int G = 2 * NFFT;             // real lines
+  // LDS rows: one complex of padding per 16 keeps the first exchange's writes
+  // (16 points a lane) off each other's banks, odd strides the lanes of
+  // different rows
+  static constexpr int MP = (M + M / 16) | 1;  // complex row stride
+  static constexpr int RS = M | 1;             // staged real row stride
+  static constexpr size_t LDSC = (size_t)NFFT * MP * sizeof(typename CT<R>::C);
+  static constexpr size_t LDSR = (size_t)G * RS * sizeof(R);
+  static constexpr size_t LDS = LDSC > LDSR ? LDSC : LDSR;
+};
+template <typename C, typename R>
+__device__ __forceinline__ C tw_at(const C *__restrict__ tw, int j, R sign) {
+  C w = tw[j];
+  if (sign > 0) w.y = -w.y;
+  return w;
+}
+
+// two radix-4 passes, strides NS and 4 NS, on the points v[j] = x[b + j M/16];
+// afterwards v[j] belongs at position (b - k) 16 + k + j NS (k = b mod NS)
+template <int M, int NS, typename R, typename C>
+__device__ __forceinline__ void pass44(C (&v)[16], int b, R sign, const C *__restrict__ tw) {
+  const int k = b & (NS - 1);
+  if (NS > 1 && k > 0) {
+#pragma unroll
+    for (int t = 1; t < 4; t++) {
+      const C w = tw_at<C>(tw, t * k * (M / (4 * NS)), sign);
+#pragma unroll
+      for (int u = 0; u < 4; u++) v[u + 4 * t] = cmul(v[u + 4 * t], w);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    C x[4] = {v[u], v[u + 4], v[u + 8], v[u + 12]};
+    bfly4(x, sign);
+#pragma unroll
+    for (int t = 0; t < 4; t++) v[u + 4 * t] = x[t];
+  }
+#pragma unroll
+  for (int t = 0; t < 4; t++) {  // the butterfly of the outputs t
+    C x[4] = {v[4 * t], v[4 * t + 1], v[4 * t + 2], v[4 * t + 3]};
+    const int kk = t * NS + k;
+    if (t > 0 || (NS > 1 && k > 0)) {
+#pragma unroll
+      for (int u = 1; u < 4; u++) x[u] = cmul(x[u], tw_at<C>(tw, u * kk * (M / (16 * NS)), sign));
+    }
+    bfly4(x, sign);
+#pragma unroll
+    for (int u = 0; u < 4; u++) v[4 * t + u] = x[u];
+  }
+  C o[16];  // output u of butterfly t is point t + 4 u
+#pragma unroll
+  for (int t = 0; t < 4; t++)
+#pragma unroll
+    for (int u = 0; u < 4; u++) o[t + 4 * u] = v[4 * t + u];
+#pragma unroll
+  for (int j = 0; j < 16; j++) v[j] = o[j];
+}
+
+// the closing passes on the points v[j] = x[b + j M/16], in place: REM 1
+// radix 2, 2 radix 4, 3 radix 4 then radix 2
+template <int M, int REM, typename R, typename C>
+__device__ __forceinline__ void pass_rem(C (&v)[16], int b, R sign, const C *__restrict__ tw) {
+  if constexpr (REM >= 2) {
+    constexpr int NS = REM == 2 ? M / 4 : M / 8;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int k = (b + j * (M / 16)) & (NS - 1);
+      C x[4] = {v[j], v[j + 4], v[j + 8], v[j + 12]};
+      if (k > 0) {
+#pragma unroll
+        for (int t = 1; t < 4; t++) x[t] = cmul(x[t], tw_at<C>(tw, t * k * (M / (4 * NS)), sign));
+      }
+      bfly4(x, sign);
+#pragma unroll
+      for (int t = 0; t < 4; t++) v[j + 4 * t] = x[t];
+    }
+    if constexpr (REM == 3) {
+      // butterfly j = 2 g + h left output t at position g M/2 + b + h M/16 + t M/8
+      C o[16];
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int t = 0; t < 4; t++) o[8 * (j >> 1) + (j & 1) + 2 * t] = v[j + 4 * t];
+#pragma unroll
+      for (int j = 0; j < 16; j++) v[j] = o[j];
+    }
+  }
+  if constexpr (REM == 1 || REM == 3) {
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+      const int k = b + j * (M / 16);
+      C x1 = v[j + 8];
+      if (k > 0) x1 = cmul(x1, tw_at<C>(tw, k, sign));
+      const C x0 = v[j];
+      v[j] = cadd(x0, x1);
+      v[j + 8] = csub(x0, x1);
+    }
+  }
+}
+
+template <int M, typename R, typename TI, typename TO, int KIND = -1>
+__global__ void __launch_bounds__((P16Shape<M, R>::NT))
+    k_r2r_p16(const TI *__restrict__ src, LineMap in, TO *__restrict__ dst, LineMap out, int L1, int kind_a,
+              double scale, int accum, const typename CT<R>::C *__restrict__ tw,
+              const typename CT<R>::C *__restrict__ q, const typename CT<R>::C *__restrict__ t2, Batch bt) {
+  using S = P16Shape<M, R>;
+  using C = typename CT<R>::C;
+  constexpr int G = S::G, NT = S::NT, NFFT = S::NFFT, MP = S::MP, RS = S::RS, TPL = M / 16;
+  const int kind = KIND >= 0 ? KIND : kind_a;
+  if (bt.src) {  // case blockIdx.z of a batch of same-shaped solves
+    src = (const TI *)bt.src[blockIdx.z];
+    dst = (TO *)bt.dst[blockIdx.z];
+  }
+  extern __shared__ double2 smem_raw[];
+  C *smem = (C *)smem_raw;
+  R *Rw = (R *)smem;  // staged real lines (RS apart), overlaid by the complex lines (MP apart)
+  const int tid = threadIdx.x;
+  const int l1_0 = blockIdx.x * G;
+  const long l2 = blockIdx.y;
+  const int gcount = min(G, L1 - l1_0);
+  const bool fwd = (kind == K_R2HC || kind == K_REDFT10 || kind == K_RODFT10);
+  const bool bwd = (kind == K_HC2R || kind == K_REDFT01 || kind == K_RODFT01);
+  const int f = tid % NFFT, b = tid / NFFT;
+  C *Z = smem + (long)f * MP;
+  auto pad = [](int c) { return c + (c >> 4); };
+  // element of a line that packs into complex k (REDFT10, RODFT10), or that complex k unpacks into (REDFT01, RODFT01)
+  auto elem = [](int k) { return k <= (M - 1) / 2 ? 2 * k : 2 * (M - 1 - k) + 1; };
+  C v[16];
+  if (fwd) {  // 1. the thread's points straight from the lines 2f and 2f + 1
+    const long a0 = in.base + (long)(l1_0 + 2 * f) * in.s1 + l2 * in.s2;
+    const bool on0 = 2 * f < gcount, on1 = 2 * f + 1 < gcount;
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+      const int k = b + j * TPL, e = kind == K_R2HC ? k : elem(k);
+      v[j].x = on0 ? (R)src[a0 + (long)e * in.se] : (R)0.0;
+      v[j].y = on1 ? (R)src[a0 + in.s1 + (long)e * in.se] : (R)0.0;
+    }
+    if (kind == K_RODFT10) {
+#pragma unroll
+      for (int j = 0; j < 16; j++)
+        if (elem(b + j * TPL) & 1) v[j] = mkc(-v[j].x, -v[j].y);
+    }
+  } else {  // 1. the G real lines staged, then packed
+    constexpr int PER = G * M / NT, CH = 16;  // PER: 32
+#pragma unroll
+    for (int r0 = 0; r0 < PER; r0 += CH) {
+      R val[CH];
+#pragma unroll
+      for (int r = 0; r < CH; r++) {
+        const int idx = tid + (r0 + r) * NT;
+        const int g = idx % G, e = idx / G;
+        val[r] = g < gcount ? (R)src[in.base + (long)(l1_0 + g) * in.s1 + l2 * in.s2 + (long)e * in.se] : (R)0.0;
+      }
+#pragma unroll
+      for (int r = 0; r < CH; r++) {
+        const int idx = tid + (r0 + r) * NT;
+        const int g = idx % G, e = idx / G;
+        Rw[g * RS + e] = val[r];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; j++) v[j] = pre_value<R>(kind, Rw, f, b + j * TPL, M, q, RS);
+    __syncthreads();
+  }
+  // 2. the passes
+  const R sign = kind_is_forward(kind) ? (R)-1.0 : (R)1.0;
+  pass44<M, 1, R>(v, b, sign, tw);
+#pragma unroll
+  for (int j = 0; j < 16; j++) Z[pad(b * 16 + j)] = v[j];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 16; j++) v[j] = Z[pad(b + j * TPL)];
+  pass44<M, 16, R>(v, b, sign, tw);
+  if constexpr (M >= 512) {
+    const int k = b & 15, base = (b - k) * 16 + k;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; j++) Z[pad(base + j * 16)] = v[j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 16; j++) v[j] = Z[pad(b + j * TPL)];
+    pass_rem<M, S::LG - 8, R>(v, b, sign, tw);
+  }
+  // (the outputs are the points b + j M/16: the closing passes work in place,
+  // and two passes of stride M/16 end there too)
+  // 3. unpacking and store (what an accumulating store adds to is read first)
+  auto at = [&](int g, int k) {
+    return out.base + (long)(l1_0 + g) * out.s1 + l2 * out.s2 + (long)k * out.se;
+  };
+  auto put = [&](int g, int k, R val, TO old) {
+    const double s = (double)val * scale;
+    if (g < gcount) dst[at(g, k)] = accum ? (TO)((double)old + s) : (TO)s;
+  };
+  auto held = [&](int g, int k) { return accum && g < gcount ? dst[at(g, k)] : (TO)0; };
+  if (bwd) {
+    auto line_elem = [&](int j) { return kind == K_HC2R ? b + j * TPL : elem(b + j * TPL); };
+#pragma unroll
+    for (int j0 = 0; j0 < 16; j0 += 8) {
+      TO o[16];
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        o[2 * j] = held(2 * f, line_elem(j0 + j));
+        o[2 * j + 1] = held(2 * f + 1, line_elem(j0 + j));
+      }
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int k = line_elem(j0 + j);
+        C z = v[j0 + j];
+        if (kind == K_RODFT01 && (k & 1)) z = mkc(-z.x, -z.y);
+        put(2 * f, k, z.x, o[2 * j]);
+        put(2 * f + 1, k, z.y, o[2 * j + 1]);
+      }
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 16; j++) Z[pad(b + j * TPL)] = v[j];
+  __syncthreads();
+  if constexpr (KIND == K_R2HC) {
+    // complex values h and M - h give elements h and M - h of both lines
+#pragma unroll
+    for (int r = 0; r < 8; r++) {
+      const int idx = tid + r * NT;
+      const int ff = idx % NFFT, h = idx / NFFT;
+      const C *zf = smem + ff * MP;
+      const int hm = h ? M - h : M / 2;  // (h = 0: elements 0 and M/2, each its own mirror)
+      const C zk = zf[pad(h)], zm = zf[pad(hm)], zr = h ? zm : zk;
+      const C re = mkc((R)0.5 * (zk.x + zr.x), (R)0.5 * (zk.y + zr.y));
+      const C im = h ? mkc((R)0.5 * (zk.y - zm.y), (R)0.5 * (zm.x - zk.x))
+                     : mkc((R)0.5 * (zm.x + zm.x), (R)0.5 * (zm.y + zm.y));
+      const TO o0 = held(2 * ff, h), o1 = held(2 * ff + 1, h), o2 = held(2 * ff, hm), o3 = held(2 * ff + 1, hm);
+      put(2 * ff, h, re.x, o0);
+      put(2 * ff + 1, h, re.y, o1);
+      put(2 * ff, hm, im.x, o2);
+      put(2 * ff + 1, hm, im.y, o3);
+    }
+  } else {
+    constexpr int PER = G * M / NT;
+#pragma unroll 1
+    for (int r0 = 0; r0 < PER; r0 += 4) {
+      TO o[4];
+      R val[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int idx = tid + (r0 + r) * NT;
+        const int g = idx % G, k = idx / G;
+        o[r] = held(g, k);
+        val[r] = post_value<R>(kind, [&](int row, int c) { return smem[row * MP + pad(c)]; }, g, k, M, M, q, t2);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int idx = tid + (r0 + r) * NT;
+        put(idx % G, idx / G, val[r], o[r]);
+      }
+    }
   }
 }
 
@@ -689,6 +992,21 @@ template <int M, bool QUARTER, typename R, typename TI, typename TO>
 static void launch_p2(fz_ctx *ctx, const char *name, const fz_fftplan &P, int kind, const TI *src, LineMap in,
                       TO *dst, LineMap out, int L1, int L2, double scale, int accum, const FillSrc &fs,
                       const Batch &bt) {
+  if constexpr (!QUARTER && M * (int)sizeof(R) >= 1024 && (sizeof(R) == 4 || M >= 512) && sizeof(TI) == sizeof(TO)) {
+    if (in.se != 1 && out.se != 1 && !fs.on) {  // long strided lines
+      using S = P16Shape<M, R>;
+      const dim3 grid((L1 + S::G - 1) / S::G, L2, bt.src ? bt.n : 1);
+      const PlanTabs<R> t = tabs_of(P, R());
+#define FZ_P16_LAUNCH(KIND)                                                                                       \
+  FZ_LAUNCH(ctx, name, (k_r2r_p16<M, R, TI, TO, KIND>), grid, dim3(S::NT), S::LDS, src, in, dst, out, L1, kind,    \
+            scale, accum, t.tw, t.q, t.t2, bt)
+      if (kind == K_R2HC) FZ_P16_LAUNCH(K_R2HC);
+      else if (kind == K_HC2R) FZ_P16_LAUNCH(K_HC2R);
+      else FZ_P16_LAUNCH(-1);
+#undef FZ_P16_LAUNCH
+      return;
+    }
+  }
   // x lines (contiguous on both sides): half the lines per block (x and y
   // lines of 256 at 16 lines per block: 242 and 168 us; x lines at 8 per
   // block 223 us, at 4 per block 228 us; y lines at 8 or 32 per block 177

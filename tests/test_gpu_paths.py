@@ -201,3 +201,27 @@ def test_integrators_match_their_parts(n, vof, rng):
         F.lib().fz_rk_state_destroy(st)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("n,cbc", [([6, 256, 3], "PPPPDD"), ([70, 512, 2], "PPPPND"), ([33, 1024, 2], "NNNNDD"),
+                                   ([20, 2048, 2], "PPDDNN"), ([9, 512, 3], "DDNNDD")],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, list) else v)
+def test_long_strided_lines_bitwise(n, cbc, rng):
+    """y lines of the sixteen-point transform kernel, every kind it takes and
+    line counts that are no multiple of a block's, against the oracle; FP32
+    ones against the FP64 solve to the accuracy of their refinement."""
+    ctx = F.Context(n, [1.0, 0.9, 1.7], cbc)
+    try:
+        F.call("fz_initsolver", ctx.h, None, None, None, None, None, None, None, None, None)
+        sol = O.Solver(n, ctx.dli, ctx.dzci, ctx.dzfi, list(cbc))
+        f = np.asfortranarray(rng.uniform(-1.0, 1.0, [x + 2 for x in n]))
+        d, m = ctx.halo(f), ctx.halo(f)
+        F.call("fz_solver", ctx.h, d.ptr)
+        ref = f.copy(order="F")
+        sol.solve(ref)
+        assert np.array_equal(d.download(), ref)
+        rel = C.c_double()
+        F.call("fz_solver_mixed", ctx.h, m.ptr, 1e-12, 10, C.byref(C.c_int()), C.byref(rel))
+        assert rel.value <= 1e-11
+    finally:
+        ctx.close()
