@@ -135,7 +135,8 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
       delete c;
       return fz_set_error(FZ_ERR_HIP, "hipStreamCreate: %s", hipGetErrorString(e));
     }
-    c->own_stream = true;
+    c->home = std::make_shared<fz_stream_own>();
+    c->home->s = c->st;
   }
   double **dev[6] = {&c->dzc, &c->dzf, &c->zc, &c->zf, &c->dzci, &c->dzfi};
   const std::vector<double> *host[6] = {&c->h_dzc, &c->h_dzf, &c->h_zc, &c->h_zf, &c->h_dzci, &c->h_dzfi};
@@ -181,8 +182,17 @@ extern "C" int fz_ctx_destroy(fz_ctx *c) {
   if (c->red) (void)hipFree(c->red);
   if (c->ftab) (void)hipFree(c->ftab);
   if (c->h_small) (void)hipHostFree(c->h_small);
-  if (c->own_stream && c->st) (void)hipStreamDestroy(c->st);
-  delete c;
+  if (c->ev) (void)hipEventDestroy(c->ev);
+  if (c->guest_of) fz_batch_forget(c->guest_of, c);
+  delete c;  // (and with it its stream, unless a batch's cases still use it)
+  return FZ_OK;
+}
+
+int fz_stream_after(hipStream_t later, fz_ctx *c) {
+  if (later == c->st) return FZ_OK;
+  if (!c->ev) FZ_HIP(hipEventCreateWithFlags(&c->ev, hipEventDisableTiming));
+  FZ_HIP(hipEventRecord(c->ev, c->st));
+  FZ_HIP(hipStreamWaitEvent(later, c->ev, 0));
   return FZ_OK;
 }
 

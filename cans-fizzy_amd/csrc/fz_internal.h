@@ -5,6 +5,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -79,6 +80,14 @@ struct fz_prof_rec {
   hipEvent_t a, b;
 };
 
+// a stream the library made, kept until its last context lets go of it
+struct fz_stream_own {
+  hipStream_t s = nullptr;
+  ~fz_stream_own() {
+    if (s) (void)hipStreamDestroy(s);
+  }
+};
+
 struct fz_ctx {
   bool prof_on = false;
   std::vector<fz_prof_rec> prof_recs;
@@ -91,7 +100,10 @@ struct fz_ctx {
   char cbcpre[6];
   int per[3];
   hipStream_t st = nullptr;
-  bool own_stream = false;
+  std::shared_ptr<fz_stream_own> home;   // the context's own stream (null: the caller gave one)
+  std::shared_ptr<fz_stream_own> guest;  // in a batch: the first case's stream, which st is then
+  fz_case_batch *guest_of = nullptr;     // that batch
+  hipEvent_t ev = nullptr;               // orders other streams after this context's (fz_ctx_event)
   fz_poisson *pois = nullptr;
   double *red = nullptr;      // per-block partial results of reductions
   size_t red_cap = 0;
@@ -216,6 +228,8 @@ static inline dim3 fz_grid_halo(const fz_dims &d) {
 }
 
 // internal entry points shared between translation units
+int fz_stream_after(hipStream_t later, fz_ctx *c);  // later work on the stream waits for c's work so far
+void fz_batch_forget(fz_case_batch *b, fz_ctx *c);  // a context on the batch's stream goes
 int fz_reduce_ensure(fz_ctx *ctx, size_t nblocks);
 int fz_scratch_setup(fz_ctx *ctx);
 int fz_batch_solve(fz_ctx *c0, void **dptrs, int n);

@@ -225,3 +225,53 @@ def test_long_strided_lines_bitwise(n, cbc, rng):
         assert rel.value <= 1e-11
     finally:
         ctx.close()
+
+
+def test_cases_move_between_batches(monkeypatch):
+    """A batch takes its cases onto one stream; cases of an older batch join a
+    newer one, the older one goes first or last, a member is destroyed while
+    in a batch, and every case's fields stay those of its own steps."""
+    specs = [cases.rising_bubble_3d(ng=(16, 8, 12), rho12=(r, 1.0)) for r in (10.0, 50.0, 200.0, 900.0)]
+
+    def start():
+        out = []
+        for s in specs:
+            dc = F.DeviceCase(s)
+            dc.init()
+            dc.step(1)
+            out.append(dc)
+        return out
+
+    alone, batched = start(), start()
+    try:
+        a = cases.CaseBatch(batched[:3])
+        a.step(2)
+        mid = batched[1].get("psi")  # on the batch's stream, between its steps
+        b = cases.CaseBatch(batched[1:])  # led by a member of the first batch
+        a.close()
+        b.step(3)
+        c = cases.CaseBatch([batched[3], batched[0]])
+        c.step(2)
+        b.close()
+        batched[0].step(1)
+        c.close()
+        steps = [2 + 2 + 1, 2 + 3, 2 + 3, 3 + 2]
+        alone[1].step(2)
+        assert np.array_equal(mid, alone[1].get("psi"))
+        alone[1].step(3)
+        for q in (0, 2, 3):
+            alone[q].step(steps[q])
+        for x, y in zip(alone, batched):
+            for k in FIELDS:
+                assert np.array_equal(x.get(k), y.get(k)), k
+        d = cases.CaseBatch(batched[:2])
+        d.step(1)
+        d.close()
+        e = cases.CaseBatch(batched[1:3])
+        batched[2].close()  # a member goes before its batch
+        e.close()
+        batched[1].step(1)
+        batched[1].sync()
+    finally:
+        for x in alone + batched:
+            x.close()
