@@ -74,8 +74,8 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
   c->d.tile_y = 8;
   if (const char *e = getenv("FZ_TILE_Y")) c->d.tile_y = atoi(e);  // block-order tuning
   if (const char *e = getenv("FZ_MOM_WPE")) c->mom_variant = atoi(e);
-  if (const char *e = getenv("FZ_CORREC_KZ")) c->correc_kz = atoi(e);
-  if (const char *e = getenv("FZ_CORREC_MY")) c->correc_my = atoi(e);
+  if (const char *e = getenv("FZ_CORREC_KZ")) c->correc_kz = atoi(e), c->correc_pair = 0;
+  if (const char *e = getenv("FZ_CORREC_MY")) c->correc_my = atoi(e), c->correc_pair = 0;
   if (c->correc_my != 8 && c->correc_my != 16) c->correc_my = 4;  // the tile heights the kernel is built for
   if (const char *e = getenv("FZ_P2_XDIV")) c->p2_xdiv = atoi(e);
   if (const char *e = getenv("FZ_MARCH_PLANES")) c->march = atoi(e);

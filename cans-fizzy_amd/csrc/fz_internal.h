@@ -126,6 +126,7 @@ struct fz_ctx {
                          // (k_acdi_lds), 2 one cell per thread
   int correc_kz = 1;    // correction step: 0 one cell per thread, 1 dp, u, v staged in LDS (k_correc_lds),
                         // 8 or 16 cells per thread marching in z (k_correc_step_mz)
+  int correc_pair = 1;  // 0: the LDS correction kernel also for rows of even length
   int correc_my = 4;    // rows of cells per block of the LDS correction kernel: 4, 8 or 16
   int ncu = 256;        // the device's compute units
   int march = 0;        // planes per block of the z-marching kernels; 0: by the grid (march_planes)

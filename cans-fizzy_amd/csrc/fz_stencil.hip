@@ -9,7 +9,9 @@
 // without FMA contraction) so that, transcendental functions aside, results
 // round exactly as the reference's own CPU build does.
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
+#include <initializer_list>
 
 #include "fz_internal.h"
 #include "fz_math.h"
@@ -570,10 +572,191 @@ __global__ void __launch_bounds__(COR_MX *MY) k_correc_lds(fz_dims d, int kz, co
   }
 }
 
+// The correction step with two cells in x to a lane, without LDS and without
+// a march: memory bound (5 fields read, 4 written). An aligned pair (2m, 2m+1)
+// of a halo'd row of even length is one 16-byte load or store and a wave, the
+// rows of the plane flattened over the lanes, is 1 KB of each field, so the
+// address unit (84 % busy in k_correc_lds) sees half the requests. A pair's x
+// neighbours come from the lanes beside it (the wave's ends load theirs), the
+// neighbours in y and z from the caches. 256x256x512 590 -> 524 us (a copy
+// kernel of as many bytes 425), 256^3 287 -> 242, 192x192x256 162 -> 142,
+// 128x128x256 73 -> 68, 96x96x192 43 -> 31, walls 300x180x200 177 -> 161,
+// 64x64x128 15 -> 12. The same kernel marching over 2, 4, 8 and 16 planes (dp,
+// w from the level before): 534, 555, 585, 685 us at 256x256x512. The x halo
+// cells of a periodic row in the row's own pairs: as stores of their own
+// beside their images' they cost 60 (2 planes) to 130 us (16) there. Same
+// expressions and values as k_correc_lds, which rows of odd length take.
+struct d2_t {
+  double x, y;
+};
+struct PairFld {
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ d2_t get(unsigned e, unsigned so) const {  // the pair at element e (even), so bytes on
+    return __builtin_bit_cast(d2_t, __builtin_amdgcn_raw_buffer_load_b128(r, e * 8u, so, 0));
+  }
+  __device__ __forceinline__ double one(unsigned e, unsigned so) const {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, e * 8u, so, 0));
+  }
+  __device__ __forceinline__ void put(unsigned e, unsigned so, d2_t v) const {
+    __builtin_amdgcn_raw_buffer_store_b128(
+        __builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b128(r, 0u, 0u, 0)), v), r, e * 8u, so, 0);
+  }
+};
+__device__ __forceinline__ PairFld pair_fld(const double *p, const fz_dims &d) {
+  return PairFld{buf_fld(p, d).r};
+}
+// the value of the lane below / above (the wave's ends keep own)
+__device__ __forceinline__ double lane_down(double v, double own) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(own), __double2loint(v), 0x138, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(own), __double2hiint(v), 0x138, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane_up(double v, double own) {
+  const int lo = __builtin_amdgcn_update_dpp(__double2loint(own), __double2loint(v), 0x130, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(__double2hiint(own), __double2hiint(v), 0x130, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+template <bool BT = false>
+__global__ void __launch_bounds__(256) k_correc_pair(fz_dims d, const double *__restrict__ dzci,
+                                                     double factori_v, double factorj_v, double dt_v, double dxi,
+                                                     double dyi, const double *__restrict__ stc, double rhop,
+                                                     const double *__restrict__ dp, const double *__restrict__ p,
+                                                     const double *__restrict__ u, const double *__restrict__ v,
+                                                     const double *__restrict__ w, double *__restrict__ un,
+                                                     double *__restrict__ vn, double *__restrict__ wn,
+                                                     double *__restrict__ p_out,
+                                                     unsigned long long *__restrict__ slots, fz_bref br, int xper,
+                                                     unsigned rlo) {
+  // (blocks in x fastest, so that the blocks of an XCD are neighbours in y)
+  const unsigned gx = gridDim.x, gz = BT ? br.gz : gridDim.z;
+  unsigned L = fz_xcd_block(blockIdx.x + gx * blockIdx.z, gx * gridDim.z);
+  const unsigned cs = L / (gx * gz);
+  L -= cs * (gx * gz);
+  const unsigned bz = L / gx, bx = L - bz * gx;
+  if constexpr (BT) {  // this block's case of a batch: the momentum step's velocity in the spare buffers
+    const fz_bcase &B = br.bt[cs];
+    stc = B.stc;
+    rhop = B.rho0;
+    slots = B.gslots;
+    dp = (const double *)fz_brole(br, cs, BR_DP);
+    p = (const double *)fz_brole(br, cs, BR_P);
+    u = (const double *)fz_brole(br, cs, BR_UN);
+    v = (const double *)fz_brole(br, cs, BR_VN);
+    w = (const double *)fz_brole(br, cs, BR_WN);
+    un = (double *)fz_brole(br, cs, BR_U);
+    vn = (double *)fz_brole(br, cs, BR_V);
+    wn = (double *)fz_brole(br, cs, BR_W);
+    p_out = (double *)fz_brole(br, cs, BR_PO);
+  }
+  const double dt = stc ? stc[FZ_STC_DT] : dt_v;
+  const double factori = stc ? dt * dxi : factori_v, factorj = stc ? dt * dyi : factorj_v;
+  // the rows and planes: halo to halo, or in the directions of bits 1 and 2 of
+  // rlo (whose halo cells the boundary conditions that follow overwrite) 1 to n
+  const int ylo = (rlo >> 1) & 1u, zlo = (rlo >> 2) & 1u;
+  const int npx = (d.n1 + 2) / 2, rows = d.n2 + 2 - 2 * ylo;
+  const int t = (int)(bx * 256u + threadIdx.x), lane = threadIdx.x & 63;
+  const bool act = t < npx * rows;
+  const int tc = act ? t : npx * rows - 1;  // (lanes past the last pair read the last)
+  const int row = tc / npx, m = tc - row * npx, j = ylo + row, iA = 2 * m, iB = iA + 1;
+  const int k = zlo + (int)bz;
+  const unsigned sy = (unsigned)d.sy, szb = (unsigned)d.sz * 8u;
+  const unsigned e = (unsigned)iA + sy * (unsigned)j, es = j > 0 ? e - sy : e, en = j <= d.n2 ? e + sy : e;
+  const bool in_j = j >= 1 && j <= d.n2;
+  // the row's first or last pair, with a halo cell, and that cell's image
+  const bool img = xper && in_j && k >= 1 && k <= d.n3 && (iA == 0 || iB > d.n1);
+  const unsigned eimg = iA == 0 ? e + (unsigned)d.n1 : e + 1u - (unsigned)d.n1;
+  const PairFld DP = pair_fld(dp, d), P = pair_fld(p, d), U = pair_fld(u, d), V = pair_fld(v, d), W = pair_fld(w, d);
+  const PairFld UN = pair_fld(un, d), VN = pair_fld(vn, d), WN = pair_fld(wn, d), PO = pair_fld(p_out, d);
+  const unsigned so = szb * (unsigned)k;
+  const d2_t dpc = DP.get(e, so), dpz = DP.get(e, k <= d.n3 ? so + szb : so), dn = DP.get(en, so),
+             ds = DP.get(es, so), uc = U.get(e, so), vc = V.get(e, so), vs = V.get(es, so), wc = W.get(e, so),
+             pc = P.get(e, so);
+  d2_t wl = wc, dpl = dpc;  // the cells below: the gamma speeds' only
+  if (slots && k >= 1) wl = W.get(e, so - szb), dpl = DP.get(e, so - szb);
+  // (xper: in an interior row the halo cells take the values of their
+  // periodic images: dp and the velocity have theirs there already, p may
+  // not and is read at the image, as is dp past the last cell)
+  double dr = 0.0, dl = 0.0, ul = 0.0, di = 0.0, pi = 0.0;
+  if (lane == 63 && iB <= d.n1) dr = DP.one(e + 2u, so);
+  if (lane == 0 && iA >= 1) {
+    dl = DP.one(e - 1u, so);
+    ul = U.one(e - 1u, so);
+  }
+  if (img) {
+    di = DP.one(eimg + 1u, so);
+    pi = P.one(eimg, so);
+  }
+  dr = lane_up(dpc.x, dr);
+  d2_t uq = uc, vq = vc, wq = wc, pq;
+  if (iA <= d.n1) uq.x = uc.x - factori * (dpc.y - dpc.x) / rhop;
+  if (iB <= d.n1) uq.y = uc.y - factori * (dr - dpc.y) / rhop;
+  if (j <= d.n2) {
+    vq.x = vc.x - factorj * (dn.x - dpc.x) / rhop;
+    vq.y = vc.y - factorj * (dn.y - dpc.y) / rhop;
+  }
+  if (k <= d.n3) {
+    wq.x = wc.x - dt * dzci[k] * (dpz.x - dpc.x) / rhop;
+    wq.y = wc.y - dt * dzci[k] * (dpz.y - dpc.y) / rhop;
+  }
+  pq.x = dpc.x + pc.x;
+  pq.y = dpc.y + pc.y;
+  if (img) {
+    if (iA == 0) pq.x = dpc.x + pi;
+    else {
+      uq.y = uc.y - factori * (di - dpc.y) / rhop;
+      pq.y = dpc.y + pi;
+    }
+  }
+  if (act) {
+    UN.put(e, so, uq);
+    VN.put(e, so, vq);
+    WN.put(e, so, wq);
+    PO.put(e, so, pq);
+  }
+  if (!slots) return;  // uniform across the grid
+  // (the new u below cell A is the pair below's; the wave's first lane has none)
+  const double um = lane_down(uq.y, ul - factori * (dpc.x - dl) / rhop);
+  double mx = 0.0;
+  if (act && in_j && k >= 1 && k <= d.n3) {
+    const double vmA = vs.x - factorj * (dpc.x - ds.x) / rhop, vmB = vs.y - factorj * (dpc.y - ds.y) / rhop;
+    const double wmA = wl.x - dt * dzci[k - 1] * (dpc.x - dpl.x) / rhop;
+    const double wmB = wl.y - dt * dzci[k - 1] * (dpc.y - dpl.y) / rhop;
+    const double ua = 0.5 * (uq.x + um), va = 0.5 * (vq.x + vmA), wa = 0.5 * (wq.x + wmA);
+    const double ub = 0.5 * (uq.y + uq.x), vb = 0.5 * (vq.y + vmB), wb = 0.5 * (wq.y + wmB);
+    if (iA >= 1 && iA <= d.n1) mx = fmax(mx, ua * ua + va * va + wa * wa);
+    if (iB <= d.n1) mx = fmax(mx, ub * ub + vb * vb + wb * wb);
+  }
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_down(mx, o, 64));
+  __shared__ double sh[4];
+  if (lane == 0) sh[threadIdx.x >> 6] = mx;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double b = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
+    if (b > 0.0)
+      atomicMax(slots + ((blockIdx.x + gridDim.x * blockIdx.z) & (FZ_GAMMA_SLOTS - 1)),
+                (unsigned long long)__double_as_longlong(b));
+  }
+}
+// (rows of even length, fields at 16 bytes: every pair is aligned; the
+// tiled and marching kernels where a knob names them)
+static bool correc_pairs(const fz_ctx *c, std::initializer_list<const void *> f) {
+  if (c->d.n1 % 2 != 0 || c->correc_kz != 1 || !c->correc_pair) return false;
+  for (const void *q : f)
+    if ((uintptr_t)q % 16 != 0) return false;
+  return true;
+}
+
 int fz_launch_correc_step(fz_ctx *c, double rho0, double dt, const double *stc, const double *dp, const double *p,
                           const double *u, const double *v, const double *w, double *un, double *vn, double *wn,
                           double *p_out, unsigned long long *slots, int xper, unsigned rlo) {
-  if (c->correc_kz == 1) {  // dp, u, v staged in LDS
+  if (correc_pairs(c, {dp, p, u, v, w, un, vn, wn, p_out})) {  // pairs of cells
+    FZ_TRY(fits_buffers(c, "correc_step"));
+    const int rows = c->d.n2 + 2 - 2 * (int)((rlo >> 1) & 1u), nz = c->d.n3 + 2 - 2 * (int)((rlo >> 2) & 1u);
+    dim3 grid((unsigned)(((long)((c->d.n1 + 2) / 2) * rows + 255) / 256), 1u, (unsigned)nz);
+    FZ_LAUNCH(c, "correc_step", k_correc_pair<>, grid, dim3(256), 0, c->d, c->dzci, dt * c->dli[0],
+              dt * c->dli[1], dt, c->dli[0], c->dli[1], stc, rho0, dp, p, u, v, w, un, vn, wn, p_out, slots, kNoBRef,
+              xper, rlo);
+  } else if (c->correc_kz == 1) {  // dp, u, v staged in LDS
     FZ_TRY(fits_buffers(c, "correc_step"));
     const int my = c->correc_my;
     // (rlo: the directions whose range is 1 to n, see k_correc_lds)
@@ -2994,6 +3177,17 @@ template int fz_batch_mom<float, float>(fz_ctx *, fz_bref, int);
 // gamma from its slots
 int fz_batch_correc_gamma(fz_ctx *c, fz_bref br, int ncase, bool gamma) {
   FZ_TRY(fits_buffers(c, "correc_step"));
+  if (correc_pairs(c, {})) {
+    dim3 grid((unsigned)(((long)((c->d.n1 + 2) / 2) * (c->d.n2 + 2) + 255) / 256), 1u, (unsigned)(c->d.n3 + 2));
+    fz_bref b = br;
+    b.gz = grid.z;
+    grid.z *= (unsigned)ncase;
+    FZ_LAUNCH(c, "correc_step", k_correc_pair<true>, grid, dim3(256), 0, c->d, c->dzci, 0.0, 0.0, 0.0, c->dli[0],
+              c->dli[1], (const double *)nullptr, 0.0, (const double *)nullptr, (const double *)nullptr,
+              (const double *)nullptr, (const double *)nullptr, (const double *)nullptr, (double *)nullptr,
+              (double *)nullptr, (double *)nullptr, (double *)nullptr, (unsigned long long *)nullptr, b, 0, 0u);
+    FZ_LAUNCHED();
+  } else {
   const int my = c->correc_my;
   dim3 grid((c->d.n1 + 2 + COR_MX - 1) / COR_MX, (c->d.n2 + 2 + my - 1) / my);
   const int kz = march_planes(c, grid, c->d.n3 + 2, ncase, 24 / my);
@@ -3010,6 +3204,7 @@ int fz_batch_correc_gamma(fz_ctx *c, fz_bref br, int ncase, bool gamma) {
   else FZ_CORREC_LDS_B(4);
 #undef FZ_CORREC_LDS_B
   FZ_LAUNCHED();
+  }
   if (gamma) {
     FZ_LAUNCH(c, "gamma_fin", k_gamma_fin<true>, dim3((unsigned)ncase), dim3(FZ_GAMMA_SLOTS), 0,
               (unsigned long long *)nullptr, 0.0, 0.0, (double *)nullptr, br, (unsigned *)nullptr);

@@ -275,3 +275,52 @@ def test_cases_move_between_batches(monkeypatch):
     finally:
         for x in alone + batched:
             x.close()
+
+
+def cavity(n):
+    return dict(cases.lid_driven_cavity(), ng=n, l=[x / 10.0 for x in n])
+
+
+PAIRS = {
+    # n1 + 2 cells a row in pairs: rows per wave below and above one, ends of rows at the ends of waves
+    "one pair a row": lambda: cases.rising_bubble_3d(ng=(2, 6, 8)),
+    "periodic 60": lambda: cases.rising_bubble_3d(ng=(60, 5, 9)),
+    "periodic 126": lambda: cases.rising_bubble_3d(ng=(126, 9, 8)),
+    "periodic 130": lambda: cases.rising_bubble_3d(ng=(130, 3, 6)),
+    "walls 40": lambda: dict(cases.hysing_2d(ng=(40, 2, 12)), ng=[40, 7, 12], l=[1.0, 7 / 40, 12 / 40]),
+    "cavity 14": lambda: cavity([14, 9, 11]),
+    "droplets 28": lambda: cases.vof_droplets(ng=(28, 24, 18), ndrop=2, r=0.6),
+    "mixed 78": lambda: dict(cases.rising_bubble_3d(ng=(78, 6, 10)), precision="mixed", refine=1),
+}
+
+
+@pytest.mark.parametrize("name", list(PAIRS))
+def test_correction_in_pairs_matches_the_tiled_kernel(name, rng, monkeypatch):
+    """The correction of rows of even length, pairs of cells a lane, against
+    the LDS kernel's on whole fields, halos included, from a pressure whose
+    halo is not its boundary condition's; alone, and for some as a batch."""
+    out = []
+    spec = PAIRS[name]()
+    n = spec["ng"]
+    dp = rng.uniform(-1e-3, 1e-3, [x + 2 for x in n])
+    for tiled in (False, True):
+        monkeypatch.delenv("FZ_CORREC_MY", raising=False)
+        if tiled:
+            monkeypatch.setenv("FZ_CORREC_MY", "4")
+        dcs = [F.DeviceCase(spec) for _ in range(3)]
+        try:
+            for q, dc in enumerate(dcs):
+                dc.init()
+                dc.step(1)
+                dc.set("p", dc.get("p") + (q + 1) * dp)
+            dcs[0].step(3)
+            if name.startswith(("periodic", "walls")):
+                b = cases.CaseBatch(dcs[1:])
+                b.step(3)
+                b.close()
+            out.append([(dc.get(k), k) for dc in dcs for k in ("u", "v", "w", "p", "psi")] + [(dcs[0].scalars(), "s")])
+        finally:
+            for dc in dcs:
+                dc.close()
+    for (a, k), (b, _) in zip(*out):
+        assert np.array_equal(a, b, equal_nan=True), k
