@@ -950,7 +950,7 @@ struct LdsZ {
   }
 };
 
-template <typename T, bool BT = false>  // BT: a batched launch (fz_bref)
+template <typename T>
 __global__ void __launch_bounds__(ACD_MX *ACD_MY) k_acdi_lds(fz_dims d, int kz, const double *__restrict__ dzci,
                                                             const double *__restrict__ dzfi, double dxi, double dyi,
                                                             const double *__restrict__ d_gam, double gam_v,
@@ -962,30 +962,12 @@ __global__ void __launch_bounds__(ACD_MX *ACD_MY) k_acdi_lds(fz_dims d, int kz, 
                                                             const T *__restrict__ phi, const T *__restrict__ psio,
                                                             T *__restrict__ dpsio, T *__restrict__ psi_out,
                                                             T *__restrict__ flux_x, T *__restrict__ flux_y,
-                                                            T *__restrict__ flux_z, fz_bref br) {
+                                                            T *__restrict__ flux_z) {
   constexpr int NT = ACD_MX * ACD_MY, PL = ACD_PL, NPT = (PL + NT - 1) / NT;
   __shared__ double s_u[2 * PL], s_v[2 * PL], s_w[2 * PL];
   __shared__ T s_nx[2 * PL], s_ny[2 * PL], s_nz[2 * PL], s_phi[2 * PL], s_psi[2 * PL];
-  FZ_BLOCK_XYZB(d, br, cs, bx, by, bz);
-  if constexpr (BT) {  // this block's case of a batch
-    d_gam = br.bt[cs].dsc;
-    seps = br.bt[cs].seps;
-    stc = br.bt[cs].stc;
-    first = 0;
-    u = (const double *)fz_brole(br, cs, BR_U);
-    v = (const double *)fz_brole(br, cs, BR_V);
-    w = (const double *)fz_brole(br, cs, BR_W);
-    normx = (const T *)fz_brole(br, cs, BR_NX);
-    normy = (const T *)fz_brole(br, cs, BR_NY);
-    normz = (const T *)fz_brole(br, cs, BR_NZ);
-    phi = (const T *)fz_brole(br, cs, BR_PHI);
-    psio = (const T *)fz_brole(br, cs, BR_PSI_OLD);
-    dpsio = (T *)fz_brole(br, cs, BR_DPSIO);
-    psi_out = (T *)fz_brole(br, cs, BR_PSI_NEW);
-    flux_x = (T *)fz_brole(br, cs, BR_FX);
-    flux_y = (T *)fz_brole(br, cs, BR_FY);
-    flux_z = (T *)fz_brole(br, cs, BR_FZ);
-  }
+  unsigned bx, by, bz;
+  fz_stencil_block(d.tile_y, bx, by, bz);
   const double gam = d_gam ? *d_gam : gam_v;
   const double factor1 = stc ? stc[FZ_STC_F1] : factor1_v, factor2 = stc ? stc[FZ_STC_F2] : factor2_v;
   const int tx = threadIdx.x, ty = threadIdx.y, t = tx + ACD_MX * ty;
@@ -1119,7 +1101,7 @@ __device__ __forceinline__ void acdi_face(T psa, T psb, T pha, T phb, T nxa, T n
 // are those of k_acdi_lds bit for bit. The velocities are read at the cell
 // only (and below the tile's edges), straight from memory.
 // (RK: psi_out is an interior array)
-template <typename T, bool XPER = false, int MY = ACD_MY, bool RK = false>
+template <typename T, bool XPER = false, int MY = ACD_MY, bool RK = false, bool BT = false>
 __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const double *__restrict__ dzci,
                                                            const double *__restrict__ dzfi, double dxi_d,
                                                            double dyi_d, const double *__restrict__ d_gam,
@@ -1131,7 +1113,8 @@ __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const
                                                            const T *__restrict__ normz, const T *__restrict__ phi,
                                                            const T *__restrict__ psio, T *__restrict__ dpsio,
                                                            T *__restrict__ psi_out, T *__restrict__ flux_x,
-                                                           T *__restrict__ flux_y, T *__restrict__ flux_z, int xper) {
+                                                           T *__restrict__ flux_y, T *__restrict__ flux_z, int xper,
+                                                           fz_bref br) {
   constexpr int NT = ACD_MX * MY, PL = ACD_PX * (MY + 2), NPT = (PL + NT - 1) / NT;
   __shared__ T s_nx[2 * PL], s_ny[2 * PL], s_nz[2 * PL], s_phi[2 * PL], s_psi[2 * PL];
   // the faces of a level: x faces of the tile's rows (index 0 the face below
@@ -1140,8 +1123,26 @@ __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const
   // advective and regularisation parts
   __shared__ T f_xu[MY][ACD_MX + 1], f_xr[MY][ACD_MX + 1];
   __shared__ T f_yu[MY + 1][ACD_MX], f_yr[MY + 1][ACD_MX];
-  unsigned cs_, bx, by, bz;
-  fz_stencil_block_b(d.tile_y, gridDim.z, cs_, bx, by, bz);
+  FZ_BLOCK_XYZB(d, br, cs, bx, by, bz);
+  if constexpr (BT) {  // this block's case of a batch
+    d_gam = br.bt[cs].dsc;
+    seps_d = br.bt[cs].seps;
+    stc = br.bt[cs].stc;
+    first = 0;
+    u = (const double *)fz_brole(br, cs, BR_U);
+    v = (const double *)fz_brole(br, cs, BR_V);
+    w = (const double *)fz_brole(br, cs, BR_W);
+    normx = (const T *)fz_brole(br, cs, BR_NX);
+    normy = (const T *)fz_brole(br, cs, BR_NY);
+    normz = (const T *)fz_brole(br, cs, BR_NZ);
+    phi = (const T *)fz_brole(br, cs, BR_PHI);
+    psio = (const T *)fz_brole(br, cs, BR_PSI_OLD);
+    dpsio = (T *)fz_brole(br, cs, BR_DPSIO);
+    psi_out = (T *)fz_brole(br, cs, BR_PSI_NEW);
+    flux_x = (T *)fz_brole(br, cs, BR_FX);
+    flux_y = (T *)fz_brole(br, cs, BR_FY);
+    flux_z = (T *)fz_brole(br, cs, BR_FZ);
+  }
   const double gam_dd = d_gam ? *d_gam : gam_v;
   const double factor1 = stc ? stc[FZ_STC_F1] : factor1_v, factor2 = stc ? stc[FZ_STC_F2] : factor2_v;
   const T dxi = (T)dxi_d, dyi = (T)dyi_d, gam = (T)gam_dd, seps = (T)seps_d;
@@ -1290,19 +1291,25 @@ int fz_launch_acdi_step(fz_ctx *c, const double *d_gam, double gam, double seps,
     // run-time test there too: measured 550 against 565 us in FP32 without
     // it. FP32 tiles of 64 x 8: 550 -> 532 us; FP64 ones, 70 KB of LDS, 925
     // against 923 us, keep 64 x 4)
+    // Two-dimensional boxes (n2 <= 2) take tiles of 2 rows, whose waves all
+    // have cells: 8 cases of 128x2x128 26 -> 21 us, with the six-face kernel
+    // that batches ran before.
     constexpr int MY = sizeof(T) == 4 ? 8 : ACD_MY;
-    dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + MY - 1) / MY);
-    const int kz = march_planes(c, grid, c->d.n3, 1, 3);
-    auto kern = xper ? k_acdi_sf<T, true, MY> : k_acdi_sf<T, false, MY>;
-    FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", kern, grid, dim3(ACD_MX, MY), 0, c->d, kz, c->dzci,
+    const bool thin = c->d.n2 <= 2;
+    const int my = thin ? 2 : MY;
+    dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + my - 1) / my);
+    const int kz = march_planes(c, grid, c->d.n3, 1, thin ? 6 : 3);
+    auto kern = thin ? (xper ? k_acdi_sf<T, true, 2> : k_acdi_sf<T, false, 2>)
+                     : (xper ? k_acdi_sf<T, true, MY> : k_acdi_sf<T, false, MY>);
+    FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", kern, grid, dim3(ACD_MX, my), 0, c->d, kz, c->dzci,
               c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc, first, u, v, w, normx, normy,
-              normz, phi, psio, dpsio, psi_out, flux_x, flux_y, flux_z, xper);
+              normz, phi, psio, dpsio, psi_out, flux_x, flux_y, flux_z, xper, kNoBRef);
   } else if (variant == 1) {  // fields staged in LDS
     dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY);
     const int kz = march_planes(c, grid, c->d.n3, 1, 3);
     FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", (k_acdi_lds<T>), grid, dim3(ACD_MX, ACD_MY), 0,
               c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc, first, u, v, w,
-              normx, normy, normz, phi, psio, dpsio, psi_out, flux_x, flux_y, flux_z, kNoBRef);
+              normx, normy, normz, phi, psio, dpsio, psi_out, flux_x, flux_y, flux_z);
   } else {
     FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", k_acdi_step<T>, fz_grid_interior(c->d),
               fz_block3(), 0, c->d, c->dzci, c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc,
@@ -2247,7 +2254,7 @@ FZ_MOM_FUSED_KERNEL(k_mom_fused_w5, __attribute__((amdgpu_waves_per_eu(5))), fal
 // registers while level k is computed. The cell arithmetic is
 // mom_fused_body's through an LDS accessor (LdsAt), so the results are the
 // same bit for bit.
-constexpr int MOM_MX = 32, MOM_MY = 8, MOM_PX = MOM_MX + 2, MOM_PL = MOM_PX * (MOM_MY + 2);
+constexpr int MOM_MX = 32, MOM_MY = 8, MOM_PX = MOM_MX + 2;
 
 
 // a field's three plane slots in LDS, seen from one cell
@@ -2269,8 +2276,8 @@ struct LdsAt {
 // the pressure of the step before the last in pn instead of p, and the new
 // velocity written to interior arrays)
 template <typename PT, typename HT, int WPE, bool BT = false, bool STEADY = false, bool XPER = false,
-          bool RK = false>
-__global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_per_eu(WPE))) k_mom_lds(
+          bool RK = false, int MY = MOM_MY>
+__global__ void __launch_bounds__(MOM_MX *MY) __attribute__((amdgpu_waves_per_eu(WPE))) k_mom_lds(
     fz_dims d, int kz, const double *__restrict__ dzci, const double *__restrict__ dzfi, double dxi, double dyi, double rho,
     double drho, double mu, double dmu, double factor1_v, double factor2_v, int first, double factor12_v,
     double dt_r_v, const double *__restrict__ stc, double surf_factor, double rho0, double bfx, double bfy,
@@ -2280,7 +2287,7 @@ __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_pe
     const PT *__restrict__ psio, const double *__restrict__ p, const double *__restrict__ pn,
     const double *__restrict__ po, const PT *__restrict__ kappa, HT *__restrict__ duo, HT *__restrict__ dvo,
     HT *__restrict__ dwo, double *__restrict__ un, double *__restrict__ vn, double *__restrict__ wn, fz_bref br) {
-  constexpr int NT = MOM_MX * MOM_MY, PL = MOM_PL;
+  constexpr int NT = MOM_MX * MY, PL = MOM_PX * (MY + 2);
   constexpr int NPT = (PL + NT - 1) / NT;  // plane positions per thread
   // u, v, w, psi and the z flux are read at k-1, k, k+1 (three plane slots);
   // the x and y fluxes at k and k+1 only (two slots)
@@ -2319,7 +2326,7 @@ __global__ void __launch_bounds__(MOM_MX *MOM_MY) __attribute__((amdgpu_waves_pe
   const double factor1 = stc ? stc[FZ_STC_F1] : factor1_v, factor2 = stc ? stc[FZ_STC_F2] : factor2_v;
   const double factor12 = stc ? stc[FZ_STC_F12] : factor12_v, dt_r = stc ? stc[FZ_STC_DTR] : dt_r_v;
   const int tx = threadIdx.x, ty = threadIdx.y, t = tx + MOM_MX * ty;
-  const int i0 = (int)bx * MOM_MX + 1, j0 = (int)by * MOM_MY + 1, k0 = (int)bz * kz + 1;
+  const int i0 = (int)bx * MOM_MX + 1, j0 = (int)by * MY + 1, k0 = (int)bz * kz + 1;
   const int i = i0 + tx, j = j0 + ty;
   const bool act = i <= d.n1 && j <= d.n2;
   const int kend = min(k0 + kz - 1, d.n3);
@@ -2452,8 +2459,12 @@ int fz_launch_mom_fused(fz_ctx *c, const double rho12[2], const double mu12[2], 
   int variant = c->mom_variant;
   if (variant == 0) variant = 8;
   if (variant == 8) {  // stencil fields staged in LDS
-    dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY);
-    const int kz = march_planes<true>(c, grid, c->d.n3, 1, sizeof(PT) == 4 ? 3 : 2);
+    // (two-dimensional boxes, n2 <= 2: tiles of 2 rows, one wave a block,
+    // instead of 8 rows of which 6 idle: 8 cases of 128x2x128 35 -> 22 us)
+    const bool thin = c->d.n2 <= 2;
+    const int my = thin ? 2 : MOM_MY;
+    dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + my - 1) / my);
+    const int kz = march_planes<true>(c, grid, c->d.n3, 1, thin ? 7 : (sizeof(PT) == 4 ? 3 : 2));
     // (3 waves per SIMD fit FP32 phase fields' registers, 169 -> 168 VGPRs;
     // FP64 needs 188, and a 3-wave FP64 build spills 36 and runs 2.2x slower)
     // With FP32 phase fields, a step after the first without a bulk-density
@@ -2469,8 +2480,10 @@ int fz_launch_mom_fused(fz_ctx *c, const double rho12[2], const double mu12[2], 
                                                   : k_mom_lds<PT, HT, 3, false, true, false>)
                                           : (xper ? k_mom_lds<PT, HT, W, false, false, true>
                                                   : k_mom_lds<PT, HT, W, false, false, false>);
+    if (thin) kern = xper ? k_mom_lds<PT, HT, 1, false, false, true, false, 2>
+                          : k_mom_lds<PT, HT, 1, false, false, false, false, 2>;
     FZ_LAUNCH(c, sizeof(PT) == 4 ? "mom_fused_f32" : "mom_fused", kern,
-              grid, dim3(MOM_MX, MOM_MY), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], rho12[1],
+              grid, dim3(MOM_MX, my), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], rho12[1],
               rho12[0] - rho12[1], mu12[1], mu12[0] - mu12[1], factor1, factor2, first, factor12, dt_r, stc,
               surf_factor, rho0, bforce[0], bforce[1], bforce[2], gacc[0], gacc[1], gacc[2], rho_av[0], rho_av[1],
               rho_av[2], fx, fy, fz, u, v, w, psi, psio, p, p, po, kappa, duo, dvo, dwo, un, vn, wn, kNoBRef);
@@ -2952,7 +2965,7 @@ int fz_launch_rk_2fl_fused(fz_ctx *c, double factor1, double factor2, int first,
     const int kz = march_planes(c, grid, c->d.n3, 1, 3);
     FZ_LAUNCH(c, "rk_acdi", (k_acdi_sf<double, false, ACD_MY, true>), grid, dim3(ACD_MX, ACD_MY), 0, c->d, kz,
               c->dzci, c->dzfi, c->dli[0], c->dli[1], d_gam, gam, seps, factor1, factor2, stc, first, u, v, w, nx, ny,
-              nz, phi, psi, dpsio, ps, fx, fy, fz, 0);
+              nz, phi, psi, dpsio, ps, fx, fy, fz, 0, kNoBRef);
   }
   FZ_LAUNCHED();
   const dim3 rows((c->d.n1 + 63) / 64, (c->d.n2 + 2 + 3) / 4, c->d.n3 + 2);
@@ -3104,15 +3117,19 @@ extern "C" int fz_phase_geometry_eval(fz_ctx *c, double seps, const double *psi,
 template <typename T>
 int fz_batch_acdi_step(fz_ctx *c, fz_bref br, int ncase) {
   FZ_TRY(fits_buffers(c, "acdi_step"));
-  dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY);
-  const int kz = march_planes(c, grid, c->d.n3, ncase, 3);
+  constexpr int MY = sizeof(T) == 4 ? 8 : ACD_MY;
+  const bool thin = c->d.n2 <= 2;
+  const int my = thin ? 2 : MY;
+  dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + my - 1) / my);
+  const int kz = march_planes(c, grid, c->d.n3, ncase, thin ? 6 : 3);
   br.gz = grid.z;
   grid.z *= (unsigned)ncase;
-  FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", (k_acdi_lds<T, true>), grid, dim3(ACD_MX, ACD_MY), 0,
-            c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], (const double *)nullptr, 0.0, 0.0, 0.0, 0.0,
-            (const double *)nullptr, 0, (const double *)nullptr, (const double *)nullptr, (const double *)nullptr,
-            (const T *)nullptr, (const T *)nullptr, (const T *)nullptr, (const T *)nullptr, (const T *)nullptr,
-            (T *)nullptr, (T *)nullptr, (T *)nullptr, (T *)nullptr, (T *)nullptr, br);
+  auto kern = thin ? k_acdi_sf<T, false, 2, false, true> : k_acdi_sf<T, false, MY, false, true>;
+  FZ_LAUNCH(c, sizeof(T) == 4 ? "acdi_step_f32" : "acdi_step", kern, grid, dim3(ACD_MX, my), 0, c->d, kz, c->dzci,
+            c->dzfi, c->dli[0], c->dli[1], (const double *)nullptr, 0.0, 0.0, 0.0, 0.0, (const double *)nullptr, 0,
+            (const double *)nullptr, (const double *)nullptr, (const double *)nullptr, (const T *)nullptr,
+            (const T *)nullptr, (const T *)nullptr, (const T *)nullptr, (const T *)nullptr, (T *)nullptr,
+            (T *)nullptr, (T *)nullptr, (T *)nullptr, (T *)nullptr, 0, br);
   FZ_LAUNCHED();
   return FZ_OK;
 }
@@ -3148,12 +3165,15 @@ int fz_batch_mom(fz_ctx *c, fz_bref br, int ncase) {
       (const double *)nullptr, PN (const double *)nullptr, (const PT *)nullptr, (HT *)nullptr, (HT *)nullptr,      \
       (HT *)nullptr, (double *)nullptr, (double *)nullptr, (double *)nullptr, br
   if (variant == 8) {
-    dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY);
-    const int kz = march_planes<true>(c, grid, c->d.n3, ncase, sizeof(PT) == 4 ? 3 : 2);
+    const bool thin = c->d.n2 <= 2;
+    const int my = thin ? 2 : MOM_MY;
+    dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + my - 1) / my);
+    const int kz = march_planes<true>(c, grid, c->d.n3, ncase, thin ? 7 : (sizeof(PT) == 4 ? 3 : 2));
     br.gz = grid.z;
     grid.z *= (unsigned)ncase;
-    FZ_LAUNCH(c, name, (k_mom_lds<PT, HT, sizeof(PT) == 4 ? 3 : 1, true, sizeof(PT) == 4>), grid,
-              dim3(MOM_MX, MOM_MY), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+    auto kern = thin ? k_mom_lds<PT, HT, 1, true, false, false, false, 2>
+                     : k_mom_lds<PT, HT, sizeof(PT) == 4 ? 3 : 1, true, sizeof(PT) == 4>;
+    FZ_LAUNCH(c, name, kern, grid, dim3(MOM_MX, my), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
               FZ_MOM_NULLS((const double *)nullptr FZ_COMMA));
   } else {
     auto kern = variant == 4   ? k_mom_fused_w4<PT, HT, true>

@@ -324,3 +324,38 @@ def test_correction_in_pairs_matches_the_tiled_kernel(name, rng, monkeypatch):
                 dc.close()
     for (a, k), (b, _) in zip(*out):
         assert np.array_equal(a, b, equal_nan=True), k
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [[33, 1, 9], [40, 2, 33], [130, 2, 20], [65, 3, 12]],
+                         ids=lambda n: "x".join(map(str, n)))
+def test_tiles_of_thin_boxes_match_the_plain_kernels(n, precision, monkeypatch):
+    """Boxes of one and two rows take momentum and ACDI tiles of two rows (three
+    rows do not): the plain kernels' fields bit for bit, and a batch's as its
+    cases' alone."""
+    spec = dict(cases.hysing_2d(ng=tuple(n)), precision=precision, refine=-1)
+
+    def start(count):
+        out = [F.DeviceCase(dict(spec, sigma=24.5 * (q + 1))) for q in range(count)]
+        for dc in out:
+            dc.init()
+            dc.step(1)
+        return out
+
+    tiled, batched = start(2), start(2)
+    monkeypatch.setenv("FZ_MOM_WPE", "2")
+    monkeypatch.setenv("FZ_ACDI_VARIANT", "2")
+    plain = start(2)
+    try:
+        b = cases.CaseBatch(batched)
+        b.step(5)
+        b.close()
+        for t, p, q in zip(tiled, plain, batched):
+            t.step(5)
+            p.step(5)
+            for k in FIELDS:
+                assert np.array_equal(t.get(k), p.get(k)), k
+                assert np.array_equal(t.get(k), q.get(k)), k
+    finally:
+        for dc in tiled + batched + plain:
+            dc.close()
