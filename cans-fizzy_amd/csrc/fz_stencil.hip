@@ -1492,6 +1492,8 @@ __device__ inline double quarter_normal(double x) {
 
 // sqrt(s) by the device's correctly rounded FP64 sequence without its range
 // scaling: the same result for s = 0 and s in [2^-767, 2^1023]
+// (ZERO false: s is not 0)
+template <bool ZERO = true>
 __device__ inline double sqrt_inrange(double s) {
   const double y0 = __builtin_amdgcn_rsq(s);
   double g = s * y0, h = y0 * 0.5;
@@ -1502,7 +1504,7 @@ __device__ inline double sqrt_inrange(double s) {
   g = __builtin_fma(e, h, g);
   e = __builtin_fma(-g, g, s);
   g = __builtin_fma(e, h, g);
-  return s == 0.0 ? s : g;
+  return ZERO && s == 0.0 ? s : g;
 }
 
 // (x, y, z) / (sqrt(x*x + y*y + z*z) + eps), src/two_fluid.f90:140-162.
@@ -1526,7 +1528,11 @@ __device__ __forceinline__ void unit3(T &x, T &y, T &z, bool &ok) {
                         __builtin_amdgcn_frexp_exp(z));
       ok = ok && s <= 0x1p600 && e >= -299;
     }
-    const double d = sqrt_inrange(s) + (double)FZ_EPS;
+    // (NOCHECK: s is 0 or far above 2^-767; a zero s taken as 2^-767 gives the
+    // same denominator, eps, with one maximum instead of a compare and two
+    // selects, 18 of the marching cell's 540 instructions, whose issue bounds
+    // it: 627 -> 606 us at 256x256x512)
+    const double d = (NOCHECK ? sqrt_inrange<false>(__builtin_fmax(s, 0x1p-767)) : sqrt_inrange(s)) + (double)FZ_EPS;
     double w = __builtin_amdgcn_rcp(d);
     double t = __builtin_fma(-d, w, 1.0);
     w = __builtin_fma(w, t, w);
@@ -1837,9 +1843,14 @@ static int launch_youngs(fz_ctx *c, const char *name, const T *psi, T *normx, T 
   // FP64 the check-free marching kernel and its checked twin where the range
   // flag applies (the marching FP64 kernel with both forms needs 236 VGPRs,
   // two waves per SIMD, and took 758 against 705-745 us for one cell per
-  // thread; capped, it spills), one cell per thread elsewhere
-  const int yv = c->youngs_variant ? c->youngs_variant : (sizeof(T) == 4 ? 1 : 3);
+  // thread; capped, it spills), one cell per thread elsewhere and on grids
+  // below about 4 million cells, where one launch without a march beats two:
+  // 17 against 24 us at 64x64x128, 51 against 64 at 96x96x192, 85 against
+  // 89 at 128x128x256, but 192 against 181 at 192x192x256 and 692 against
+  // 606 at 256x256x512
   dim3 mgrid = fz_grid_interior(c->d);
+  const bool small = (long)mgrid.x * mgrid.y * mgrid.z < 60l * c->ncu;
+  const int yv = c->youngs_variant ? c->youngs_variant : (sizeof(T) == 4 ? 1 : (small ? 2 : 3));
   const int kz = march_planes(c, mgrid, c->d.n3, 1, 4);
   const uint3 tiles = {mgrid.x, mgrid.y, mgrid.z};
   if (!br.bt && yv == 1) {  // marching in z
