@@ -73,6 +73,9 @@ def test_line_transforms_of_any_length_bitwise(kind, rng):
 RAGGED = {
     # the right-hand side evaluated in the load of a forward x transform whose length is no power of two
     "bubble_30x18x22": lambda: cases.rising_bubble_3d(ng=(30, 18, 22)),
+    # the phase-field step whose waves own 62 cells of the halo'd plane: rows of one wave, rows across waves
+    "droplets_60x6x7": lambda: cases.vof_droplets(ng=(60, 6, 7), ndrop=1, r=1.2),
+    "droplets_26x9x21": lambda: cases.vof_droplets(ng=(26, 9, 21), ndrop=1, r=1.2),
     "walls_45x14x20": lambda: dict(cases.hysing_2d(ng=(45, 2, 20)), ng=[45, 14, 20], l=[1.0, 14 / 45, 20 / 45]),
 }
 
