@@ -1283,6 +1283,83 @@ __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const
   }
 }
 
+// The FP64 ACDI step without LDS: a wave is 64 consecutive cells of the halo'd
+// plane, its own the inner 62, whatever the row length, where a tile's last
+// column leaves lanes idle. The cell above in x and the flux of the face below
+// come from the lanes beside, the face below in z from the level before (kz
+// planes a block); the face below in y is evaluated again, four faces a cell
+// instead of three. Bound by memory latency at these sizes. Same expressions
+// and values as k_acdi_sf: 96x96x192 77 -> 66 us, 90x75x130 42 -> 29,
+// 120x78x130 46 -> 40; but 920 -> 1010 at 256x256x512, whose tiles are full:
+// see fz_launch_acdi_step.
+constexpr int ROW_W = 62;
+struct Acd5 {
+  double ps, ph, nx, ny, nz;
+};
+__global__ void __launch_bounds__(256) k_acdi_row(
+    fz_dims d, int kz, const double *__restrict__ dzci, const double *__restrict__ dzfi, double dxi, double dyi,
+    const double *__restrict__ d_gam, double gam_v, double seps, double factor1_v, double factor2_v,
+    const double *__restrict__ stc, int first, const double *__restrict__ u, const double *__restrict__ v,
+    const double *__restrict__ w, const double *__restrict__ normx, const double *__restrict__ normy,
+    const double *__restrict__ normz, const double *__restrict__ phi, const double *__restrict__ psio,
+    double *__restrict__ dpsio, double *__restrict__ psi_out, double *__restrict__ flux_x,
+    double *__restrict__ flux_y, double *__restrict__ flux_z) {
+  const unsigned gx = gridDim.x, L = fz_xcd_block(blockIdx.x + gx * blockIdx.z, gx * gridDim.z);
+  const unsigned bz = L / gx, bx = L - bz * gx;
+  const double gam = d_gam ? *d_gam : gam_v;
+  const double factor1 = stc ? stc[FZ_STC_F1] : factor1_v, factor2 = stc ? stc[FZ_STC_F2] : factor2_v;
+  const double gs = gam * seps, g4 = 0.25 * gam;
+  const int lane = threadIdx.x & 63, sy = (int)d.sy, cells = sy * d.n2;
+  const int f = (int)(bx * 4 + (threadIdx.x >> 6)) * ROW_W + lane - 1;
+  const unsigned e = (unsigned)(sy + min(f, cells));
+  const int j = (int)(e / (unsigned)sy), i = (int)e - j * sy;
+  const bool act = lane >= 1 && lane <= ROW_W && f < cells && i >= 1 && i <= d.n1;
+  const int k0 = (int)bz * kz + 1, kend = min(k0 + kz - 1, d.n3);
+  const BufFld<double> GU = buf_fld(u, d), GV = buf_fld(v, d), GW = buf_fld(w, d);
+  const BufFld<double> GNX = buf_fld(normx, d), GNY = buf_fld(normy, d), GNZ = buf_fld(normz, d),
+                       GPH = buf_fld(phi, d), GPS = buf_fld(psio, d);
+  auto load = [&](unsigned q) { return Acd5{GPS(q, 0), GPH(q, 0), GNX(q, 0), GNY(q, 0), GNZ(q, 0)}; };
+  const unsigned sz = (unsigned)d.sz, usy = (unsigned)sy;
+  unsigned q = e + sz * (unsigned)k0;
+  Acd5 C = load(q);
+  double zu, zr;
+  {
+    const Acd5 B = load(q - sz);
+    acdi_face<2, double>(B.ps, C.ps, B.ph, C.ph, B.nx, C.nx, B.ny, C.ny, B.nz, C.nz, GW(q - sz, 0),
+                         dzci[k0 - 1], gs, g4, seps, zu, zr);
+  }
+  for (int k = k0; k <= kend; k++, q += sz) {
+    const long r = act ? (i - 1) + (long)d.n1 * ((j - 1) + (long)d.n2 * (k - 1)) : 0;
+    const Acd5 Z = load(q + sz), N = load(q + usy), S = load(q - usy);
+    const double uc = GU(q, 0), vc = GV(q, 0), vs = GV(q - usy, 0), wc = GW(q, 0);
+    const double Rp = first ? 0 : dpsio[r];
+    double xu, xr, yu, yr, su, sr, wu, wr;
+    acdi_face<0, double>(C.ps, lane_up(C.ps, C.ps), C.ph, lane_up(C.ph, C.ph), C.nx, lane_up(C.nx, C.nx), C.ny,
+                         lane_up(C.ny, C.ny), C.nz, lane_up(C.nz, C.nz), uc, dxi, gs, g4, seps, xu, xr);
+    acdi_face<1, double>(S.ps, C.ps, S.ph, C.ph, S.nx, C.nx, S.ny, C.ny, S.nz, C.nz, vs, dyi, gs, g4, seps, su, sr);
+    acdi_face<1, double>(C.ps, N.ps, C.ph, N.ph, C.nx, N.nx, C.ny, N.ny, C.nz, N.nz, vc, dyi, gs, g4, seps, yu, yr);
+    acdi_face<2, double>(C.ps, Z.ps, C.ph, Z.ph, C.nx, Z.nx, C.ny, Z.ny, C.nz, Z.nz, wc, dzci[k], gs, g4,
+                         seps, wu, wr);
+    const double xmu = lane_down(xu, xu), xmr = lane_down(xr, xr);
+    if (act) {
+      const double dzfi_c = dzfi[k];
+      const double adv = dxi * (xu - xmu) + dyi * (yu - su) + dzfi_c * (wu - zu);
+      const double rglr = (xr - xmr) * dxi + (yr - sr) * dyi + (wr - zr) * dzfi_c;
+      const double R = -adv + rglr;
+      const double Ro = first ? R : Rp;
+      dpsio[r] = R;
+      flux_x[q] = xu - xr;
+      flux_y[q] = yu - yr;
+      flux_z[q] = wu - wr;
+      const double pn = C.ps + factor1 * R + factor2 * Ro;
+      psi_out[q] = fmin(fmax(0.0, pn), 1.0);
+    }
+    zu = wu;
+    zr = wr;
+    C = Z;
+  }
+}
+
 template <typename T>
 int fz_launch_acdi_step(fz_ctx *c, const double *d_gam, double gam, double seps, double factor1, double factor2,
                         const double *stc, int first, const double *u, const double *v, const double *w,
@@ -1293,7 +1370,24 @@ int fz_launch_acdi_step(fz_ctx *c, const double *d_gam, double gam, double seps,
   // 1000-1040 us for the LDS kernel of six faces per cell (1), FP32 547
   // against 557 us; the LDS kernel measured FP32 619 against 663 us and
   // FP64 1047 against 1120 us for the plain one (2)
-  const int variant = c->acdi_variant ? c->acdi_variant : 3;
+  // (FP64 tiles whose last column or row leaves more than a fourteenth of the
+  // lanes idle: waves over the plane's rows (4); equal at 300x180x200, 6 %
+  // idle, and 0-10 % slower where the tiles are full)
+  const double fill = (double)c->d.n1 / ((c->d.n1 + ACD_MX - 1) / ACD_MX * ACD_MX) * c->d.n2 /
+                      ((c->d.n2 + ACD_MY - 1) / ACD_MY * ACD_MY);
+  const bool ragged = sizeof(T) == 8 && c->d.n2 > 2 && fill < 13.0 / 14.0;
+  const int variant = c->acdi_variant ? c->acdi_variant : (ragged ? 4 : 3);
+  if constexpr (sizeof(T) == 8) {
+    if (variant == 4) {  // waves over the plane's rows
+      dim3 grid((unsigned)(((long)c->d.sy * c->d.n2 + 4 * ROW_W - 1) / (4 * ROW_W)));
+      const int kz = march_planes(c, grid, c->d.n3, 1, 4);
+      FZ_LAUNCH(c, "acdi_step", k_acdi_row, grid, dim3(256), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+                d_gam, gam, seps, factor1, factor2, stc, first, u, v, w, normx, normy, normz, phi, psio, dpsio,
+                psi_out, flux_x, flux_y, flux_z);
+      FZ_LAUNCHED();
+      return xper ? xhalo_copy<T>(c, flux_x, flux_y, flux_z, psi_out) : FZ_OK;
+    }
+  }
   if (variant == 3) {  // each face evaluated once
     // (the x-halo stores compiled only into the instance that makes them; a
     // run-time test there too: measured 550 against 565 us in FP32 without

@@ -362,3 +362,27 @@ def test_tiles_of_thin_boxes_match_the_plain_kernels(n, precision, monkeypatch):
     finally:
         for dc in tiled + batched + plain:
             dc.close()
+
+
+@pytest.mark.parametrize("n", [[5, 3, 2], [33, 7, 9], [60, 5, 6], [65, 4, 33], [96, 6, 7]],
+                         ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("walls", [False, True], ids=["bubble", "walls"])
+def test_phase_steps_over_rows_match_the_tiles(n, walls, monkeypatch):
+    """The ACDI step whose waves own 62 cells of the halo'd plane (taken where
+    tiles would idle) against the tiled kernel bit for bit: rows shorter than
+    a wave, of one wave's cells, and across waves; one block and several in z."""
+    spec = cases.rising_bubble_3d(ng=tuple(n))
+    if walls:
+        spec = dict(cases.hysing_2d(ng=(n[0], 2, n[2])), ng=n, l=[1.0, n[1] / n[0], n[2] / n[0]])
+    out = []
+    for variant in ("3", "4"):
+        monkeypatch.setenv("FZ_ACDI_VARIANT", variant)
+        dc = F.DeviceCase(spec)
+        try:
+            dc.init()
+            dc.step(4)
+            out.append({k: dc.get(k) for k in FIELDS})
+        finally:
+            dc.close()
+    for k in FIELDS:
+        assert np.array_equal(out[0][k], out[1][k], equal_nan=True), k
