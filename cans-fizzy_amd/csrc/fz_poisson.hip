@@ -2236,7 +2236,13 @@ static int solver_rest(fz_ctx *ctx, T *W, double *p, int accum) {
     // rows per chunk: the context's choice (FP32 columns move half the
     // bytes per load, so their default keeps twice the rows in flight)
     int tk = mixed ? ctx->tk32 : ctx->tk64;
-    const bool reg = tk == 0 && P->zpre && reg_fits<T>(ctx);
+    // (FP32 columns of more than 256 rows, once about 49152 of them fill the
+    // device: two columns a lane move wider lines at 5.5 TB/s, 192 against
+    // 217 us at 256x256x512, 143 against 167 at 256x256x384, 180 against 187
+    // at 224x224x512; but 166 against 131 at 192x192x512, and 95 against 77
+    // at 256^3)
+    const bool pairs = mixed && ps % 2 == 0 && ctx->d.n3 > 256 && ps >= 49152;
+    const bool reg = tk == 0 && P->zpre && reg_fits<T>(ctx) && !pairs;
     if (tk == 0) tk = mixed ? -8 : 16;
     const dim3 grid((int)((ps + 63) / 64)), blk(64);
     const char *name = mixed ? "thomas_f32" : "thomas";

@@ -386,3 +386,15 @@ def test_phase_steps_over_rows_match_the_tiles(n, walls, monkeypatch):
             dc.close()
     for k in FIELDS:
         assert np.array_equal(out[0][k], out[1][k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("n", [[256, 192, 257], [245, 225, 257]], ids=["even columns", "odd columns"])
+def test_many_long_fp32_columns(n, rng, monkeypatch):
+    """FP32 columns of more than 256 rows go two to a lane where an even number
+    of at least 49152 fill the device, an odd number in registers: as the
+    chunked kernel's bit for bit."""
+    f = np.asfortranarray(rng.uniform(-1.0, 1.0, [x + 2 for x in n]))
+    monkeypatch.delenv("FZ_THOMAS_ROWS32", raising=False)
+    got = solve(n, "PPPPNN", f, True)
+    monkeypatch.setenv("FZ_THOMAS_ROWS32", "16")
+    assert np.array_equal(got, solve(n, "PPPPNN", f, True))
