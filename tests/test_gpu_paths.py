@@ -1,6 +1,6 @@
 """Launch shapes chosen from the grid give the fields of any other choice.
 
-The z-marching kernels (momentum, ACDI step, correction, normals) take their
+The z-marching kernels (momentum, phase-field step, normals) take their
 planes per block from the grid; FZ_MARCH_PLANES, read when a context is made,
 fixes the number. Every number gives the same fields bit for bit."""
 import ctypes as C
