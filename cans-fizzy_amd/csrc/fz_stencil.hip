@@ -1472,18 +1472,14 @@ __global__ void k_vof_phi(long nh, double beta_d, const T *__restrict__ psi, T *
   }
 }
 
-// vof_thinc_transport_psi fluxes, src/vof_thinc_qq.f90:66-121 (faces 0..n)
+// vof_thinc_transport_psi's fluxes through the + faces of cell q, src/vof_thinc_qq.f90:66-121
 template <typename T>
-__global__ void k_vof_flux(fz_dims d, double beta_d, const double *__restrict__ u, const double *__restrict__ v,
-                           const double *__restrict__ w, const T *__restrict__ normx, const T *__restrict__ normy,
-                           const T *__restrict__ normz, const T *__restrict__ phi, T *__restrict__ flux_x,
-                           T *__restrict__ flux_y, T *__restrict__ flux_z) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int j = blockIdx.y * blockDim.y + threadIdx.y;
-  const int k = blockIdx.z;
-  if (i > d.n1 || j > d.n2) return;
-  const T beta = (T)beta_d;
-  const long q = i + d.sy * j + d.sz * k;
+__device__ __forceinline__ void vof_flux_cell(const fz_dims &d, long q, T beta, const double *__restrict__ u,
+                                              const double *__restrict__ v, const double *__restrict__ w,
+                                              const T *__restrict__ normx, const T *__restrict__ normy,
+                                              const T *__restrict__ normz, const T *__restrict__ phi,
+                                              T *__restrict__ flux_x, T *__restrict__ flux_y,
+                                              T *__restrict__ flux_z) {
   const T vel_x = (T)u[q], vel_y = (T)v[q], vel_z = (T)w[q];
   long qx, qy, qz;
   T xx, yy, zz;
@@ -1497,11 +1493,48 @@ __global__ void k_vof_flux(fz_dims d, double beta_d, const double *__restrict__ 
   flux_y[q] = vel_y * lfy;
   flux_z[q] = vel_z * lfz;
 }
+// (cells 0..n in every direction)
+template <typename T>
+__global__ void k_vof_flux(fz_dims d, double beta_d, const double *__restrict__ u, const double *__restrict__ v,
+                           const double *__restrict__ w, const T *__restrict__ normx, const T *__restrict__ normy,
+                           const T *__restrict__ normz, const T *__restrict__ phi, T *__restrict__ flux_x,
+                           T *__restrict__ flux_y, T *__restrict__ flux_z) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int j = blockIdx.y * blockDim.y + threadIdx.y;
+  const int k = blockIdx.z;
+  if (i > d.n1 || j > d.n2) return;
+  vof_flux_cell<T>(d, i + d.sy * j + d.sz * k, (T)beta_d, u, v, w, normx, normy, normz, phi, flux_x, flux_y, flux_z);
+}
+// the cells of k_vof_flux that k_vof_step leaves out, those with an index 0:
+// the plane k = 0, then the rows j = 0 and the cells i = 0 of the others
+__global__ void __launch_bounds__(256) k_vof_flux_low(fz_dims d, double beta, const double *__restrict__ u,
+                                                      const double *__restrict__ v, const double *__restrict__ w,
+                                                      const double *__restrict__ normx,
+                                                      const double *__restrict__ normy,
+                                                      const double *__restrict__ normz,
+                                                      const double *__restrict__ phi, double *__restrict__ flux_x,
+                                                      double *__restrict__ flux_y, double *__restrict__ flux_z) {
+  const long m1 = d.n1 + 1, plane = m1 * (d.n2 + 1), edge = m1 + d.n2;
+  const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= plane + edge * d.n3) return;
+  long i, j, k = 0;
+  if (t < plane) {
+    j = t / m1;
+    i = t - j * m1;
+  } else {
+    k = (t - plane) / edge;
+    const long r = t - plane - k * edge;
+    k++;
+    i = r < m1 ? r : 0;
+    j = r < m1 ? 0 : r - m1 + 1;
+  }
+  vof_flux_cell<double>(d, i + d.sy * j + d.sz * k, beta, u, v, w, normx, normy, normz, phi, flux_x, flux_y, flux_z);
+}
 
 constexpr int VOF_W = 62;  // cells of a wave of k_vof_step
 
 // THINC/QQ flux through the face between a cell and the one above it, the
-// expression of k_vof_flux, from both cells' normal and phi
+// expression of vof_flux_cell, from both cells' normal and phi
 template <typename T>
 __device__ __forceinline__ T vof_face_flux(T beta, T vv, T n, T ph, T n_up, T ph_up) {
   const bool own = vv > (T)0.0;
@@ -3110,6 +3143,11 @@ int fz_launch_rk_2fl_fused(fz_ctx *c, double factor1, double factor2, int first,
     FZ_LAUNCH(c, "rk_vof", (k_vof_step<double, true>), grid, dim3(256), 0, c->d, kz, c->dzfi,
               c->dli[0], c->dli[1], beta, factor1, factor2, stc, first, u, v, w, nx, ny, nz, phi, psi, dpsio, ps, fx,
               fy, fz);
+    FZ_LAUNCHED();
+    // (the transport of the routine has the faces at index 0 too, which a case's step sets as boundary values)
+    const long low = (long)(c->d.n1 + 1) * (c->d.n2 + 1) + (long)(c->d.n1 + 1 + c->d.n2) * c->d.n3;
+    FZ_LAUNCH(c, "rk_vof_low", k_vof_flux_low, dim3((unsigned)((low + 255) / 256)), dim3(256), 0, c->d, beta, u, v, w,
+              nx, ny, nz, phi, fx, fy, fz);
   } else {
     dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY);
     const int kz = march_planes(c, grid, c->d.n3, 1, 3);

@@ -398,3 +398,33 @@ def test_many_long_fp32_columns(n, rng, monkeypatch):
     got = solve(n, "PPPPNN", f, True)
     monkeypatch.setenv("FZ_THOMAS_ROWS32", "16")
     assert np.array_equal(got, solve(n, "PPPPNN", f, True))
+
+
+@pytest.mark.parametrize("n", [[1, 1, 2], [5, 3, 2], [33, 7, 9], [64, 8, 17], [70, 13, 40]],
+                         ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("vof", [0, 1], ids=["acdi", "thinc"])
+def test_rk_2fl_writes_the_faces_of_its_transport(n, vof, rng):
+    """The flux arrays after rk_2fl are the transport routine's in every
+    element, halo included: THINC/QQ has the faces at index 0 (src/
+    vof_thinc_qq.f90:66-121), and what neither writes keeps its value."""
+    ctx = F.Context(n, [1.0, 0.9, 1.7], "PPPPNN", gr=0.5)
+    try:
+        rand = lambda lo=-1.0, hi=1.0: np.asfortranarray(rng.uniform(lo, hi, [x + 2 for x in n]))  # noqa: E731
+        h = {q: ctx.halo(rand()) for q in ("u", "v", "w", "nx", "ny", "nz", "phi")}
+        h["psi"] = ctx.halo(rand(0.0, 1.0))
+        before = [rand() for _ in range(3)]
+        one, two = [ctx.halo(f) for f in before], [ctx.halo(f) for f in before]
+        args = [h[q].ptr for q in ("u", "v", "w", "nx", "ny", "nz", "phi", "psi")]
+        name, par = ("fz_vof_thinc_transport_psi", [40.0]) if vof else ("fz_acdi_transport_pf", [0.7, 0.02])
+        F.call(name, ctx.h, *par, *args, ctx.interior().ptr, *[d.ptr for d in one])
+        st = C.c_void_p()
+        F.call("fz_rk_state_create", ctx.h, C.byref(st))
+        F.call("fz_rk_2fl", ctx.h, st, (C.c_double * 2)(1.5, -0.5), 1e-3, 0.7, 0.02, 40.0, vof, *args,
+               *[d.ptr for d in two])
+        for a, b, f in zip(one, two, before):
+            a = a.download()
+            assert np.array_equal(b.download(), a)
+            assert not np.array_equal(a, f)
+        F.lib().fz_rk_state_destroy(st)
+    finally:
+        ctx.close()
