@@ -11,6 +11,7 @@
 //    previous step, which then becomes po; pn is p itself (pn == p whenever
 //    mom_xyz_oth reads it).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -112,6 +113,8 @@ struct fz_case {
     hipGraphExec_t exec = nullptr;
     const void *key[2] = {nullptr, nullptr};
   } graph[2];
+  // false once the case is destroyed: a batch of it may be there still
+  std::shared_ptr<std::atomic<bool>> alive = std::make_shared<std::atomic<bool>>(true);
 };
 
 // fields held in FP32 by the mixed-precision mode
@@ -201,6 +204,7 @@ static int case_alloc(fz_case *cs) {
 
 extern "C" int fz_case_destroy(fz_case *cs) {
   if (!cs) return FZ_OK;
+  *cs->alive = false;
   if (cs->ctx) (void)hipStreamSynchronize(cs->ctx->st);
   for (int q = 0; q < F_N; q++) {
     if (cs->f[q]) (void)hipFree(cs->f[q]);
@@ -946,6 +950,7 @@ int fz_bounds_group_batch(fz_ctx *c, int n, const FzBcItem *items, const int *ro
 
 struct fz_case_batch {
   std::vector<fz_case *> cs;
+  std::vector<std::shared_ptr<std::atomic<bool>>> alive;  // of each case: a destroyed one is not touched
   fz_bcase *dtab = nullptr;  // the role table, one entry per case
   int *dpar = nullptr;       // each case's pointer state
   void **dsolve = nullptr;   // the correction buffers, work arrays and pivots of the cases
@@ -1045,7 +1050,8 @@ static int batch_join(fz_case_batch *b, fz_ctx *c0, fz_ctx *c) {
 
 extern "C" int fz_case_batch_destroy(fz_case_batch *b) {
   if (!b) return FZ_OK;
-  if (!b->cs.empty()) (void)hipStreamSynchronize(b->cs[0]->ctx->st);
+  // (the first case's end waited for its stream, and with it for the batch's work)
+  if (!b->cs.empty() && *b->alive[0]) (void)hipStreamSynchronize(b->cs[0]->ctx->st);
   while (!b->guests.empty()) batch_part(b->guests.back());
   if (b->dtab) (void)hipFree(b->dtab);
   if (b->dpar) (void)hipFree(b->dpar);
@@ -1066,6 +1072,7 @@ extern "C" int fz_case_batch_create(fz_case *const *cases, int n, fz_case_batch 
   }
   fz_case_batch *b = new fz_case_batch();
   b->cs.assign(cases, cases + n);
+  for (const fz_case *cs : b->cs) b->alive.push_back(cs->alive);
   b->mixed = cases[0]->precision == FZ_PREC_MIXED;
   std::vector<fz_bcase> tab(n);
   std::vector<void *> sol(3 * (size_t)n);
@@ -1214,14 +1221,15 @@ static int batch_leave(fz_case_batch *b) {
 }
 
 // the checks enqueued by a step read back: the next dt and the stop conditions
+// (of the cases that are still there)
 static int batch_checks(fz_case_batch *b, int *killed, bool *stop) {
   bool pending = false;
-  for (fz_case *cs : b->cs) pending = pending || cs->check_pending;
+  for (size_t q = 0; q < b->cs.size(); q++) pending = pending || (*b->alive[q] && b->cs[q]->check_pending);
   if (!pending) return FZ_OK;
-  FZ_HIP(hipStreamSynchronize(b->cs[0]->ctx->st));
+  if (*b->alive[0]) FZ_HIP(hipStreamSynchronize(b->cs[0]->ctx->st));
   for (size_t q = 0; q < b->cs.size(); q++) {
     fz_case *cs = b->cs[q];
-    if (!cs->check_pending) continue;
+    if (!*b->alive[q] || !cs->check_pending) continue;
     int kill = 0;
     check_finish(cs, &kill);
     if (kill) {
@@ -1229,6 +1237,15 @@ static int batch_checks(fz_case_batch *b, int *killed, bool *stop) {
       if (killed) killed[q] = 1;
     }
   }
+  return FZ_OK;
+}
+
+// why the batch cannot step now (FZ_OK: it can)
+static int batch_ready(const fz_case_batch *b, const char *who) {
+  for (const auto &a : b->alive)
+    if (!*a) return fz_set_error(FZ_ERR_STATE, "%s: a case of the batch has been destroyed", who);
+  for (const fz_case *cs : b->cs)
+    if (cs->check_pending) return fz_set_error(FZ_ERR_STATE, "%s: a case has a step not ended", who);
   return FZ_OK;
 }
 
@@ -1252,8 +1269,7 @@ extern "C" int fz_case_batch_step(fz_case_batch *b, int nsteps, int *killed) {
   const int n = (int)b->cs.size();
   if (killed)
     for (int q = 0; q < n; q++) killed[q] = 0;
-  for (fz_case *cs : b->cs)
-    if (cs->check_pending) return fz_set_error(FZ_ERR_STATE, "fz_case_batch_step: a case has a step not ended");
+  FZ_TRY(batch_ready(b, "fz_case_batch_step"));
   FZ_TRY(batch_enter(b));
   int rc = FZ_OK;
   bool stop = false;
@@ -1269,8 +1285,7 @@ extern "C" int fz_case_batch_step(fz_case_batch *b, int nsteps, int *killed) {
 extern "C" int fz_case_batch_step_begin(fz_case_batch *b, int *check_pending) {
   if (!b) return fz_set_error(FZ_ERR_ARG, "fz_case_batch_step_begin: null batch");
   if (b->pending) return fz_set_error(FZ_ERR_STATE, "fz_case_batch_step_begin: the previous step has not ended");
-  for (fz_case *cs : b->cs)
-    if (cs->check_pending) return fz_set_error(FZ_ERR_STATE, "fz_case_batch_step_begin: a case has a step not ended");
+  FZ_TRY(batch_ready(b, "fz_case_batch_step_begin"));
   FZ_TRY(batch_enter(b));
   bool pending = false;
   int rc = batch_step_enqueue(b, &pending);

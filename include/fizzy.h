@@ -310,7 +310,8 @@ int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size_t cap);
  * each case's later work waits for it. nsteps steps, or fewer when a check
  * stops a case (killed[q] = 1; killed may be null); cases must not be
  * stepped otherwise while in a batch, and a batch must be made again once
- * its cases have been stepped alone. */
+ * its cases have been stepped alone. The cases may be destroyed before it, in
+ * any order: a step of it then returns FZ_ERR_STATE, and destroy frees it. */
 typedef struct fz_case_batch fz_case_batch;
 int fz_case_batch_create(fz_case *const *cases, int n, fz_case_batch **batch);
 int fz_case_batch_step(fz_case_batch *batch, int nsteps, int *killed);
