@@ -128,15 +128,14 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
   for (int d = 0; d < 3; d++) c->per[d] = (cbcpre[2 * d] == 'P' && cbcpre[2 * d + 1] == 'P');
   hipError_t e;
   if (hip_stream) {
-    c->st = (hipStream_t)hip_stream;
+    c->own = (hipStream_t)hip_stream;
   } else {
-    e = hipStreamCreateWithFlags(&c->st, hipStreamNonBlocking);
+    e = hipStreamCreateWithFlags(&c->own, hipStreamNonBlocking);
     if (e != hipSuccess) {
       delete c;
       return fz_set_error(FZ_ERR_HIP, "hipStreamCreate: %s", hipGetErrorString(e));
     }
-    c->home = std::make_shared<fz_stream_own>();
-    c->home->s = c->st;
+    c->own_made = true;
   }
   double **dev[6] = {&c->dzc, &c->dzf, &c->zc, &c->zf, &c->dzci, &c->dzfi};
   const std::vector<double> *host[6] = {&c->h_dzc, &c->h_dzf, &c->h_zc, &c->h_zf, &c->h_dzci, &c->h_dzfi};
@@ -168,7 +167,7 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
 
 extern "C" int fz_ctx_destroy(fz_ctx *c) {
   if (!c) return FZ_OK;
-  if (c->st) (void)hipStreamSynchronize(c->st);
+  if (c->own) (void)hipStreamSynchronize(c->stream());
   double *dev[6] = {c->dzc, c->dzf, c->zc, c->zf, c->dzci, c->dzfi};
   for (int q = 0; q < 6; q++)
     if (dev[q]) (void)hipFree(dev[q]);
@@ -183,22 +182,19 @@ extern "C" int fz_ctx_destroy(fz_ctx *c) {
   if (c->ftab) (void)hipFree(c->ftab);
   if (c->h_small) (void)hipHostFree(c->h_small);
   if (c->ev) (void)hipEventDestroy(c->ev);
-  if (c->guest_of) fz_batch_forget(c->guest_of, c);
-  delete c;  // (and with it its stream, unless a batch's cases still use it)
+  if (c->own_made) (void)hipStreamDestroy(c->own);
+  delete c;
   return FZ_OK;
 }
 
-int fz_stream_after(hipStream_t later, fz_ctx *c) {
-  if (later == c->st) return FZ_OK;
-  if (!c->ev) FZ_HIP(hipEventCreateWithFlags(&c->ev, hipEventDisableTiming));
-  FZ_HIP(hipEventRecord(c->ev, c->st));
-  FZ_HIP(hipStreamWaitEvent(later, c->ev, 0));
-  return FZ_OK;
+void fz_ctx::catch_up() {
+  if (hipStreamWaitEvent(own, behind->e, 0) != hipSuccess) (void)hipEventSynchronize(behind->e);
+  behind.reset();
 }
 
 extern "C" int fz_ctx_sync(fz_ctx *c) {
   if (!c) return fz_set_error(FZ_ERR_ARG, "fz_ctx_sync: null context");
-  FZ_HIP(hipStreamSynchronize(c->st));
+  FZ_HIP(hipStreamSynchronize(c->stream()));
   return FZ_OK;
 }
 
@@ -211,7 +207,7 @@ extern "C" int fz_malloc(fz_ctx *c, size_t bytes, void **dptr) {
 extern "C" int fz_free(fz_ctx *c, void *dptr) {
   if (!c) return fz_set_error(FZ_ERR_ARG, "fz_free: null context");
   if (dptr) {
-    FZ_HIP(hipStreamSynchronize(c->st));
+    FZ_HIP(hipStreamSynchronize(c->stream()));
     FZ_HIP(hipFree(dptr));
   }
   return FZ_OK;
@@ -219,15 +215,15 @@ extern "C" int fz_free(fz_ctx *c, void *dptr) {
 
 extern "C" int fz_upload(fz_ctx *c, void *dst, const void *src, size_t bytes) {
   if (!c || (!dst && bytes) || (!src && bytes)) return fz_set_error(FZ_ERR_ARG, "fz_upload: null argument");
-  FZ_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->st));
-  FZ_HIP(hipStreamSynchronize(c->st));
+  FZ_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, c->stream()));
+  FZ_HIP(hipStreamSynchronize(c->stream()));
   return FZ_OK;
 }
 
 extern "C" int fz_download(fz_ctx *c, void *dst, const void *src, size_t bytes) {
   if (!c || (!dst && bytes) || (!src && bytes)) return fz_set_error(FZ_ERR_ARG, "fz_download: null argument");
-  FZ_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->st));
-  FZ_HIP(hipStreamSynchronize(c->st));
+  FZ_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c->stream()));
+  FZ_HIP(hipStreamSynchronize(c->stream()));
   return FZ_OK;
 }
 
@@ -249,7 +245,8 @@ extern "C" int fz_copy(fz_ctx *c, void *dst, const void *src, size_t bytes) {
   }
   const size_t done = nvec * 16;
   if (done < bytes)
-    FZ_HIP(hipMemcpyAsync((char *)dst + done, (const char *)src + done, bytes - done, hipMemcpyDeviceToDevice, c->st));
+    FZ_HIP(hipMemcpyAsync((char *)dst + done, (const char *)src + done, bytes - done, hipMemcpyDeviceToDevice,
+                          c->stream()));
   return FZ_OK;
 }
 
@@ -268,14 +265,14 @@ static hipEvent_t prof_event(fz_ctx *c) {
 fz_prof_scope::fz_prof_scope(fz_ctx *c_, const char *n) : c(c_), name(n) {
   if (!c || !c->prof_on) return;
   a = prof_event(c);
-  if (a) (void)hipEventRecord(a, c->st);
+  if (a) (void)hipEventRecord(a, c->stream());
 }
 
 fz_prof_scope::~fz_prof_scope() {
   if (!a) return;
   hipEvent_t b = prof_event(c);
   if (!b) return;
-  (void)hipEventRecord(b, c->st);
+  (void)hipEventRecord(b, c->stream());
   c->prof_recs.push_back(fz_prof_rec{name, a, b});
 }
 
@@ -288,7 +285,7 @@ extern "C" int fz_prof_enable(fz_ctx *c, int on) {
 // "name calls total_ms" lines, one per launch site, in first-seen order; clears the records
 extern "C" int fz_prof_report(fz_ctx *c, char *buf, size_t cap) {
   if (!c || !buf || cap == 0) return fz_set_error(FZ_ERR_ARG, "fz_prof_report: bad argument");
-  FZ_HIP(hipStreamSynchronize(c->st));
+  FZ_HIP(hipStreamSynchronize(c->stream()));
   std::vector<const char *> names;
   std::vector<double> tot;
   std::vector<long> cnt;
@@ -321,7 +318,7 @@ extern "C" int fz_prof_report(fz_ctx *c, char *buf, size_t cap) {
 int fz_reduce_ensure(fz_ctx *c, size_t nblocks) {
   if (nblocks <= c->red_cap) return FZ_OK;
   if (c->red) {
-    FZ_HIP(hipStreamSynchronize(c->st));
+    FZ_HIP(hipStreamSynchronize(c->stream()));
     FZ_HIP(hipFree(c->red));
     c->red = nullptr;
   }

@@ -80,11 +80,11 @@ struct fz_prof_rec {
   hipEvent_t a, b;
 };
 
-// a stream the library made, kept until its last context lets go of it
-struct fz_stream_own {
-  hipStream_t s = nullptr;
-  ~fz_stream_own() {
-    if (s) (void)hipStreamDestroy(s);
+// an event kept until the last one that waits for it lets go of it
+struct fz_event_own {
+  hipEvent_t e = nullptr;
+  ~fz_event_own() {
+    if (e) (void)hipEventDestroy(e);
   }
 };
 
@@ -99,11 +99,23 @@ struct fz_ctx {
   double *dzc = nullptr, *dzf = nullptr, *zc = nullptr, *zf = nullptr, *dzci = nullptr, *dzfi = nullptr;
   char cbcpre[6];
   int per[3];
-  hipStream_t st = nullptr;
-  std::shared_ptr<fz_stream_own> home;   // the context's own stream (null: the caller gave one)
-  std::shared_ptr<fz_stream_own> guest;  // in a batch: the first case's stream, which st is then
-  fz_case_batch *guest_of = nullptr;     // that batch
-  hipEvent_t ev = nullptr;               // orders other streams after this context's (fz_ctx_event)
+  hipStream_t own = nullptr;  // the context's stream for its whole life (work goes to stream())
+  bool own_made = false;      // the library made it (only the context's calls use it)
+  // A batched step's work on the context runs on the batch's stream (lent,
+  // while the step is enqueued). Nobody but the context's own thread looks at
+  // the members below outside such a step.
+  hipStream_t lent = nullptr;
+  std::shared_ptr<fz_event_own> behind;  // the end of that work, which own has not waited for yet
+  bool used = true;                      // own may hold work that no batch's stream has waited for
+  hipEvent_t ev = nullptr;               // the end of own's work, for a batch's stream
+  // the stream that the context's next work goes to, in order after all its work so far
+  hipStream_t stream() {
+    if (lent) return lent;
+    if (behind) catch_up();
+    used = true;
+    return own;
+  }
+  void catch_up();
   fz_poisson *pois = nullptr;
   double *red = nullptr;      // per-block partial results of reductions
   size_t red_cap = 0;
@@ -148,7 +160,7 @@ struct fz_prof_scope {
 #define FZ_LAUNCH(c, name, kernel, grid, block, shmem, ...)                              \
   do {                                                                                   \
     fz_prof_scope fz_ps_((c), name);                                                     \
-    hipLaunchKernelGGL(kernel, grid, block, shmem, (c)->st, __VA_ARGS__);                \
+    hipLaunchKernelGGL(kernel, grid, block, shmem, (c)->stream(), __VA_ARGS__);                \
   } while (0)
 
 // Workgroups are dealt round-robin to the 8 XCDs in dispatch order, each XCD
@@ -229,13 +241,12 @@ static inline dim3 fz_grid_halo(const fz_dims &d) {
 }
 
 // internal entry points shared between translation units
-int fz_stream_after(hipStream_t later, fz_ctx *c);  // later work on the stream waits for c's work so far
-void fz_batch_forget(fz_case_batch *b, fz_ctx *c);  // a context on the batch's stream goes
 int fz_reduce_ensure(fz_ctx *ctx, size_t nblocks);
 int fz_scratch_setup(fz_ctx *ctx);
 int fz_batch_solve(fz_ctx *c0, void **dptrs, int n);
 // why cs cannot join a batched step led by first (null: it can)
 const char *fz_case_batch_refusal(const fz_case *first, const fz_case *cs);
+hipStream_t fz_case_batch_stream(const fz_case_batch *b);
 void fz_bcmaps_free(fz_ctx *ctx);
 int fz_poisson_destroy(fz_poisson *p);
 int fz_solver_dev(fz_ctx *ctx, double *p);

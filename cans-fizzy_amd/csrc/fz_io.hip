@@ -40,7 +40,7 @@ static int pack_interior(fz_ctx *c, const int s[3], int to_packed, double *field
   FZ_HIP(hipMalloc((void **)&buf, sizeof(double) * n));
   int rc = FZ_OK;
   hipError_t e = hipSuccess;
-  if (!to_packed) e = hipMemcpyAsync(buf, host.data(), sizeof(double) * n, hipMemcpyHostToDevice, c->st);
+  if (!to_packed) e = hipMemcpyAsync(buf, host.data(), sizeof(double) * n, hipMemcpyHostToDevice, c->stream());
   if (e == hipSuccess) {
     const long nb = (n + 255) / 256;
     FZ_LAUNCH(c, "pack", k_pack, dim3((unsigned)nb), dim3(256), 0, d, s[0], s[1], s[2], ni, nj, nk, to_packed, field,
@@ -49,9 +49,9 @@ static int pack_interior(fz_ctx *c, const int s[3], int to_packed, double *field
   }
   if (e == hipSuccess && to_packed) {
     host.resize(n);
-    e = hipMemcpyAsync(host.data(), buf, sizeof(double) * n, hipMemcpyDeviceToHost, c->st);
+    e = hipMemcpyAsync(host.data(), buf, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream());
   }
-  if (e == hipSuccess) e = hipStreamSynchronize(c->st);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream());
   if (e != hipSuccess) rc = fz_set_error(FZ_ERR_HIP, "field transfer: %s", hipGetErrorString(e));
   (void)hipFree(buf);
   return rc;

@@ -1969,7 +1969,7 @@ extern "C" int fz_initsolver(fz_ctx *ctx, const double bcpre[6], double *lambdax
   if (rhsbz_h) memcpy(rhsbz_h, rbz.data(), sizeof(double) * rbz.size());
   // device plan
   if (ctx->pois) {
-    FZ_HIP(hipStreamSynchronize(ctx->st));
+    FZ_HIP(hipStreamSynchronize(ctx->stream()));
     fz_poisson_destroy(ctx->pois);
     ctx->pois = nullptr;
   }
@@ -2309,7 +2309,7 @@ static int mixed_buffers(fz_ctx *ctx) {
   if (!P->work32) FZ_HIP(hipMalloc((void **)&P->work32, sizeof(float) * ctx->ni));
   if (!P->rslots) {
     FZ_HIP(hipMalloc((void **)&P->rslots, sizeof(unsigned long long) * FZ_GAMMA_SLOTS));
-    FZ_HIP(hipMemsetAsync(P->rslots, 0, sizeof(unsigned long long) * FZ_GAMMA_SLOTS, ctx->st));
+    FZ_HIP(hipMemsetAsync(P->rslots, 0, sizeof(unsigned long long) * FZ_GAMMA_SLOTS, ctx->stream()));
   }
   return FZ_OK;
 }
@@ -2402,8 +2402,8 @@ static int read_slots(fz_ctx *ctx, double *out) {
   fz_poisson *P = ctx->pois;
   FZ_LAUNCH(ctx, "slots_max", k_slots_max, dim3(1), dim3(FZ_GAMMA_SLOTS), 0, P->rslots, ctx->red);
   FZ_LAUNCHED();
-  FZ_HIP(hipMemcpyAsync(ctx->h_small + 12, ctx->red, sizeof(double), hipMemcpyDeviceToHost, ctx->st));
-  FZ_HIP(hipStreamSynchronize(ctx->st));
+  FZ_HIP(hipMemcpyAsync(ctx->h_small + 12, ctx->red, sizeof(double), hipMemcpyDeviceToHost, ctx->stream()));
+  FZ_HIP(hipStreamSynchronize(ctx->stream()));
   *out = ctx->h_small[12];
   return FZ_OK;
 }
@@ -2433,7 +2433,7 @@ extern "C" int fz_solver_mixed(fz_ctx *ctx, double *p, double tol, int maxit, in
   FZ_TRY(mixed_buffers(ctx));
   FZ_TRY(fz_reduce_ensure(ctx, 1));
   if (!P->bcopy) FZ_HIP(hipMalloc((void **)&P->bcopy, sizeof(double) * ctx->nh));
-  FZ_HIP(hipMemcpyAsync(P->bcopy, p, sizeof(double) * ctx->nh, hipMemcpyDeviceToDevice, ctx->st));
+  FZ_HIP(hipMemcpyAsync(P->bcopy, p, sizeof(double) * ctx->nh, hipMemcpyDeviceToDevice, ctx->stream()));
   FillSrc fb = fill_src(ctx, 0.0, 0.0, nullptr, nullptr, nullptr);
   fb.on = SRC_B;
   fb.b = P->bcopy;
@@ -2500,7 +2500,7 @@ extern "C" int fz_solver_batched(fz_ctx *const *ctxs, double *const *ps, int n) 
   // each context's pending work on its fields first
   // (sixteen 64^3 solves: waiting for the streams 326 us a call, events between
   // them 375 us, asking each whether it has drained 440 us)
-  for (int q = 0; q < n; q++) FZ_HIP(hipStreamSynchronize(ctxs[q]->st));
+  for (int q = 0; q < n; q++) FZ_HIP(hipStreamSynchronize(ctxs[q]->stream()));
   if (P->batch_cap < 3 * (size_t)n) {
     if (P->batch_ptrs) FZ_HIP(hipFree(P->batch_ptrs));
     P->batch_ptrs = nullptr;
@@ -2522,7 +2522,7 @@ extern "C" int fz_solver_batched(fz_ctx *const *ctxs, double *const *ps, int n) 
     FZ_LAUNCHED();
   }
   FZ_TRY(fz_batch_solve(c0, P->batch_ptrs, n));
-  FZ_HIP(hipStreamSynchronize(c0->st));
+  FZ_HIP(hipStreamSynchronize(c0->stream()));
   return FZ_OK;
 }
 
@@ -2574,7 +2574,7 @@ extern "C" int fz_r2r(fz_ctx *ctx, int kind, int n, int howmany, double *x) {
   FZ_TRY(fftplan_init_kinds(&P, kind, kind, n));
   const LineMap lines = {0, n, 0, 1};
   int rc = launch_r2r<double, double, double>(ctx, "fft_lines", P, kind, x, lines, x, lines, howmany, 1, 1.0);
-  if (rc == FZ_OK && hipStreamSynchronize(ctx->st) != hipSuccess) rc = fz_set_error(FZ_ERR_HIP, "fz_r2r: sync");
+  if (rc == FZ_OK && hipStreamSynchronize(ctx->stream()) != hipSuccess) rc = fz_set_error(FZ_ERR_HIP, "fz_r2r: sync");
   fftplan_free(&P);
   return rc;
 }

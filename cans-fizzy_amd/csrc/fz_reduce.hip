@@ -206,8 +206,8 @@ int fz_acdi_gamma_dev(fz_ctx *c, double gam_factor, double gam_min, const double
 }
 
 static int fetch(fz_ctx *c, const double *d_src, int count, double *out) {
-  FZ_HIP(hipMemcpyAsync(c->h_small, d_src, sizeof(double) * count, hipMemcpyDeviceToHost, c->st));
-  FZ_HIP(hipStreamSynchronize(c->st));
+  FZ_HIP(hipMemcpyAsync(c->h_small, d_src, sizeof(double) * count, hipMemcpyDeviceToHost, c->stream()));
+  FZ_HIP(hipStreamSynchronize(c->stream()));
   for (int q = 0; q < count; q++) out[q] = c->h_small[q];
   return FZ_OK;
 }
@@ -288,10 +288,10 @@ extern "C" int fz_chkdiv_noalloc(fz_ctx *c, const double *u, const double *v, co
   if (nb > FZ_SCRATCH_BLOCKS)
     return fz_set_error(FZ_ERR_ARG, "fz_chkdiv_noalloc: %d partial sums exceed the scratch maximum of %d", nb,
                         FZ_SCRATCH_BLOCKS);
-  hipLaunchKernelGGL(k_red_div, dim3(nb), dim3(RED_THREADS), 0, c->st, c->d, c->dzfi, c->dli[0], c->dli[1], u, v, w,
-                     c->scratch);
+  hipLaunchKernelGGL(k_red_div, dim3(nb), dim3(RED_THREADS), 0, c->stream(), c->d, c->dzfi, c->dli[0], c->dli[1], u,
+                     v, w, c->scratch);
   FZ_LAUNCHED();
-  hipLaunchKernelGGL(k_fin_div, dim3(1), dim3(RED_THREADS), 0, c->st, nb, c->scratch, d_out);
+  hipLaunchKernelGGL(k_fin_div, dim3(1), dim3(RED_THREADS), 0, c->stream(), nb, c->scratch, d_out);
   FZ_LAUNCHED();
   return FZ_OK;
 }
@@ -380,7 +380,7 @@ extern "C" int fz_bulk_mean_12_stag(fz_ctx *c, int idir, const double *psi, cons
   for (int k = 0; k < nz; k++) g[k] = c->dl[0] * c->dl[1] * (idir < 3 ? c->h_dzc[k] : c->h_dzf[k]) / vol;
   double *dg = nullptr;
   FZ_HIP(hipMalloc((void **)&dg, sizeof(double) * nz));
-  (void)hipMemcpyAsync(dg, g.data(), sizeof(double) * nz, hipMemcpyHostToDevice, c->st);
+  (void)hipMemcpyAsync(dg, g.data(), sizeof(double) * nz, hipMemcpyHostToDevice, c->stream());
   double *res = c->red + 2 * (c->red_cap - 4);
   int rc = fz_bulk_mean_dev(c, idir, psi, p12, dg, res);
   if (rc == FZ_OK) rc = fetch(c, res, 1, mean);

@@ -375,11 +375,11 @@ extern "C" int fz_server_round(fz_server *s, int *n_active, int *n_queued) {
         int rc = fz_case_batch_create(cs.data(), (int)cs.size(), &g.b);
         if (rc == FZ_OK && hipEventCreate(&g.e0) != hipSuccess) rc = FZ_ERR_HIP;
         if (rc == FZ_OK && hipEventCreate(&g.e1) != hipSuccess) rc = FZ_ERR_HIP;
-        g.st = s->active[m[0]].ctx->st;
         if (rc != FZ_OK) {  // the cases step alone
           drop_group(g);
           continue;
         }
+        g.st = fz_case_batch_stream(g.b);
       }
       for (size_t q : m) gid[q] = (int)groups.size();
       groups.push_back(g);
@@ -409,9 +409,10 @@ extern "C" int fz_server_round(fz_server *s, int *n_active, int *n_queued) {
       if (!open[q] || r.nq >= want[q]) continue;
       fz_case_block_capture(r.cs, !may_capture);
       int pending = 0, rc = FZ_OK;
-      if (hipEventRecord(r.ev[2 * r.nq], r.ctx->st) != hipSuccess) rc = fz_set_error(FZ_ERR_HIP, "hipEventRecord");
+      if (hipEventRecord(r.ev[2 * r.nq], r.ctx->stream()) != hipSuccess)
+        rc = fz_set_error(FZ_ERR_HIP, "hipEventRecord");
       if (rc == FZ_OK) rc = fz_case_step_begin(r.cs, &pending);
-      if (rc == FZ_OK && hipEventRecord(r.ev[2 * r.nq + 1], r.ctx->st) != hipSuccess)
+      if (rc == FZ_OK && hipEventRecord(r.ev[2 * r.nq + 1], r.ctx->stream()) != hipSuccess)
         rc = fz_set_error(FZ_ERR_HIP, "hipEventRecord");
       if (rc != FZ_OK) {
         r.rc = rc;
@@ -496,7 +497,7 @@ extern "C" int fz_server_round(fz_server *s, int *n_active, int *n_queued) {
     if (r.rc != FZ_OK) {
       // the failed case is dropped (its stream drained first), the request
       // finishes as failed and its memory returns
-      (void)hipStreamSynchronize(r.ctx->st);
+      (void)hipStreamSynchronize(r.ctx->stream());
       fz_case_block_capture(r.cs, false);
       drop_running(r);
       fail_request(s, r.id, r.bytes, r.err);

@@ -3078,7 +3078,7 @@ int fz_launch_forcing(fz_ctx *c, int ftype, double alpha, double dt, const doubl
   const int nt = std::max(c->d.n1, std::max(c->d.n2, c->d.n3)) + 2;
   if (!c->ftab) {  // the tables, made on the first call outside a graph capture
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    FZ_HIP(hipStreamIsCapturing(c->st, &cap));
+    FZ_HIP(hipStreamIsCapturing(c->stream(), &cap));
     if (cap == hipStreamCaptureStatusNone) {
       FZ_HIP(hipMalloc((void **)&c->ftab, sizeof(double) * FT_ROWS * nt));
       FZ_LAUNCH(c, "forcing_tables", k_forcing_tables, dim3((nt + 255) / 256), dim3(256), 0, c->d, nt, c->l[0],

@@ -56,9 +56,9 @@ int trial(fz_case *sc, fz_ctx *c, const Tuned &t, bool proj32, int steps, hipEve
   FZ_TRY(fz_case_step(sc, 1, &killed));
   float best = 0.0f;
   for (int rep = 0; rep < 2; rep++) {
-    FZ_HIP(hipEventRecord(a, c->st));
+    FZ_HIP(hipEventRecord(a, c->stream()));
     FZ_TRY(fz_case_step(sc, steps, &killed));
-    FZ_HIP(hipEventRecord(b, c->st));
+    FZ_HIP(hipEventRecord(b, c->stream()));
     FZ_HIP(hipEventSynchronize(b));
     float e = 0.0f;
     FZ_HIP(hipEventElapsedTime(&e, a, b));
@@ -122,7 +122,7 @@ extern "C" int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size
     if (rc != FZ_OK) return rc;
     g_tuned[key] = best;
   }
-  FZ_HIP(hipStreamSynchronize(ctx->st));
+  FZ_HIP(hipStreamSynchronize(ctx->stream()));
   apply(ctx, best, proj32);
   fz_case_drop_graphs(cs);  // captured launches carry the old parameters
   if (report && cap > 0)
