@@ -2501,6 +2501,8 @@ extern "C" int fz_solver_batched(fz_ctx *const *ctxs, double *const *ps, int n) 
   // (sixteen 64^3 solves: waiting for the streams 326 us a call, events between
   // them 375 us, asking each whether it has drained 440 us)
   for (int q = 0; q < n; q++) FZ_HIP(hipStreamSynchronize(ctxs[q]->stream()));
+  // (and the default stream's, where a program may have filled them)
+  FZ_HIP(hipStreamSynchronize(nullptr));
   if (P->batch_cap < 3 * (size_t)n) {
     if (P->batch_ptrs) FZ_HIP(hipFree(P->batch_ptrs));
     P->batch_ptrs = nullptr;

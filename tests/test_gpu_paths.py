@@ -428,3 +428,34 @@ def test_rk_2fl_writes_the_faces_of_its_transport(n, vof, rng):
         F.lib().fz_rk_state_destroy(st)
     finally:
         ctx.close()
+
+
+def test_batched_solves_follow_the_default_stream(rng):
+    """Right-hand sides written on the default stream, behind copies that take
+    milliseconds, are there when fz_solver_batched reads them."""
+    hip, n, k = F.lib(), [32, 24, 16], 3  # (the library's own HIP runtime)
+    ctxs = [F.Context(n, [1.0, 0.9, 1.7], "PPPPNN") for _ in range(k)]
+    try:
+        for c in ctxs:
+            F.call("fz_initsolver", c.h, None, None, None, None, None, None, None, None, None)
+        f, zero = np.asfortranarray(rng.uniform(-1.0, 1.0, [x + 2 for x in n])), np.zeros([x + 2 for x in n])
+        src, ref = ctxs[0].halo(f), ctxs[0].halo(f)
+        F.call("fz_solver", ctxs[0].h, ref.ptr)
+        ref = ref.download()
+        ds = [c.halo(zero) for c in ctxs]
+        big = [F.DArray(ctxs[0], (1 << 27,)) for _ in range(2)]  # 1 GiB each
+        copy = lambda dst, s: hip.hipMemcpyAsync(dst.ptr, s.ptr, C.c_size_t(s.nbytes), 3, None)  # noqa: E731
+        for _ in range(3):
+            for d in ds:
+                d.upload(zero)
+            assert all(copy(*big) == 0 for _ in range(20))
+            assert all(copy(d, src) == 0 for d in ds)
+            F.call("fz_solver_batched", (C.c_void_p * k)(*[c.h.value for c in ctxs]),
+                   (C.c_void_p * k)(*[d.ptr.value for d in ds]), k)
+            for d in ds:
+                assert np.array_equal(d.download()[1:-1, 1:-1, 1:-1], ref[1:-1, 1:-1, 1:-1])
+        for d in big:
+            d.free()
+    finally:
+        for c in ctxs:
+            c.close()
