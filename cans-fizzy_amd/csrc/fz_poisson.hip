@@ -1910,7 +1910,7 @@ int fz_poisson_destroy(fz_poisson *p) {
 }
 
 template <typename T>
-static bool reg_fits(const fz_ctx *ctx);
+static bool reg_takes(const fz_ctx *ctx, int nbatch = 1);
 constexpr int REG_PAD = 128;  // a k_thomas_reg block's rows past the last one are fewer
 
 extern "C" int fz_initsolver(fz_ctx *ctx, const double bcpre[6], double *lambdaxy_h, double *a_h, double *b_h,
@@ -2031,7 +2031,8 @@ extern "C" int fz_initsolver(fz_ctx *ctx, const double bcpre[6], double *lambdax
     FZ_LAUNCH(ctx, "periodic_p2", k_periodic_p2, dim3((int)((ps + 255) / 256)), dim3(256), 0, P->piv, P->aux,
               P->lambdaxy, P->a, P->b, P->c, n1, n2, n3);
     FZ_LAUNCHED();
-    P->zper = ctx->thomas_reg && reg_fits<float>(ctx);  // (FP64 and FP32 solves alike)
+    // (FP64 and FP32 solves alike)
+    P->zper = ctx->thomas_reg && reg_takes<float>(ctx) && reg_takes<double>(ctx);
     if (P->zper) {  // the pivots of its n3 - 1 rows in place of the per-solve ones
       FZ_LAUNCH(ctx, "piv_pre", k_piv_pre, dim3((int)((ps + 255) / 256)), dim3(256), 0, P->piv, (double *)nullptr,
                 P->lambdaxy, P->a, P->b, P->c, n1, n2, n3 - 1);
@@ -2117,11 +2118,21 @@ static int launch_r2r(fz_ctx *ctx, const char *name, const fz_fftplan &P, int ki
   return FZ_OK;
 }
 
-// whether k_thomas_reg takes columns of T: its blocks hold 1024 FP64 or 512
-// FP32 rows, and the array's byte offsets fit in 32 bits
+// Whether k_thomas_reg solves columns of T. It fits where its blocks, of 1024
+// FP64 or 512 FP32 rows, hold a column and the array's byte offsets fit in 32
+// bits. It pays from 17 rows, a second turn of a thread's 16: a block of
+// shorter columns is one wave of which a quarter (FP64) or half has rows at
+// all; and from 24 in FP64 once there are 16384 columns, whose blocks wait for
+// each other. The chunked kernels against it, a whole solve: 64x64x16 31.2 and
+// 31.3 us, 64x64x17 32.2 and 31.4; 256x256x8 40.1 and 46.1, 256x256x17 56.1 and
+// 58.2, 256x256x24 62.0 and 63.0, 512x256x24 82.5 and 79.3, 256x256x32 66.9 and
+// 63.1; periodic 512x256x16 76.5 and 84.2, 512x256x24 91.2 and 92.2, 512x256x32
+// 113.9 and 105.2; FP32 512x256x8 146 and 153, 512x256x17 181 and 181.
 template <typename T>
-static bool reg_fits(const fz_ctx *ctx) {
-  return ctx->d.n3 <= (sizeof(T) == 8 ? 1024 : 512) && ctx->ni * (long)sizeof(double) < (1L << 32);
+static bool reg_takes(const fz_ctx *ctx, int nbatch) {
+  const bool fits = ctx->d.n3 <= (sizeof(T) == 8 ? 1024 : 512) && ctx->ni * (long)sizeof(double) < (1L << 32);
+  const bool many = sizeof(T) == 8 && (long)ctx->d.n1 * ctx->d.n2 * nbatch >= 16384;
+  return fits && ctx->d.n3 >= (many ? 24 : 17);
 }
 // (32 rows to a thread from 256 rows: half the turns, 213 -> 207 us at
 // 256x256x512, 124 -> 112 us at 256^3 periodic; 16 below, where the waves
@@ -2242,7 +2253,7 @@ static int solver_rest(fz_ctx *ctx, T *W, double *p, int accum) {
     // at 224x224x512; but 166 against 131 at 192x192x512, and 95 against 77
     // at 256^3)
     const bool pairs = mixed && ps % 2 == 0 && ctx->d.n3 > 256 && ps >= 49152;
-    const bool reg = tk == 0 && P->zpre && reg_fits<T>(ctx) && !pairs;
+    const bool reg = tk == 0 && P->zpre && reg_takes<T>(ctx) && !pairs;
     if (tk == 0) tk = mixed ? -8 : 16;
     const dim3 grid((int)((ps + 63) / 64)), blk(64);
     const char *name = mixed ? "thomas_f32" : "thomas";
@@ -2550,7 +2561,7 @@ int fz_batch_solve(fz_ctx *c0, void **dptrs, int n) {
   FZ_TRY((launch_r2r<double, double, double>(c0, "fft_y_fwd_batch", P->py, P->py.kind_f, (const double *)nullptr,
                                              w_y, (double *)nullptr, w_y, n1, n3, 1.0, 0, w_w)));
   // (the cases share the operator, so the first one's pivots serve all)
-  if (c0->tk64 == 0 && P->zpre && reg_fits<double>(c0))
+  if (c0->tk64 == 0 && P->zpre && reg_takes<double>(c0, n))
     launch_thomas_reg<double, false>(c0, "thomas_batch", (double *)nullptr, P->zpre, -1L, w_d);
   else
     FZ_LAUNCH(c0, "thomas_batch", (k_thomas<16, double>), dim3((int)((ps1 + 63) / 64), n), dim3(64), 0,

@@ -459,3 +459,17 @@ def test_batched_solves_follow_the_default_stream(rng):
     finally:
         for c in ctxs:
             c.close()
+
+
+@pytest.mark.parametrize("n", [[16, 15, 16], [16, 15, 17], [128, 126, 23], [128, 128, 23], [128, 128, 24]],
+                         ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("cbc", ["NNPPDD", "PPPPPP"])
+def test_short_columns_match_the_chunked_kernels(n, cbc, rng, monkeypatch):
+    """Both sides of the lines from which columns are held in registers (17
+    rows; 24 for 16384 FP64 columns, which the cases of a batch have together)."""
+    f = np.asfortranarray(rng.uniform(-1.0, 1.0, [x + 2 for x in n]))
+    for mixed, count in [(False, 1), (True, 1)] + ([(False, 2)] if cbc != "PPPPPP" else []):
+        monkeypatch.delenv("FZ_THOMAS_ROWS64", raising=False)
+        got = solve(n, cbc, f, mixed, count)
+        monkeypatch.setenv("FZ_THOMAS_ROWS64", "16")
+        assert np.array_equal(got, solve(n, cbc, f, mixed, count), equal_nan=True), (mixed, count)
