@@ -142,6 +142,8 @@ struct fz_ctx {
   int correc_my = 4;    // rows of cells per block of the LDS correction kernel: 4, 8 or 16
   int ncu = 256;        // the device's compute units
   int march = 0;        // planes per block of the z-marching kernels; 0: by the grid (march_planes)
+  int p16 = -1;         // long strided lines with sixteen points a thread: 0 never, 1 wherever that form exists, -1 by
+                        // the size of the launch (p16_takes)
   int p2_xdiv = 2;      // x-line transforms run 1 or 2 times fewer lines per block than y lines
   int thomas_pre = 0;   // 1: Thomas solves with the pivots made once at set-up (k_thomas_pre); set at
                         // creation (1 unless thomas_rc), cleared for cases whose solves are FP32

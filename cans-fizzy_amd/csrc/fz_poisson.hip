@@ -687,7 +687,8 @@ __global__ void __launch_bounds__((P2Shape<M, QUARTER, R, GDIV>::NT)) __attribut
 // of k_r2r_p2 needs 1024 threads for row segments of 128 bytes (512^3 FP64 y
 // lines 663 and 632 -> 578 and 539 us forward and backward; 256^3 FP32 ones 53
 // and 50 -> 37 and 38 us), not below (FP64 lines of 256 backward 132 against
-// 141 us) nor for contiguous lines (512^3 backward 505 against 551 us).
+// 141 us) nor for contiguous lines (512^3 backward 505 against 551 us), and not
+// where the waves are few; FP64 has the periodic kinds only. See p16_takes.
 template <int M, typename R>
 struct P16Shape {
   static constexpr int LG = __builtin_ctz(M);
@@ -988,12 +989,34 @@ static void launch_p2_g(fz_ctx *ctx, const char *name, const fz_fftplan &P, int 
   }
 #undef FZ_P2_LAUNCH
 }
+// Whether long strided lines run k_r2r_p16: sixteen points a thread are a
+// quarter of k_r2r_p2's waves. In FP64 for periodic lines (a transform at
+// 256x512x128 73-82 against 64-69 us, 128x512x16 18 and 17), to 16 waves a CU
+// at 2048 points (128x2048x32 77 and 76, 128x2048x64 154 and 165); the sine and
+// cosine kinds, which pass LDS value by value on one side, are slower there at
+// every size (256x512x128 89 and 84 against 103 and 94, 32x512x16 17.5 and
+// 18.2). In FP32 once the launch gives every CU 8 waves, and those kinds below
+// 1024 points 16 (both directions, sixteen points last: 128x256x32 12.7 and
+// 12.5, 12.7 and 15.4; 256x256x128 27.7 and 19.7, 27.4 and 22.0; cosines at
+// 256x256x64 18.7 and 20.9, 19.1 and 23.6, at 256x512x64 41 and 29; 32x2048x16
+// 22 and 29, 64x2048x32 41 and 31).
+template <int M, typename R>
+static bool p16_takes(const fz_ctx *ctx, int kind, int L1, long L2) {
+  using S = P16Shape<M, R>;
+  const bool periodic = kind == K_R2HC || kind == K_HC2R;
+  const long waves = (L1 + S::G - 1) / S::G * L2 * (S::NT / 64), each = waves / ctx->ncu;  // each: a CU's
+  if (sizeof(R) == 8 && !periodic) return false;
+  if (ctx->p16 >= 0) return ctx->p16 != 0;
+  if (sizeof(R) == 8) return M < 2048 || each <= 16;
+  return each >= (periodic || M >= 1024 ? 8 : 16);
+}
+
 template <int M, bool QUARTER, typename R, typename TI, typename TO>
 static void launch_p2(fz_ctx *ctx, const char *name, const fz_fftplan &P, int kind, const TI *src, LineMap in,
                       TO *dst, LineMap out, int L1, int L2, double scale, int accum, const FillSrc &fs,
                       const Batch &bt) {
   if constexpr (!QUARTER && M * (int)sizeof(R) >= 1024 && (sizeof(R) == 4 || M >= 512) && sizeof(TI) == sizeof(TO)) {
-    if (in.se != 1 && out.se != 1 && !fs.on) {  // long strided lines
+    if (in.se != 1 && out.se != 1 && !fs.on && p16_takes<M, R>(ctx, kind, L1, (long)L2 * (bt.src ? bt.n : 1))) {
       using S = P16Shape<M, R>;
       const dim3 grid((L1 + S::G - 1) / S::G, L2, bt.src ? bt.n : 1);
       const PlanTabs<R> t = tabs_of(P, R());
@@ -1002,7 +1025,7 @@ static void launch_p2(fz_ctx *ctx, const char *name, const fz_fftplan &P, int ki
             scale, accum, t.tw, t.q, t.t2, bt)
       if (kind == K_R2HC) FZ_P16_LAUNCH(K_R2HC);
       else if (kind == K_HC2R) FZ_P16_LAUNCH(K_HC2R);
-      else FZ_P16_LAUNCH(-1);
+      else if constexpr (sizeof(R) == 4) FZ_P16_LAUNCH(-1);
 #undef FZ_P16_LAUNCH
       return;
     }

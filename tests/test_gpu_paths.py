@@ -473,3 +473,48 @@ def test_short_columns_match_the_chunked_kernels(n, cbc, rng, monkeypatch):
         got = solve(n, cbc, f, mixed, count)
         monkeypatch.setenv("FZ_THOMAS_ROWS64", "16")
         assert np.array_equal(got, solve(n, cbc, f, mixed, count), equal_nan=True), (mixed, count)
+
+
+def solve_unrefined(n, cbc, f):
+    ctx = F.Context(n, [1.0, 0.9, 1.7], cbc)
+    try:
+        F.call("fz_initsolver", ctx.h, None, None, None, None, None, None, None, None, None)
+        d = ctx.halo(f)
+        F.call("fz_solver_mixed", ctx.h, d.ptr, 0.0, 0, C.byref(C.c_int()), None)
+        return d.download()[1:-1, 1:-1, 1:-1]
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("n", [[33, 256, 3], [35, 512, 2], [18, 1024, 2], [10, 2048, 2]],
+                         ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("y", ["PP", "NN", "DD"])
+def test_sixteen_points_a_thread_match_four(n, y, rng, monkeypatch):
+    """Long y lines of every kind in FP32, without refinement, and of the
+    periodic one in FP64, alone and as a batch, line counts that are no
+    multiple of a block's: bit for bit as four points a thread."""
+    f = np.asfortranarray(rng.uniform(-1.0, 1.0, [x + 2 for x in n]))
+    cbc = "PP" + y + "DD"
+    for mixed, count in [(True, 1), (False, 1), (False, 2)]:
+        out = []
+        for p16 in ("1", "0"):
+            monkeypatch.setenv("FZ_P16", p16)
+            out.append(solve_unrefined(n, cbc, f) if mixed else solve(n, cbc, f, False, count))
+        assert np.array_equal(*out), (mixed, count)
+        assert np.abs(out[0]).max() > 0.0
+
+
+@pytest.mark.parametrize("n,y", [([64, 256, 256], "PP"), ([64, 256, 255], "PP"), ([16, 1024, 256], "NN"),
+                                 ([256, 512, 64], "DD"), ([256, 512, 63], "DD")],
+                         ids=lambda v: "x".join(map(str, v)) if isinstance(v, list) else v)
+def test_long_fp32_lines_at_the_rule(n, y, rng, monkeypatch):
+    """Both sides of the launch sizes from which FP32 lines take sixteen points
+    a thread (8 waves a CU; 16 for cosine and sine lines below 1024)."""
+    f = np.asfortranarray(rng.uniform(-1.0, 1.0, [x + 2 for x in n]))
+    out = []
+    for p16 in (None, "0"):
+        monkeypatch.delenv("FZ_P16", raising=False)
+        if p16:
+            monkeypatch.setenv("FZ_P16", p16)
+        out.append(solve_unrefined(n, "PP" + y + "DD", f))
+    assert np.array_equal(*out)
