@@ -3114,14 +3114,21 @@ int fz_launch_rk_fused(fz_ctx *c, const double rho12[2], const double mu12[2], d
                        const double *po, const double *kappa, double *duo, double *dvo, double *dwo, double *un,
                        double *vn, double *wn, double *u, double *v, double *w) {
   if (fits_buffers(c, "rk") != FZ_OK) return 1;
-  dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + MOM_MY - 1) / MOM_MY);
-  const int kz = march_planes<true>(c, grid, c->d.n3, 1, 2);
-  FZ_LAUNCH(c, "rk_mom", (k_mom_lds<double, double, 1, false, false, false, true>), grid, dim3(MOM_MX, MOM_MY), 0,
-            c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1], rho12[1], rho12[0] - rho12[1], mu12[1],
-            mu12[0] - mu12[1], factor1, factor2, first, factor1 + factor2, dt_r, (const double *)nullptr,
-            sigma * 2.0 / (rho12[0] + rho12[1]), rho0, bforce[0], bforce[1], bforce[2], gacc[0], gacc[1], gacc[2],
-            rho_av[0], rho_av[1], rho_av[2], fx, fy, fz, u, v, w, psi, psio, p, pn, po, kappa, duo, dvo, dwo, un, vn,
-            wn, kNoBRef);
+  // (tiles of 2 rows where more than a tenth of the rows of 8-row tiles would
+  // idle, which made some calls slower than the four kernels: 256x1x400 16.5 us
+  // against 27.8 with 8 rows and 17.4 with the kernels, 512x2x1024 61, 109 and 93,
+  // 33x9x400 21, 29 and 23, 256x33x400 195, 207 and 292; full tiles are faster
+  // with 8 rows: 256^3 863 against 918)
+  const int full = (c->d.n2 + MOM_MY - 1) / MOM_MY * MOM_MY, my = 10 * c->d.n2 < 9 * full ? 2 : MOM_MY;
+  dim3 grid((c->d.n1 + MOM_MX - 1) / MOM_MX, (c->d.n2 + my - 1) / my);
+  const int kz = march_planes<true>(c, grid, c->d.n3, 1, my == 2 ? 7 : 2);
+  auto kern = my == 2 ? k_mom_lds<double, double, 1, false, false, false, true, 2>
+                      : k_mom_lds<double, double, 1, false, false, false, true>;
+  FZ_LAUNCH(c, "rk_mom", kern, grid, dim3(MOM_MX, my), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+            rho12[1], rho12[0] - rho12[1], mu12[1], mu12[0] - mu12[1], factor1, factor2, first, factor1 + factor2,
+            dt_r, (const double *)nullptr, sigma * 2.0 / (rho12[0] + rho12[1]), rho0, bforce[0], bforce[1],
+            bforce[2], gacc[0], gacc[1], gacc[2], rho_av[0], rho_av[1], rho_av[2], fx, fy, fz, u, v, w, psi, psio,
+            p, pn, po, kappa, duo, dvo, dwo, un, vn, wn, kNoBRef);
   FZ_LAUNCHED();
   FZ_LAUNCH(c, "rk_mom_back", k_rk_mom_back, fz_grid_interior(c->d), fz_block3(), 0, c->d, un, vn, wn, u, v, w);
   FZ_LAUNCHED();

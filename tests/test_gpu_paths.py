@@ -518,3 +518,11 @@ def test_long_fp32_lines_at_the_rule(n, y, rng, monkeypatch):
             monkeypatch.setenv("FZ_P16", p16)
         out.append(solve_unrefined(n, "PP" + y + "DD", f))
     assert np.array_equal(*out)
+
+
+@pytest.mark.parametrize("n", [[33, 1, 9], [40, 2, 33], [1, 12, 20], [20, 14, 6], [20, 15, 6], [64, 16, 5], [60, 16, 5],
+                               [59, 16, 5], [65, 33, 4], [130, 4, 40]], ids=lambda n: "x".join(map(str, n)))
+def test_integrators_at_the_rules_of_their_tiles(n, rng):
+    """rk and rk_2fl (ACDI) against their parts on both sides of the fill of
+    their tiles' rows and lanes that picks another form."""
+    test_integrators_match_their_parts(n, 0, rng)
