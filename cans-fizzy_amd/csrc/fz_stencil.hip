@@ -1292,10 +1292,12 @@ __global__ void __launch_bounds__(ACD_MX *MY) k_acdi_sf(fz_dims d, int kz, const
 // and values as k_acdi_sf: 96x96x192 77 -> 66 us, 90x75x130 42 -> 29,
 // 120x78x130 46 -> 40; but 920 -> 1010 at 256x256x512, whose tiles are full:
 // see fz_launch_acdi_step.
+// (RK: psi_out is an interior array)
 constexpr int ROW_W = 62;
 struct Acd5 {
   double ps, ph, nx, ny, nz;
 };
+template <bool RK = false>
 __global__ void __launch_bounds__(256) k_acdi_row(
     fz_dims d, int kz, const double *__restrict__ dzci, const double *__restrict__ dzfi, double dxi, double dyi,
     const double *__restrict__ d_gam, double gam_v, double seps, double factor1_v, double factor2_v,
@@ -1352,12 +1354,25 @@ __global__ void __launch_bounds__(256) k_acdi_row(
       flux_y[q] = yu - yr;
       flux_z[q] = wu - wr;
       const double pn = C.ps + factor1 * R + factor2 * Ro;
-      psi_out[q] = fmin(fmax(0.0, pn), 1.0);
+      psi_out[RK ? r : q] = fmin(fmax(0.0, pn), 1.0);
     }
     zu = wu;
     zr = wr;
     C = Z;
   }
+}
+
+// the blocks of k_acdi_row, and whether FP64 tiles whose last column or row
+// leaves more than a fourteenth of the lanes idle give way to it
+static dim3 acdi_row_grid(const fz_ctx *c, int &kz) {
+  dim3 grid((unsigned)(((long)c->d.sy * c->d.n2 + 4 * ROW_W - 1) / (4 * ROW_W)));
+  kz = march_planes(c, grid, c->d.n3, 1, 4);
+  return grid;
+}
+static bool acdi_ragged(const fz_ctx *c) {
+  const double fill = (double)c->d.n1 / ((c->d.n1 + ACD_MX - 1) / ACD_MX * ACD_MX) * c->d.n2 /
+                      ((c->d.n2 + ACD_MY - 1) / ACD_MY * ACD_MY);
+  return fill < 13.0 / 14.0;
 }
 
 template <typename T>
@@ -1370,18 +1385,15 @@ int fz_launch_acdi_step(fz_ctx *c, const double *d_gam, double gam, double seps,
   // 1000-1040 us for the LDS kernel of six faces per cell (1), FP32 547
   // against 557 us; the LDS kernel measured FP32 619 against 663 us and
   // FP64 1047 against 1120 us for the plain one (2)
-  // (FP64 tiles whose last column or row leaves more than a fourteenth of the
-  // lanes idle: waves over the plane's rows (4); equal at 300x180x200, 6 %
-  // idle, and 0-10 % slower where the tiles are full)
-  const double fill = (double)c->d.n1 / ((c->d.n1 + ACD_MX - 1) / ACD_MX * ACD_MX) * c->d.n2 /
-                      ((c->d.n2 + ACD_MY - 1) / ACD_MY * ACD_MY);
-  const bool ragged = sizeof(T) == 8 && c->d.n2 > 2 && fill < 13.0 / 14.0;
+  // (ragged FP64 tiles: waves over the plane's rows (4); equal at 300x180x200,
+  // 6 % idle, and 0-10 % slower where the tiles are full)
+  const bool ragged = sizeof(T) == 8 && c->d.n2 > 2 && acdi_ragged(c);
   const int variant = c->acdi_variant ? c->acdi_variant : (ragged ? 4 : 3);
   if constexpr (sizeof(T) == 8) {
     if (variant == 4) {  // waves over the plane's rows
-      dim3 grid((unsigned)(((long)c->d.sy * c->d.n2 + 4 * ROW_W - 1) / (4 * ROW_W)));
-      const int kz = march_planes(c, grid, c->d.n3, 1, 4);
-      FZ_LAUNCH(c, "acdi_step", k_acdi_row, grid, dim3(256), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+      int kz;
+      const dim3 grid = acdi_row_grid(c, kz);
+      FZ_LAUNCH(c, "acdi_step", k_acdi_row<>, grid, dim3(256), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
                 d_gam, gam, seps, factor1, factor2, stc, first, u, v, w, normx, normy, normz, phi, psio, dpsio,
                 psi_out, flux_x, flux_y, flux_z);
       FZ_LAUNCHED();
@@ -3155,6 +3167,14 @@ int fz_launch_rk_2fl_fused(fz_ctx *c, double factor1, double factor2, int first,
     const long low = (long)(c->d.n1 + 1) * (c->d.n2 + 1) + (long)(c->d.n1 + 1 + c->d.n2) * c->d.n3;
     FZ_LAUNCH(c, "rk_vof_low", k_vof_flux_low, dim3((unsigned)((low + 255) / 256)), dim3(256), 0, c->d, beta, u, v, w,
               nx, ny, nz, phi, fx, fy, fz);
+  } else if (acdi_ragged(c)) {
+    // (also boxes of one and two rows: 1024x1x1024 54 us against 80 in tiles of
+    // 2 rows, 79 of 4 and 63 by transport, update and clip; 130x25x400 47, 76,
+    // 77 and 70; 130x66x64 36.3 in tiles of 4 and 34.5 by the three)
+    int kz;
+    const dim3 grid = acdi_row_grid(c, kz);
+    FZ_LAUNCH(c, "rk_acdi", k_acdi_row<true>, grid, dim3(256), 0, c->d, kz, c->dzci, c->dzfi, c->dli[0], c->dli[1],
+              d_gam, gam, seps, factor1, factor2, stc, first, u, v, w, nx, ny, nz, phi, psi, dpsio, ps, fx, fy, fz);
   } else {
     dim3 grid((c->d.n1 + ACD_MX - 1) / ACD_MX, (c->d.n2 + ACD_MY - 1) / ACD_MY);
     const int kz = march_planes(c, grid, c->d.n3, 1, 3);
