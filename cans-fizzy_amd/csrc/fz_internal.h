@@ -246,6 +246,14 @@ static inline dim3 fz_grid_halo(const fz_dims &d) {
 int fz_reduce_ensure(fz_ctx *ctx, size_t nblocks);
 int fz_scratch_setup(fz_ctx *ctx);
 int fz_batch_solve(fz_ctx *c0, void **dptrs, int n);
+// the z solve that a solver of the context runs (T = float: of a mixed one's FP32 solves)
+struct FzThomas {
+  enum Kind { REG, PRE, RC, PAIRS, CHUNKS } kind;  // columns in registers, pivots made at set-up, no pivot array, two
+                                                   // FP32 columns a lane, pivots of each solve
+  int rows;                                        // a thread's rows (REG) or a chunk's
+};
+template <typename T>
+FzThomas fz_thomas(const fz_ctx *ctx);
 // why cs cannot join a batched step led by first (null: it can)
 const char *fz_case_batch_refusal(const fz_case *first, const fz_case *cs);
 hipStream_t fz_case_batch_stream(const fz_case_batch *b);

@@ -2160,13 +2160,14 @@ static bool reg_takes(const fz_ctx *ctx, int nbatch) {
 // (32 rows to a thread from 256 rows: half the turns, 213 -> 207 us at
 // 256x256x512, 124 -> 112 us at 256^3 periodic; 16 below, where the waves
 // count: 16 solves of 64^3 26 -> 18 us, 64x2x64 9 -> 7 us)
+static int reg_rows(const fz_ctx *ctx) { return ctx->d.n3 >= 256 ? 32 : 16; }
 template <typename T, bool PER>
 static void launch_thomas_reg(fz_ctx *ctx, const char *name, T *W, const double *Z, long gauge, const Batch &bt) {
   const fz_poisson *P = ctx->pois;
   const int n3 = ctx->d.n3, m = PER ? n3 - 1 : n3;
   const long ps = (long)ctx->d.n1 * ctx->d.n2;
   constexpr int CB = 128 / (int)sizeof(T);
-  const int rpt = n3 >= 256 ? 32 : 16;
+  const int rpt = reg_rows(ctx);
   const int nt = (CB * ((m + rpt - 1) / rpt) + 63) / 64 * 64;
   const dim3 grid((unsigned)((ps + CB - 1) / CB), bt.src ? bt.n : 1);
   if (rpt == 32)
@@ -2176,6 +2177,34 @@ static void launch_thomas_reg(fz_ctx *ctx, const char *name, T *W, const double 
     FZ_LAUNCH(ctx, name, (k_thomas_reg<T, CB, 16, PER>), grid, dim3(nt), 0, W, Z, P->aux, P->lambdaxy, P->a, P->b,
               P->c, P->apad, P->cpad, ps, n3, gauge, bt);
 }
+
+// The z solve: the context's choice of rows a chunk (tk64, tk32), or by
+// default (0) the columns in registers where that pays, else 16 rows in FP64
+// and two FP32 columns a lane, 8 rows (FP32 columns move half the bytes a load).
+// FP32 columns of more than 256 rows go two to a lane once about 49152 of them
+// fill the device, which moves wider lines at 5.5 TB/s: 192 against 217 us at
+// 256x256x512, 143 against 167 at 256x256x384, 180 against 187 at 224x224x512;
+// but 166 against 131 at 192x192x512, and 95 against 77 at 256^3.
+template <typename T>
+FzThomas fz_thomas(const fz_ctx *ctx) {
+  const fz_poisson *P = ctx->pois;
+  const long ps = (long)ctx->d.n1 * ctx->d.n2;
+  constexpr bool f32 = sizeof(T) == 4;
+  const bool even = f32 && ps % 2 == 0;
+  const int set = f32 ? ctx->tk32 : ctx->tk64, tk = set ? set : (f32 ? -8 : 16), rows = tk < 0 ? -tk : tk;
+  if (P->periodic_z) {
+    if (P->zper) return {FzThomas::REG, reg_rows(ctx)};
+    return {even && tk < 0 ? FzThomas::PAIRS : FzThomas::CHUNKS, 16};
+  }
+  const bool pairs = even && ctx->d.n3 > 256 && ps >= 49152;
+  if (set == 0 && P->zpre && reg_takes<T>(ctx) && !pairs) return {FzThomas::REG, reg_rows(ctx)};
+  if (P->zpre && tk > 0) return {FzThomas::PRE, rows == 8 ? 8 : 16};
+  if (ctx->thomas_rc && tk > 0) return {FzThomas::RC, rows == 8 ? 8 : 16};
+  if (even && tk < 0) return {FzThomas::PAIRS, rows == 8 ? 8 : 16};
+  return {FzThomas::CHUNKS, tk == 8 || tk == 32 ? tk : 16};
+}
+template FzThomas fz_thomas<double>(const fz_ctx *);
+template FzThomas fz_thomas<float>(const fz_ctx *);
 
 // everything after the forward x transform: y transform, z solve, inverses
 // (T = double: the reference's solver; T = float: one FP32 solve of the
@@ -2266,61 +2295,40 @@ static int solver_rest(fz_ctx *ctx, T *W, double *p, int accum) {
   const LineMap w_y = {0, 1, ps, n1};
   FZ_TRY((launch_r2r<T, T, T>(ctx, mixed ? "fft_y_fwd_f32" : "fft_y_fwd", P->py, P->py.kind_f, W, w_y, W, w_y, n1, n3,
                               1.0)));
+  const FzThomas z = fz_thomas<T>(ctx);
+  const bool short8 = z.rows == 8;
+  const dim3 grid((int)((ps + 63) / 64)), pairs((int)((ps / 2 + 63) / 64)), blk(64);
+  float *W32 = (float *)(void *)W;
   if (!P->periodic_z) {
-    // rows per chunk: the context's choice (FP32 columns move half the
-    // bytes per load, so their default keeps twice the rows in flight)
-    int tk = mixed ? ctx->tk32 : ctx->tk64;
-    // (FP32 columns of more than 256 rows, once about 49152 of them fill the
-    // device: two columns a lane move wider lines at 5.5 TB/s, 192 against
-    // 217 us at 256x256x512, 143 against 167 at 256x256x384, 180 against 187
-    // at 224x224x512; but 166 against 131 at 192x192x512, and 95 against 77
-    // at 256^3)
-    const bool pairs = mixed && ps % 2 == 0 && ctx->d.n3 > 256 && ps >= 49152;
-    const bool reg = tk == 0 && P->zpre && reg_takes<T>(ctx) && !pairs;
-    if (tk == 0) tk = mixed ? -8 : 16;
-    const dim3 grid((int)((ps + 63) / 64)), blk(64);
     const char *name = mixed ? "thomas_f32" : "thomas";
-    if (reg) {  // columns in registers
+    if (z.kind == FzThomas::REG) {
       launch_thomas_reg<T, false>(ctx, name, W, P->zpre, gauge, kNoBatch);
-    } else if (P->zpre && tk > 0) {  // pivots made at set-up
-      if (tk == 8) FZ_LAUNCH(ctx, name, (k_thomas_pre<8, T>), grid, blk, 0, W, P->zpre, P->dpre, P->a, n1, n2, n3,
-                             gauge);
-      else FZ_LAUNCH(ctx, name, (k_thomas_pre<16, T>), grid, blk, 0, W, P->zpre, P->dpre, P->a, n1, n2, n3, gauge);
-    } else if (ctx->thomas_rc && tk > 0) {  // no pivot array: the elimination is re-run per chunk
-      if (tk == 8) FZ_LAUNCH(ctx, name, (k_thomas_rc<8, T>), grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c,
-                             n1, n2, n3, gauge, kNoBatch);
-      else FZ_LAUNCH(ctx, name, (k_thomas_rc<16, T>), grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2,
-                     n3, gauge, kNoBatch);
-    } else if (mixed && tk < 0 && ps % 2 == 0) {  // two FP32 columns per lane (tk = -rows per chunk)
-      const dim3 g2((int)((ps / 2 + 63) / 64));
-      float *W32 = (float *)(void *)W;
-      if (P->zpre) {  // pivots made at set-up
-        if (tk == -8) FZ_LAUNCH(ctx, name, k_thomas_pre_x2<8>, g2, blk, 0, W32, P->zpre, P->dpre, P->a, n1, n2, n3,
-                                gauge);
-        else FZ_LAUNCH(ctx, name, k_thomas_pre_x2<16>, g2, blk, 0, W32, P->zpre, P->dpre, P->a, n1, n2, n3, gauge);
-      } else if (tk == -8) {
-        FZ_LAUNCH(ctx, name, k_thomas_x2<8>, g2, blk, 0, W32, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3,
-                  gauge);
-      } else {
-        FZ_LAUNCH(ctx, name, k_thomas_x2<16>, g2, blk, 0, W32, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3,
-                  gauge);
-      }
-    } else if (tk == 8) FZ_LAUNCH(ctx, name, (k_thomas<8, T>), grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2,
-                           n3, gauge, kNoBatch);
-    else if (tk == 32) FZ_LAUNCH(ctx, name, (k_thomas<32, T>), grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c,
-                                 n1, n2, n3, gauge, kNoBatch);
-    else FZ_LAUNCH(ctx, name, (k_thomas<16, T>), grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3,
-                   gauge, kNoBatch);
+    } else if (z.kind == FzThomas::PRE) {
+      auto kern = short8 ? k_thomas_pre<8, T> : k_thomas_pre<16, T>;
+      FZ_LAUNCH(ctx, name, kern, grid, blk, 0, W, P->zpre, P->dpre, P->a, n1, n2, n3, gauge);
+    } else if (z.kind == FzThomas::RC) {
+      auto kern = short8 ? k_thomas_rc<8, T> : k_thomas_rc<16, T>;
+      FZ_LAUNCH(ctx, name, kern, grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3, gauge, kNoBatch);
+    } else if (z.kind == FzThomas::PAIRS && P->zpre) {
+      auto kern = short8 ? k_thomas_pre_x2<8> : k_thomas_pre_x2<16>;
+      FZ_LAUNCH(ctx, name, kern, pairs, blk, 0, W32, P->zpre, P->dpre, P->a, n1, n2, n3, gauge);
+    } else if (z.kind == FzThomas::PAIRS) {
+      auto kern = short8 ? k_thomas_x2<8> : k_thomas_x2<16>;
+      FZ_LAUNCH(ctx, name, kern, pairs, blk, 0, W32, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3, gauge);
+    } else {
+      auto kern = short8 ? k_thomas<8, T> : (z.rows == 32 ? k_thomas<32, T> : k_thomas<16, T>);
+      FZ_LAUNCH(ctx, name, kern, grid, blk, 0, W, P->piv, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3, gauge, kNoBatch);
+    }
   } else {
-    if (P->zper)  // columns in registers
-      launch_thomas_reg<T, true>(ctx, mixed ? "thomas_periodic_f32" : "thomas_periodic", W, P->piv, gauge, kNoBatch);
-    else if (mixed && ctx->tk32 <= 0 && ps % 2 == 0)  // two FP32 columns per lane
-      FZ_LAUNCH(ctx, "thomas_periodic_f32", k_thomas_periodic_x2<16>, dim3((int)((ps / 2 + 63) / 64)), dim3(64), 0,
-                (float *)(void *)W, P->piv, P->aux, P->lambdaxy, P->a, P->b, P->c, n1, n2, n3, gauge);
+    const char *name = mixed ? "thomas_periodic_f32" : "thomas_periodic";
+    if (z.kind == FzThomas::REG)
+      launch_thomas_reg<T, true>(ctx, name, W, P->piv, gauge, kNoBatch);
+    else if (z.kind == FzThomas::PAIRS)
+      FZ_LAUNCH(ctx, name, k_thomas_periodic_x2<16>, pairs, blk, 0, W32, P->piv, P->aux, P->lambdaxy, P->a, P->b, P->c,
+                n1, n2, n3, gauge);
     else
-      FZ_LAUNCH(ctx, mixed ? "thomas_periodic_f32" : "thomas_periodic", (k_thomas_periodic_pc<16, T>),
-                dim3((int)((ps + 63) / 64)), dim3(64), 0, W, P->piv, P->aux, P->lambdaxy, P->a, P->b, P->c, n1, n2,
-                n3, gauge);
+      FZ_LAUNCH(ctx, name, (k_thomas_periodic_pc<16, T>), grid, blk, 0, W, P->piv, P->aux, P->lambdaxy, P->a, P->b,
+                P->c, n1, n2, n3, gauge);
   }
   FZ_LAUNCHED();
   FZ_TRY((launch_r2r<T, T, T>(ctx, mixed ? "fft_y_bwd_f32" : "fft_y_bwd", P->py, P->py.kind_b, W, w_y, W, w_y, n1, n3,

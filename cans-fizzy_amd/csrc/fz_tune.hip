@@ -106,7 +106,12 @@ extern "C" int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size
     for (int dim = 0; dim < 4 && rc == FZ_OK; dim++) {
       const int *cand = dim == 0 ? tiles : (dim == 1 ? moms : (dim == 2 ? tks : rcs));
       int ncand = dim == 0 ? 5 : (dim == 1 ? 5 : (dim == 2 ? (proj32 ? 5 : 3) : 2));
-      if (dim == 3 && (periodic_z || best.tk <= 0)) ncand = 0;  // no such kernel there
+      if (dim == 3) {  // where the solve has, or would have, no pivot array
+        apply(c, best, proj32);
+        const FzThomas::Kind k = proj32 ? fz_thomas<float>(c).kind : fz_thomas<double>(c).kind;
+        const bool either = k == FzThomas::RC || (k == FzThomas::CHUNKS && (!proj32 || best.tk > 0));
+        if (periodic_z || !either) ncand = 0;
+      }
       for (int q = 0; q < ncand && rc == FZ_OK; q++) {
         Tuned t = best;
         int &field = dim == 0 ? t.tile_y : (dim == 1 ? t.mom_variant : (dim == 2 ? t.tk : t.rc));
@@ -125,9 +130,12 @@ extern "C" int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size
   FZ_HIP(hipStreamSynchronize(ctx->stream()));
   apply(ctx, best, proj32);
   fz_case_drop_graphs(cs);  // captured launches carry the old parameters
-  if (report && cap > 0)
-    snprintf(report, cap, "tile_y=%d mom_variant=%d thomas_rows=%d%s ms_per_step=%.4f%s", best.tile_y,
-             best.mom_variant, best.tk < 0 ? -best.tk : (best.tk ? best.tk : 16), best.tk < 0 ? "x2" : (best.rc ? "rc" : ""), best.ms,
-             cached ? " (cached)" : "");
+  if (report && cap > 0) {  // (the z solve as the case now runs it)
+    const FzThomas z = proj32 ? fz_thomas<float>(ctx) : fz_thomas<double>(ctx);
+    const char *kind[] = {"registers", "setup_pivots", "no_pivots", "pairs", "chunks"};
+    snprintf(report, cap, "tile_y=%d mom_variant=%d thomas_rows=%d%s ms_per_step=%.4f thomas=%s%s", best.tile_y,
+             best.mom_variant, z.rows, z.kind == FzThomas::PAIRS ? "x2" : (z.kind == FzThomas::RC ? "rc" : ""), best.ms,
+             kind[z.kind], cached ? " (cached)" : "");
+  }
   return FZ_OK;
 }

@@ -294,8 +294,9 @@ int fz_case_set_graphs(fz_case *cs, int on);
  * occupancy, Thomas rows per chunk) by timing trial_steps steps per
  * candidate on a scratch case of the same parameters; applies the choice to
  * the case and caches it per shape for later cases. Results are the same
- * bit for bit under every choice. report (if not null) receives the choice
- * and its time. No reference counterpart. */
+ * bit for bit under every choice. report (if not null) receives the choice,
+ * its time and the z solve it runs (thomas_rows: a thread's rows with
+ * thomas=registers, else a chunk's). No reference counterpart. */
 int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size_t cap);
 /* batched steps of same-shaped cases (no reference counterpart): one launch
  * per stage of the step for all the cases, each block taking its case's
