@@ -132,10 +132,10 @@ struct fz_ctx {
   int tk32 = 0;         // the same for the FP32 one; negative: two columns per lane, -8 or -16 rows per chunk
                         // (-8 where the columns do not fit in registers)
   int thomas_reg = 1;   // 0: periodic z keeps its chunked kernel too
-  int acdi_variant = 0;  // ACDI step: 0 the default (3), 1 fields staged in LDS, 2 one cell per thread, 3 each face once
-  int youngs_variant = 0;  // Youngs kernel: 0 the default (FP32 1, FP64 3), 1 marching in z, 2 one cell per thread,
-                           // 3 marching without range checks when the range flag allows, else one cell per thread
-                         // (k_acdi_lds), 2 one cell per thread
+  int acdi_variant = 0;    // ACDI step: 0 the default (3, or 4 where FP64 tiles would idle), 1 fields staged in LDS,
+                           // 2 one cell per thread, 3 each face once, 4 (FP64) waves over the plane's rows
+  int youngs_variant = 0;  // Youngs kernel: 0 the default (FP32 1; FP64 3, or 2 on small grids), 1 marching in z, 2 one
+                           // cell per thread, 3 marching without range checks when the range flag allows, else 2
   int correc_kz = 1;    // correction step: 0 one cell per thread, 1 dp, u, v staged in LDS (k_correc_lds),
                         // 8 or 16 cells per thread marching in z (k_correc_step_mz)
   int correc_pair = 1;  // 0: the LDS correction kernel also for rows of even length
@@ -145,8 +145,8 @@ struct fz_ctx {
   int p16 = -1;         // long strided lines with sixteen points a thread: 0 never, 1 wherever that form exists, -1 by
                         // the size of the launch (p16_takes)
   int p2_xdiv = 2;      // x-line transforms run 1 or 2 times fewer lines per block than y lines
-  int thomas_pre = 0;   // 1: Thomas solves with the pivots made once at set-up (k_thomas_pre); set at
-                        // creation (1 unless thomas_rc), cleared for cases whose solves are FP32
+  int thomas_pre = 0;   // 1: the pivots of a non-periodic z are made once at set-up (k_thomas_reg, k_thomas_pre); set
+                        // at creation (1 unless thomas_rc)
   int thomas_rc = 0;    // 1: Thomas kernels without a pivot array (the elimination re-run per chunk);
                         // set at creation from the column count
 };
@@ -162,7 +162,7 @@ struct fz_prof_scope {
 #define FZ_LAUNCH(c, name, kernel, grid, block, shmem, ...)                              \
   do {                                                                                   \
     fz_prof_scope fz_ps_((c), name);                                                     \
-    hipLaunchKernelGGL(kernel, grid, block, shmem, (c)->stream(), __VA_ARGS__);                \
+    hipLaunchKernelGGL(kernel, grid, block, shmem, (c)->stream(), __VA_ARGS__);          \
   } while (0)
 
 // Workgroups are dealt round-robin to the 8 XCDs in dispatch order, each XCD

@@ -1556,7 +1556,9 @@ __device__ __forceinline__ ColBuf<T> col_buf(const T *p, long n) {
 // holding the RPT rows from g*RPT of column col and their pivots, all loaded
 // together. The elimination then runs through the groups in turn, by a shuffle
 // inside a wave and through LDS from wave to wave, and the substitution runs
-// back the same way; the other blocks of the CU load meanwhile. The chain is
+// back the same way; another block of the CU, where it holds one (not beside
+// FP32 columns of 512 rows or FP64 ones of 1024, whose 512 threads take the
+// registers), loads meanwhile. The chain is
 // three dependent operations a row forward and two back, the products
 // d = c z being made beside it, and everything it reads is in registers before
 // its turn (ap and cp are a and c, -1 past the end, where a row passes the
@@ -1567,8 +1569,10 @@ __device__ __forceinline__ ColBuf<T> col_buf(const T *p, long n) {
 // PER: gaussel_periodic with the second solve P2 made at set-up, as
 // k_thomas_periodic_pc (32 bytes a row against 88): the first n3-1 rows, then
 // the cyclic unknown and the update on the values in registers.
-// What bounds it: the bytes where the columns fill the device (256x256x512
-// 207 us against 287 for k_thomas_pre, 3.9 TB/s; 256^3 periodic 112 against
+// What bounds it: the registers where the columns fill the device (244 to 256
+// with 32 rows a thread, some spilled in FP32 and with a periodic z, so 2 waves
+// a SIMD wait 58 % of their cycles on memory and turns at 3.9 TB/s: 256x256x512
+// 207 us against 287 for k_thomas_pre; 256^3 periodic 112 against
 // 212; FP32 256^3 77 against 95), the chain of a block elsewhere
 // (64x64x128 10 against 27 us, 128x128x256 FP32 25 against 69, sixteen 64^3
 // in a batch 18 against 35, whose kernel k_thomas divides per row). The

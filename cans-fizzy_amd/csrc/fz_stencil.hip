@@ -327,15 +327,15 @@ static int fits_buffers(const fz_ctx *c, const char *who) {
 // of one case). Sixteen planes read each plane of a large grid nearly once,
 // and a grid that fills the device several times over takes them. A smaller
 // one waits for its blocks' marches: it takes the number of planes with the
-// least (rounds of resident blocks) x (planes + start-up), res blocks per CU
-// being resident and the start-up (the planes around the first, one memory
+// least (rounds of blocks) x (planes + start-up), res blocks per CU making a
+// round (a nominal number per kernel, not what its build can hold) and
+// the start-up (the planes around the first, one memory
 // latency each) costing about START levels. WHOLE: a last round that is
 // not full costs a full one (the momentum kernel, bound by latency; the
 // others share the bandwidth that its absence leaves, and 1.3 rounds take
-// 1.3 times as long as one). Measured, 16 planes against this choice: 64x2x64
-// momentum 45 -> 10 us, ACDI 43 -> 10, correction 26 -> 9, normals 18 -> 8;
-// 64x64x128 53 -> 27, 48 -> 23, 30 -> 15, 20 -> 12; 96x96x192 90 -> 81,
-// 95 -> 78, 48 -> 42, 35 -> 30; 128x128x256 and larger unchanged.
+// 1.3 times as long as one). Measured, 16 planes against this choice: momentum
+// 64x2x64 45 -> 10 us, 64x64x128 53 -> 27, 96x96x192 90 -> 81; ACDI tiles
+// 64x2x64 43 -> 10, 64x64x128 48 -> 23; 128x128x256 and larger unchanged.
 // FZ_MARCH_PLANES fixes it. most: the planes per block on large grids.
 template <bool WHOLE = false>
 static int march_planes(const fz_ctx *c, dim3 &grid, int nz, int ncase, int res, int most = 16) {
@@ -1635,8 +1635,9 @@ int fz_launch_vof_step(fz_ctx *c, double beta, double factor1, double factor2, c
                        T *flux_z) {
   int kz;
   const dim3 grid = vof_grid(c, kz);
-  FZ_LAUNCH(c, sizeof(T) == 4 ? "vof_step_f32" : "vof_step", k_vof_step<T>, grid, dim3(256), 0, c->d, kz, c->dzfi, c->dli[0], c->dli[1], beta, factor1, factor2, stc, first, u, v, w, normx, normy, normz,
-            phi, psio, dpsio, psi_out, flux_x, flux_y, flux_z);
+  FZ_LAUNCH(c, sizeof(T) == 4 ? "vof_step_f32" : "vof_step", k_vof_step<T>, grid, dim3(256), 0, c->d, kz, c->dzfi,
+            c->dli[0], c->dli[1], beta, factor1, factor2, stc, first, u, v, w, normx, normy, normz, phi, psio, dpsio,
+            psi_out, flux_x, flux_y, flux_z);
   FZ_LAUNCHED();
   return FZ_OK;
 }
@@ -2026,10 +2027,10 @@ static int launch_youngs(fz_ctx *c, const char *name, const T *psi, T *normx, T 
   // flag applies (the marching FP64 kernel with both forms needs 236 VGPRs,
   // two waves per SIMD, and took 758 against 705-745 us for one cell per
   // thread; capped, it spills), one cell per thread elsewhere and on grids
-  // below about 4 million cells, where one launch without a march beats two:
-  // 17 against 24 us at 64x64x128, 51 against 64 at 96x96x192, 85 against
-  // 89 at 128x128x256, but 192 against 181 at 192x192x256 and 692 against
-  // 606 at 256x256x512
+  // below 60 blocks a CU (3.9 million cells), where one launch without a march
+  // beats two: 17 against 24 us at 64x64x128, 51 against 64 at 96x96x192; just
+  // above the line, at 128x128x256, 85 against 89, but 192 against 181 at
+  // 192x192x256 and 692 against 606 at 256x256x512
   dim3 mgrid = fz_grid_interior(c->d);
   const bool small = (long)mgrid.x * mgrid.y * mgrid.z < 60l * c->ncu;
   const int yv = c->youngs_variant ? c->youngs_variant : (sizeof(T) == 4 ? 1 : (small ? 2 : 3));
@@ -3423,22 +3424,22 @@ int fz_batch_correc_gamma(fz_ctx *c, fz_bref br, int ncase, bool gamma) {
               (double *)nullptr, (double *)nullptr, (double *)nullptr, (unsigned long long *)nullptr, b, 0, 0u);
     FZ_LAUNCHED();
   } else {
-  const int my = c->correc_my;
-  dim3 grid((c->d.n1 + 2 + COR_MX - 1) / COR_MX, (c->d.n2 + 2 + my - 1) / my);
-  const int kz = march_planes(c, grid, c->d.n3 + 2, ncase, 24 / my);
-  fz_bref b = br;
-  b.gz = grid.z;
-  grid.z *= (unsigned)ncase;
+    const int my = c->correc_my;
+    dim3 grid((c->d.n1 + 2 + COR_MX - 1) / COR_MX, (c->d.n2 + 2 + my - 1) / my);
+    const int kz = march_planes(c, grid, c->d.n3 + 2, ncase, 24 / my);
+    fz_bref b = br;
+    b.gz = grid.z;
+    grid.z *= (unsigned)ncase;
 #define FZ_CORREC_LDS_B(MY)                                                                                        \
   FZ_LAUNCH(c, "correc_step", (k_correc_lds<MY, true>), grid, dim3(COR_MX, MY), 0, c->d, kz, c->dzci, 0.0, 0.0, 0.0, \
             c->dli[0], c->dli[1], (const double *)nullptr, 0.0, (const double *)nullptr, (const double *)nullptr,   \
             (const double *)nullptr, (const double *)nullptr, (const double *)nullptr, (double *)nullptr,          \
             (double *)nullptr, (double *)nullptr, (double *)nullptr, (unsigned long long *)nullptr, b, 0, 0u)
-  if (my == 16) FZ_CORREC_LDS_B(16);
-  else if (my == 8) FZ_CORREC_LDS_B(8);
-  else FZ_CORREC_LDS_B(4);
+    if (my == 16) FZ_CORREC_LDS_B(16);
+    else if (my == 8) FZ_CORREC_LDS_B(8);
+    else FZ_CORREC_LDS_B(4);
 #undef FZ_CORREC_LDS_B
-  FZ_LAUNCHED();
+    FZ_LAUNCHED();
   }
   if (gamma) {
     FZ_LAUNCH(c, "gamma_fin", k_gamma_fin<true>, dim3((unsigned)ncase), dim3(FZ_GAMMA_SLOTS), 0,

@@ -8,8 +8,9 @@
 //  - the Thomas kernel: the columns in registers, or chunks of 8, 16 or 32
 //    rows (FP64, or FP32 in mixed cases, where two columns per lane are a
 //    candidate too);
-//  - for a non-periodic z, the Thomas kernel without a pivot array (it
-//    reads a column twice instead of storing and reloading pivots).
+//  - for a non-periodic z whose pivots are not made at set-up (from 512x512
+//    columns on), the Thomas kernel without a pivot array (it reads a column
+//    twice instead of storing and reloading pivots) or with one.
 // A scratch case with the same parameters (dt checks off, so every trial
 // times the same work) is stepped once per candidate to warm up and then
 // twice `trial_steps` times between HIP events on its stream (the faster
