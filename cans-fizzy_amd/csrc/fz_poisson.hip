@@ -1578,16 +1578,19 @@ __device__ __forceinline__ ColBuf<T> col_buf(const T *p, long n) {
 // in a batch 18 against 35, whose kernel k_thomas divides per row). The
 // coefficients read from memory inside the chain instead: 313 us at
 // 256x256x512.
+// (16 rows a thread: fewer than 256 rows, so 16 groups; 32: 512 threads. 16
+// rows at 4 waves a SIMD, 128 registers, with a few spilled in FP32, where 3
+// waves take 1185 against 1070 us a refined solve at 256x256x255; but 154
+// registers for the FP64 form of a periodic z, which spilled 18 at 128 into
+// scratch memory: 8 MB a hardware queue, and 179 against 166 us at 256x256x100,
+// 37.5 against 36.5 at 16x16x255)
 template <typename T, int CB, int RPT, bool PER>
-__global__ void __launch_bounds__(1024 / (RPT / 16)) k_thomas_reg(T *__restrict__ W, const double *__restrict__ Z,
-                                                                  const double *__restrict__ P2,
-                                                                  const double *__restrict__ lambdaxy,
-                                                                  const double *__restrict__ a,
-                                                                  const double *__restrict__ b,
-                                                                  const double *__restrict__ c,
-                                                                  const double *__restrict__ ap,
-                                                                  const double *__restrict__ cp, long ps, int n3,
-                                                                  long gauge, Batch bt) {
+__global__ void __launch_bounds__(RPT == 16 ? 16 * CB : 512)
+    __attribute__((amdgpu_waves_per_eu(RPT == 16 && !(sizeof(T) == 8 && PER) ? 4 : 1)))
+    k_thomas_reg(T *__restrict__ W, const double *__restrict__ Z, const double *__restrict__ P2,
+                 const double *__restrict__ lambdaxy, const double *__restrict__ a, const double *__restrict__ b,
+                 const double *__restrict__ c, const double *__restrict__ ap, const double *__restrict__ cp, long ps,
+                 int n3, long gauge, Batch bt) {
   constexpr int SUB = 64 / CB;  // groups of a wave
   if (bt.src) W = (T *)bt.src[blockIdx.y];
   __shared__ double hand[CB], last[CB];
