@@ -675,11 +675,22 @@ static int graph_step(fz_case *cs, const StepArgs &a) {
     slot = cs->graph[0].exec ? 1 : 0;
     if (cs->graph[slot].exec) drop_graphs(cs), slot = 0;
     // capture from a copy of the host-side pointer state; the launches
-    // then rotate the real state exactly as the replay will
-    FZ_HIP(hipStreamBeginCapture(c->stream(), hipStreamCaptureModeThreadLocal));
-    const int rc = enqueue_step(cs, a);
+    // then rotate the real state exactly as the replay will. The launches go to
+    // a stream made for the capture: while a stream is captured no other thread
+    // can wait for an event that was recorded on it before, as cases of a batch
+    // that this case leads may have to (the wait fails and ends the capture).
+    hipStream_t cap = nullptr;
+    FZ_HIP(hipStreamCreateWithFlags(&cap, hipStreamNonBlocking));
+    int rc = FZ_OK;
     hipGraph_t gr = nullptr;
-    const hipError_t e = hipStreamEndCapture(c->stream(), &gr);
+    hipError_t e = hipStreamBeginCapture(cap, hipStreamCaptureModeThreadLocal);
+    if (e == hipSuccess) {
+      c->lent = cap;
+      rc = enqueue_step(cs, a);
+      c->lent = nullptr;
+      e = hipStreamEndCapture(cap, &gr);
+    }
+    (void)hipStreamDestroy(cap);
     if (rc != FZ_OK) {
       if (gr) (void)hipGraphDestroy(gr);
       return rc;
@@ -953,10 +964,8 @@ struct fz_case_batch {
   fz_bcase *dtab = nullptr;  // the role table, one entry per case
   int *dpar = nullptr;       // each case's pointer state
   void **dsolve = nullptr;   // the correction buffers, work arrays and pivots of the cases
-  // the stream of the batch's work: the first case's if the caller gave it, else one of the batch's own
-  hipStream_t st = nullptr;
-  bool st_made = false;
-  std::shared_ptr<fz_event_own> done;  // the end of the latest step's work
+  hipStream_t st = nullptr;             // the first case's own stream, for the batch's work
+  std::shared_ptr<fz_stream_own> made;  // that stream, if the library made it
   bool mixed = false;
   bool pending = false;  // a step begun and not ended
 };
@@ -1022,9 +1031,8 @@ const char *fz_case_batch_refusal(const fz_case *first, const fz_case *cs) { ret
 
 extern "C" int fz_case_batch_destroy(fz_case_batch *b) {
   if (!b) return FZ_OK;
-  // (a first case on a stream that the caller gave waits for it in its own end)
-  if (b->st && (b->st_made || *b->alive[0])) (void)hipStreamSynchronize(b->st);
-  if (b->st_made) (void)hipStreamDestroy(b->st);
+  // (the first case's end waited for its stream, and with it for the batch's work)
+  if (!b->cs.empty() && *b->alive[0]) (void)hipStreamSynchronize(b->st);
   if (b->dtab) (void)hipFree(b->dtab);
   if (b->dpar) (void)hipFree(b->dpar);
   if (b->dsolve) (void)hipFree(b->dsolve);
@@ -1044,6 +1052,8 @@ extern "C" int fz_case_batch_create(fz_case *const *cases, int n, fz_case_batch 
   }
   fz_case_batch *b = new fz_case_batch();
   b->cs.assign(cases, cases + n);
+  b->st = cases[0]->ctx->own;
+  b->made = cases[0]->ctx->made;
   for (const fz_case *cs : b->cs) b->alive.push_back(cs->alive);
   b->mixed = cases[0]->precision == FZ_PREC_MIXED;
   std::vector<fz_bcase> tab(n);
@@ -1088,14 +1098,6 @@ extern "C" int fz_case_batch_create(fz_case *const *cases, int n, fz_case_batch 
   if (rc == FZ_OK) hip(hipMemcpy(b->dtab, tab.data(), sizeof(fz_bcase) * n, hipMemcpyHostToDevice), "upload");
   if (rc == FZ_OK) hip(hipMemcpy(b->dpar, par.data(), sizeof(int) * n, hipMemcpyHostToDevice), "upload");
   if (rc == FZ_OK) hip(hipMemcpy(b->dsolve, sol.data(), sizeof(void *) * 3 * n, hipMemcpyHostToDevice), "upload");
-  if (rc == FZ_OK && !cases[0]->ctx->own_made) {
-    b->st = cases[0]->ctx->own;
-  } else if (rc == FZ_OK) {
-    hip(hipStreamCreateWithFlags(&b->st, hipStreamNonBlocking), "stream");
-    b->st_made = rc == FZ_OK;
-  }
-  b->done = std::make_shared<fz_event_own>();
-  if (rc == FZ_OK) hip(hipEventCreateWithFlags(&b->done->e, hipEventDisableTiming), "event");
   if (rc != FZ_OK) {
     fz_case_batch_destroy(b);
     return rc;
@@ -1174,42 +1176,44 @@ static int batch_enqueue(fz_case_batch *b) {
 
 // While the batch steps, every case's context uses the batch's stream (its own
 // launches: dt scalars, checks). The batch's work comes after each case's
-// earlier work: an event between the streams only where a case has work that
-// the batch's stream has not waited for, which a case whose stream the library
-// made has not while it steps in this batch alone (events before and after
-// every step took 104 of 294 us a step of eight 128x2x128 cases). A caller may
-// put work of its own on a stream that it gave.
+// earlier work, and each case's later work on its own stream after the batch's.
+// Where the library made both streams, the order takes an event only when a
+// case has been used by itself in between: the context knows whether its stream
+// has work that the batch's has not waited for (used), and waits for the
+// batch's when it next uses its own (behind). Events before and after every
+// step took 104 of 294 us a step of eight 128x2x128 cases, one event a step 8
+// of 249 us of eleven 256x2x107 ones. (A wait put off like that fails while the
+// other stream is captured: the library captures none of these streams.) A
+// caller may put work of its own on a stream that it gave, so those are ordered
+// at every step.
 static int batch_enter(fz_case_batch *b) {
   for (fz_case *cs : b->cs) {
     fz_ctx *c = cs->ctx;
-    if (c->behind && c->behind != b->done) FZ_HIP(hipStreamWaitEvent(b->st, c->behind->e, 0));
-    if (c->own == b->st || (b->st_made && c->own_made && !c->used)) continue;
-    if (!c->ev) FZ_HIP(hipEventCreateWithFlags(&c->ev, hipEventDisableTiming));
-    FZ_HIP(hipEventRecord(c->ev, c->own));
-    FZ_HIP(hipStreamWaitEvent(b->st, c->ev, 0));
+    if (c->behind && c->behind != b->made) FZ_TRY(fz_stream_after(c, b->st, c->behind->s));
+    if (c->used || !c->made || !b->made) FZ_TRY(fz_stream_after(c, b->st, c->own));
   }
   for (fz_case *cs : b->cs) cs->ctx->lent = b->st;
   return FZ_OK;
 }
-// Each case's later work on its own stream comes after the batch's: one event
-// a call, which the cases' streams wait for now, or, where the library made
-// both streams, when the context next uses its own (fz_ctx::stream). (A wait
-// put off like that fails while the event's stream is captured, so that stream
-// is neither a case's, whose steps are, nor a caller's.)
 static int batch_leave(fz_case_batch *b) {
-  hipError_t e = hipEventRecord(b->done->e, b->st);
+  int rc = FZ_OK;
   for (fz_case *cs : b->cs) {
     fz_ctx *c = cs->ctx;
-    const bool later = b->st_made && c->own_made;
     c->lent = nullptr;
     c->behind.reset();
-    c->used = !later;
-    if (e == hipSuccess && later) c->behind = b->done;
-    if (e == hipSuccess && !later && c->own != b->st) e = hipStreamWaitEvent(c->own, b->done->e, 0);
+    if (c->own != b->st && c->made && b->made) {
+      c->behind = b->made;
+      c->used = false;
+      continue;
+    }
+    c->used = true;
+    const int e = fz_stream_after(c, c->own, b->st);
+    if (e != FZ_OK) {
+      rc = e;
+      (void)hipStreamSynchronize(b->st);
+    }
   }
-  if (e == hipSuccess) return FZ_OK;
-  (void)hipStreamSynchronize(b->st);
-  return fz_set_error(FZ_ERR_HIP, "fz_case_batch_step: %s", hipGetErrorString(e));
+  return rc;
 }
 
 // the checks enqueued by a step read back: the next dt and the stop conditions
@@ -1218,7 +1222,7 @@ static int batch_checks(fz_case_batch *b, int *killed, bool *stop) {
   bool pending = false;
   for (size_t q = 0; q < b->cs.size(); q++) pending = pending || (*b->alive[q] && b->cs[q]->check_pending);
   if (!pending) return FZ_OK;
-  if (b->st_made || *b->alive[0]) FZ_HIP(hipStreamSynchronize(b->st));
+  if (*b->alive[0]) FZ_HIP(hipStreamSynchronize(b->st));
   for (size_t q = 0; q < b->cs.size(); q++) {
     fz_case *cs = b->cs[q];
     if (!*b->alive[q] || !cs->check_pending) continue;

@@ -136,7 +136,8 @@ extern "C" int fz_ctx_create(fz_ctx **out, const int n[3], const double l[3], co
       delete c;
       return fz_set_error(FZ_ERR_HIP, "hipStreamCreate: %s", hipGetErrorString(e));
     }
-    c->own_made = true;
+    c->made = std::make_shared<fz_stream_own>();
+    c->made->s = c->own;
   }
   double **dev[6] = {&c->dzc, &c->dzf, &c->zc, &c->zf, &c->dzci, &c->dzfi};
   const std::vector<double> *host[6] = {&c->h_dzc, &c->h_dzf, &c->h_zc, &c->h_zf, &c->h_dzci, &c->h_dzfi};
@@ -183,13 +184,21 @@ extern "C" int fz_ctx_destroy(fz_ctx *c) {
   if (c->ftab) (void)hipFree(c->ftab);
   if (c->h_small) (void)hipHostFree(c->h_small);
   if (c->ev) (void)hipEventDestroy(c->ev);
-  if (c->own_made) (void)hipStreamDestroy(c->own);
-  delete c;
+  delete c;  // (and with it its stream, unless a case of a batch it led has yet to wait for that)
+  return FZ_OK;
+}
+
+// work on `later` comes after the work so far on `first`
+int fz_stream_after(fz_ctx *c, hipStream_t later, hipStream_t first) {
+  if (later == first) return FZ_OK;
+  if (!c->ev) FZ_HIP(hipEventCreateWithFlags(&c->ev, hipEventDisableTiming));
+  FZ_HIP(hipEventRecord(c->ev, first));
+  FZ_HIP(hipStreamWaitEvent(later, c->ev, 0));
   return FZ_OK;
 }
 
 void fz_ctx::catch_up() {
-  if (hipStreamWaitEvent(own, behind->e, 0) != hipSuccess) (void)hipEventSynchronize(behind->e);
+  if (fz_stream_after(this, own, behind->s) != FZ_OK) (void)hipStreamSynchronize(behind->s);
   behind.reset();
 }
 

@@ -80,11 +80,11 @@ struct fz_prof_rec {
   hipEvent_t a, b;
 };
 
-// an event kept until the last one that waits for it lets go of it
-struct fz_event_own {
-  hipEvent_t e = nullptr;
-  ~fz_event_own() {
-    if (e) (void)hipEventDestroy(e);
+// a stream the library made, kept until the last one that may wait for it lets go of it
+struct fz_stream_own {
+  hipStream_t s = nullptr;
+  ~fz_stream_own() {
+    if (s) (void)hipStreamDestroy(s);
   }
 };
 
@@ -100,14 +100,15 @@ struct fz_ctx {
   char cbcpre[6];
   int per[3];
   hipStream_t own = nullptr;  // the context's stream for its whole life (work goes to stream())
-  bool own_made = false;      // the library made it (only the context's calls use it)
-  // A batched step's work on the context runs on the batch's stream (lent,
-  // while the step is enqueued). Nobody but the context's own thread looks at
-  // the members below outside such a step.
+  std::shared_ptr<fz_stream_own> made;  // that stream, if the library made it (only its contexts' calls use it)
+  // A batched step's work on the context runs on the batch's stream, and a
+  // captured step's goes to the capture's (lent, while the step is enqueued).
+  // Nobody but the context's own thread looks at the members below outside a
+  // batched step.
   hipStream_t lent = nullptr;
-  std::shared_ptr<fz_event_own> behind;  // the end of that work, which own has not waited for yet
-  bool used = true;                      // own may hold work that no batch's stream has waited for
-  hipEvent_t ev = nullptr;               // the end of own's work, for a batch's stream
+  std::shared_ptr<fz_stream_own> behind;  // a batch's stream, whose work so far own has not waited for yet
+  bool used = true;                       // own may hold work that no batch's stream has waited for
+  hipEvent_t ev = nullptr;                // orders own and a batch's stream
   // the stream that the context's next work goes to, in order after all its work so far
   hipStream_t stream() {
     if (lent) return lent;
@@ -243,6 +244,7 @@ static inline dim3 fz_grid_halo(const fz_dims &d) {
 }
 
 // internal entry points shared between translation units
+int fz_stream_after(fz_ctx *c, hipStream_t later, hipStream_t first);
 int fz_reduce_ensure(fz_ctx *ctx, size_t nblocks);
 int fz_scratch_setup(fz_ctx *ctx);
 int fz_batch_solve(fz_ctx *c0, void **dptrs, int n);

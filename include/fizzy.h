@@ -307,12 +307,11 @@ int fz_case_autotune(fz_case *cs, int trial_steps, char *report, size_t cap);
  * homogeneous pressure boundary values; create refuses others with
  * FZ_ERR_UNSUPPORTED and the reason. A step of the batch gives every case
  * the fields, scalars and checks of its own fz_case_step bit for bit; the
- * work comes after each case's earlier work and before its later work, each
- * case's own on its own stream (it runs on the first case's stream if the
- * caller gave that, else on one of the batch's). A call on a batch drives all
- * its cases; between such calls each case may be driven by a thread of its
- * own, as if there were no batch. nsteps steps, or fewer when a check stops a
- * case (killed[q] = 1; killed may be null); cases must not be
+ * work runs on the first case's stream after each case's earlier work, and
+ * each case's later work, on its own stream, waits for it. A call on a batch
+ * drives all its cases; between such calls each case may be driven by a
+ * thread of its own, as if there were no batch. nsteps steps, or fewer when a
+ * check stops a case (killed[q] = 1; killed may be null); cases must not be
  * stepped otherwise while in a batch, and a batch must be made again once
  * its cases have been stepped alone. The cases may be destroyed before it, in
  * any order: a step of it then returns FZ_ERR_STATE, and destroy frees it. */
